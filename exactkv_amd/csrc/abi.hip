@@ -1,6 +1,9 @@
 // C-ABI plumbing: version, error messages, the split planner.
 #include <stdarg.h>
+#include <stdint.h>
 #include <stdio.h>
+
+#include <algorithm>
 
 #include "common.hpp"
 #include "../../include/exactkv.h"
@@ -36,49 +39,105 @@ extern "C" int exkv_error_bits(uint32_t* out, int32_t clear, hipStream_t stream)
 
 extern "C" const char* exkv_last_error(void) { return exkv::g_err; }
 
-// Split plan for MI355X: about target_blocks workgroups in total over B * (Hkv / HW) * head
-// groups, where a workgroup covers HW = min(gcd(Hkv, 8), 4) KV heads -- 256 by default, one per
-// CU, since a workgroup holds ~150 KB of LDS -- with
-// at least min_split tokens per split (16 by default, one page: a wavefront's pages follow
-// one another at about one memory round trip each, so a few units are served best by many
-// short splits; measured with one round of workgroups, 64- / 32- / 16-token splits: a
-// 1024-token window of one B1 x 128K sequence 14.2 / 11.1 / 9.6 us, B8 x 1024 15.8 / 14.7
-// us, B1 x 8192 16.1 / 14.3 us) and a split length that is a multiple of 32, or 16. Plays
-// the role of the reference's choose_split
-// (kernels.py:273-277), which targets 512 programs for a 128-SM-class GPU.
-// The split count for `units` workgroup units: up to target_blocks units, one round of
-// about target_blocks workgroups; more units than that: the fewest splits that give at
-// least two rounds (the second round's workgroups start as the first ones end, which
-// staggers the tail) with the last round at least 95% full (else the fullest within 16
-// splits). Every workgroup pays a first-page latency of a few us, so long splits win once
-// the GPU is full: measured at B256 x 4352, 1/2/4/8 splits: 610/601/614/636 us; B620: 2
-// splits 1454 us, 4 splits 1490 us.
-static void plan_core(int64_t units, int32_t T, int64_t target_blocks, int32_t min_split, int32_t* nsplit,
-                      int32_t* split_len) {
+// Split plan for MI355X, over units = B * (Hkv / HW) * query-head groups, where a workgroup
+// covers HW = min(gcd(Hkv, 8), 4) KV heads and `slots` workgroups run side by side (256: one
+// per CU, by its LDS ring; the head-dim-256 kernel two per CU). Plays the role of the
+// reference's choose_split (kernels.py:273-277), which targets 512 programs.
+//
+// A call's time follows the rounds its grid needs, R = ceil(r), r = units * ns / slots, and the
+// pages that one wavefront walks per workgroup, j = ceil(split pages / page phases). In pages
+// (2.05 us at head dim 128 with every CU streaming, 6.4 TB/s; 0.85 of that where the last
+// round leaves CUs idle, when the page's compute bounds it): every round costs j pages and
+// `ramp` more (a workgroup's first page's latency and its epilogue, 6 us), and the last
+// workgroups end spread over a sixteenth of their own time:
+//   cost = R ramp + j (R - 1 + max(last round's share, 0.85)) + (ramp + j) / 16.
+// It fits the sweep behind it (B 1 to 220, 2 to 440 units, T 1000 to 16000) within 5%:
+// 24 x 4093 at 32q/8kv, 5 splits x 832 (240 workgroups) 57.0 us, 6 x 704 (288: two rounds, the
+// second nearly empty) 86.9, 10 x 416 63.2. For each R the best plan is the most splits that
+// fit R rounds, so eight of them are compared, and of equal ones the first (fewer rounds,
+// more splits) is taken. Rounding the split count up instead of down, as before, cost 1.3 to
+// 1.65 times the time wherever the unit count does not divide 256 (same calls, split count
+// up / down: 3 x 4093 24.0 / 17.0 us, 6 x 8192 53.8 / 33.0, 12 x 4093 51.4 / 33.3, 40 x 2048
+// 73.1 / 49.4; head dim 64 24 x 4093 57.0 / 38.8; head dim 256 9 x 4093 88.8 / 56.2).
+// Short splits cost little: a wavefront's pages follow one another at about one memory round
+// trip each, so few units are served best by many splits, down to min_split tokens (16 by
+// default, one page; measured with one round, 64- / 32- / 16-token splits: a 1024-token window
+// of one B1 x 128K sequence 14.2 / 11.1 / 9.6 us).
+static double plan_cost(int64_t units, int64_t ns, int64_t pages, int64_t slots, int nph, double ramp) {
+    const double j = (double)(((pages + ns - 1) / ns + nph - 1) / nph);
+    const double full = (double)((units * ns + slots - 1) / slots - 1);            // rounds before the last
+    const double last = (double)(units * ns) / (double)slots - full;
+    return (full + 1.0) * ramp + j * (full + std::max(last, 0.85)) + (ramp + j) / 16.0;
+}
+
+// The fewest splits with at least two rounds and the last one at least 95% full, else the
+// fullest: the plan of grids larger than the GPU (the second round's workgroups start as the
+// first ones end, which staggers the tail; measured at B256 x 4352, 1/2/4/8 splits:
+// 610/601/614/636 us; B620: 2 splits 1454 us, 4 splits 1490 us), unless plan_cost finds one
+// more than a sixteenth (its error) cheaper, as it does for short contexts (B220 x 1000:
+// 4 x 256 152.7 us, 1 x 1008 125.2).
+static int64_t full_rounds(int64_t units, int64_t slots) {
     int64_t ns = 1;
-    if (units < target_blocks) {
-        ns = (target_blocks + units - 1) / units;
-    } else {
-        double best = -1.0;
-        for (int64_t n = 1; n <= 16; ++n) {
-            const double rounds = (double)(units * n) / target_blocks;
-            if (rounds < 2.0) continue;
-            const double full = rounds / (double)(int64_t)(rounds + 0.999999);
-            if (full > best) {
-                best = full;
-                ns = n;
-            }
-            if (full >= 0.95) break;
+    double best = -1.0;
+    for (int64_t n = 1; n <= 16; ++n) {
+        const double rounds = (double)(units * n) / slots;
+        if (rounds < 2.0) continue;
+        const double full = rounds / (double)(int64_t)(rounds + 0.999999);
+        if (full > best) {
+            best = full;
+            ns = n;
+        }
+        if (full >= 0.95) break;
+    }
+    return ns;
+}
+
+// The plan, for workgroups of nph page phases; `most`: the splits whose partials fit the
+// no-alloc entry point's scratch, so that it takes every plan.
+static void plan_core(int64_t units, int32_t T, int64_t slots, int32_t min_split, int nph, double ramp, int64_t most,
+                      int32_t* nsplit, int32_t* split_len) {
+    const int64_t pages = ((int64_t)T + exkv::kPage - 1) / exkv::kPage;
+    const int64_t cap = std::max<int64_t>(1, ((int64_t)T + min_split - 1) / min_split);
+    const int64_t first = (units + slots - 1) / slots;
+    int64_t ns = 1;
+    double cost = 0.0;
+    for (int64_t r = first; r < first + 8; ++r) {
+        const int64_t n = std::min(std::max<int64_t>(1, slots * r / units), std::min(cap, most));
+        const double c = plan_cost(units, n, pages, slots, nph, ramp);
+        if (r == first || c < cost) {
+            cost = c;
+            ns = n;
+        }
+        if (n == cap || n == most) break;
+    }
+    if (units >= slots) {
+        const int64_t n = std::min(full_rounds(units, slots), cap);
+        if (plan_cost(units, n, pages, slots, nph, ramp) <= cost * 17.0 / 16.0) {
+            const int64_t sl = ((int64_t)T + n - 1) / n;
+            *split_len = (int32_t)(sl <= exkv::kPage ? exkv::kPage : (sl + 31) / 32 * 32);
+            *nsplit = (int32_t)(((int64_t)T + *split_len - 1) / *split_len);
+            return;
         }
     }
-    const int64_t cap = ((int64_t)T + min_split - 1) / min_split;
-    if (ns > cap) ns = cap;
-    if (ns < 1) ns = 1;
-    int64_t sl = ((int64_t)T + ns - 1) / ns;
-    sl = sl <= exkv::kPage ? exkv::kPage : (sl + 31) / 32 * 32;
-    *split_len = (int32_t)sl;
-    *nsplit = (int32_t)(((int64_t)T + sl - 1) / sl);
+    *split_len = (int32_t)((pages + ns - 1) / ns * exkv::kPage);
+    *nsplit = (int32_t)(((int64_t)T + *split_len - 1) / *split_len);
 }
+
+// KV heads (or pairs of them) per workgroup: min(gcd(n, 8), 4)
+static int heads_per_block(int n) {
+    int hw = n, m = 8;
+    while (m) {
+        const int t = hw % m;
+        hw = m;
+        m = t;
+    }
+    return hw > 4 ? 4 : hw;
+}
+static int64_t scratch_splits(int64_t B, int64_t Hq, int64_t D) {
+    return std::max<int64_t>(1, exkv_noalloc_scratch_bytes() / ((D + 2) * 4) / (B * Hq));
+}
+constexpr int kComputeWaves = 8;
+constexpr double kRamp = 2.9, kRampD256 = 5.4;         // head dim 128 and pairs; 256 (2.1 us a page, 11 us a workgroup)
 
 extern "C" int exkv_plan_splits(int32_t B, int32_t Hkv, int32_t Hq, int32_t T, int32_t target_blocks,
                                 int32_t min_split, int32_t* nsplit, int32_t* split_len) {
@@ -86,15 +145,9 @@ extern "C" int exkv_plan_splits(int32_t B, int32_t Hkv, int32_t Hq, int32_t T, i
     EXKV_REQUIRE(nsplit && split_len, "plan_splits: null output");
     if (target_blocks <= 0) target_blocks = 256;
     if (min_split <= 0) min_split = exkv::kPage;
-    const int64_t hg = (Hq / Hkv + 15) / 16;
-    int hw = Hkv, m = 8;                               // KV heads per workgroup: gcd(Hkv, 8), at most 4
-    while (m) {
-        const int t = hw % m;
-        hw = m;
-        m = t;
-    }
-    if (hw > 4) hw = 4;
-    plan_core((int64_t)B * (Hkv / hw) * hg, T, target_blocks, min_split, nsplit, split_len);
+    const int hw = heads_per_block(Hkv);
+    plan_core((int64_t)B * (Hkv / hw) * ((Hq / Hkv + 15) / 16), T, target_blocks, min_split, kComputeWaves / hw, kRamp,
+              scratch_splits(B, Hq, exkv::kD), nsplit, split_len);
     return EXKV_OK;
 }
 
@@ -114,17 +167,19 @@ extern "C" int exkv_plan_splits_hd(int32_t B, int32_t Hkv, int32_t Hq, int32_t T
     EXKV_REQUIRE(B > 0 && Hkv > 0 && Hq > 0 && Hq % Hkv == 0 && T > 0, "plan_splits_hd: bad arguments");
     EXKV_REQUIRE(nsplit && split_len, "plan_splits_hd: null output");
     if (D == 64 && Hkv % 2 == 0) {
-        int hw = Hkv / 2, m = 8;                       // virtual heads per workgroup: gcd(Hkv / 2, 8), at most 4
-        while (m) {
-            const int t = hw % m;
-            hw = m;
-            m = t;
-        }
-        if (hw > 4) hw = 4;
-        plan_core((int64_t)B * (Hkv / 2 / hw) * ((Hq / Hkv + 15) / 16), T, 256, exkv::kPage, nsplit, split_len);
+        const int hw = heads_per_block(Hkv / 2);
+        plan_core((int64_t)B * (Hkv / 2 / hw) * ((Hq / Hkv + 15) / 16), T, 256, exkv::kPage, kComputeWaves / hw, kRamp,
+                  scratch_splits(B, Hq, D), nsplit, split_len);
         return EXKV_OK;
     }
     const int64_t units = (int64_t)B * Hkv * ((Hq / Hkv + 15) / 16);
-    plan_core(units, T, D == 64 && units < 512 ? 768 : 512, 64, nsplit, split_len);
+    if (D == 256) {
+        plan_core(units, T, 512, 64, 2, kRampD256, scratch_splits(B, Hq, D), nsplit, split_len);
+        return EXKV_OK;
+    }
+    const int64_t slots = units < 512 ? 768 : 512, cap = std::max<int64_t>(1, ((int64_t)T + 63) / 64);
+    const int64_t ns = std::min(units < slots ? (slots + units - 1) / units : full_rounds(units, slots), cap);
+    *split_len = (int32_t)std::max<int64_t>(exkv::kPage, (((int64_t)T + ns - 1) / ns + 31) / 32 * 32);
+    *nsplit = (int32_t)(((int64_t)T + *split_len - 1) / *split_len);
     return EXKV_OK;
 }

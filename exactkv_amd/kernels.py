@@ -43,10 +43,10 @@ def plan_splits_hd(B, Hkv, Hq, T, D):
 
 
 def plan_splits(B, Hkv, Hq, T, target_blocks=256, min_split=16):
-    """MI355X split plan (native): about `target_blocks` workgroups (one per CU) when there
-    are fewer (sequence, head-block) units than that, else at least two full rounds -- at
-    least `min_split` tokens per split, split length a multiple of 32 (or one 16-token page).
-    Returns (nsplit, split_len). Short splits cost little: a wavefront's pages follow one
+    """MI355X split plan (native): the split count whose rounds of `target_blocks` workgroups
+    (one per CU) a cost model finds cheapest -- one round of as many splits as fit it for few
+    (sequence, head-block) units, else the fewest rounds that end nearly full -- at least
+    `min_split` tokens per split, split length a multiple of 16. Returns (nsplit, split_len). Short splits cost little: a wavefront's pages follow one
     another at about one round trip each, so few units are best served by many splits
     (measured: B1 x 8K 36 -> 18 -> 14.3 us going from 256- to 64- to 32-token splits)."""
     ns, sl = ctypes.c_int32(), ctypes.c_int32()

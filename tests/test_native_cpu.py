@@ -120,6 +120,26 @@ def test_plan_splits_hd(B, Hkv, Hq, T, D, expect):
         assert (ns, sl) == plan_splits(B, Hkv // 2, Hq // 2, T)
 
 
+@pytest.mark.parametrize("B,Hkv,Hq,T,D,slots,expect", [
+    (3, 8, 32, 4093, 128, 256, (37, 112)),     # 6 units: 42 splits fit one round, 256 pages over them: 7 a split
+    (24, 8, 32, 4093, 128, 256, (5, 832)),     # 48 units: 240 workgroups (6 splits would make 288)
+    (24, 8, 32, 4093, 64, 256, (10, 416)),     # 24 units of pairs
+    (9, 8, 32, 4093, 256, 512, (7, 592)),      # 72 units, two workgroups per CU
+    (65, 8, 32, 4093, 128, 256, (5, 832)),     # 130 units: three rounds, 2.5 of them filled
+    (220, 8, 32, 1000, 128, 256, (1, 1008)),   # short contexts: no second workgroup ramp
+    (1, 1, 1, 1, 128, 256, (1, 16)),
+    (1, 8, 128, 524288, 128, 256, (256, 2048)),
+])
+def test_plan_rounds(B, Hkv, Hq, T, D, slots, expect):
+    from exactkv_amd import _lib
+    from exactkv_amd.kernels import plan_splits_hd
+    ns, sl = plan_splits_hd(B, Hkv, Hq, T, D)
+    assert (ns, sl) == expect
+    assert sl % 16 == 0 and ns * sl >= T and (ns - 1) * sl < T
+    # every plan's partials fit the no-alloc entry point's scratch
+    assert B * Hq * ns * (D + 2) * 4 <= _lib.load().exkv_noalloc_scratch_bytes()
+
+
 def test_rebuild_bitmath_exhaustive(tmp_path):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
