@@ -1,8 +1,9 @@
 // Page encoder, deterministic raw-slot assignment, device-side append and the
 // compressed -> bf16 decoder, for gfx950.
 //
-// Encoding one call's pages takes four launches on the caller's stream (two when the caller
-// gives a scan workspace: 2-4 then run as one chained scan kernel, scan_chain_kernel):
+// Encoding one call's pages takes two launches on the caller's stream up to 65,536 units (the
+// page kernel, then scan_direct_kernel for 2-4 below); above, four, or two when the caller
+// gives a scan workspace (2-4 then run as one chained scan kernel, scan_chain_kernel):
 //   1. enc_pages_kernel    one wavefront per (sequence, page, head): exponent window,
 //                          zero flag, codes, sign|mantissa bytes, base bytes, rowmask
 //                          (reference kernels.py:216-264, codec.py:31-49);
@@ -198,6 +199,8 @@ __global__ void __launch_bounds__(256) enc_pages_kernel(EncArgs a, int nunits) {
     const uint16_t* src = a.src + (int64_t)bi * a.s_b + (int64_t)pg * a.s_pg + (int64_t)hk * a.s_h;
     const int64_t pidx = unit_pidx(a, (int)bi, pg);
     const int64_t row0 = pidx * kPage * a.H + hk, page = pidx * a.H + hk;
+    // the raw-row counter as the call finds it, where scan_direct_kernel's blocks read it
+    if (u == 0 && lane == 0) a.rowoff[page] = *a.cnt;
     encode_page<D>(src, a.s_p, nullptr, lane, a.sm + row0 * D, a.code + row0 * (D / 2), a.H, a.base + page * D,
                    a.rowmask + page);
 }
@@ -494,19 +497,126 @@ __global__ void __launch_bounds__(1024) scan_chain_kernel(EncArgs a, int nunits,
     copy_escaped_rows<VEC16, D>(a, m, off, a.src + bi * a.s_b + pg * a.s_pg + hk * a.s_h, lane);
 }
 
-// Encode n units: the page kernel, then the chained scan when the workspace has at least
-// 2 + ceil(n / kScanUnits) words, else the three-launch scan.
+// ---- two-launch encode of up to kDirectUnits units: no block waits for another
+//
+// scan_direct_kernel: block of `ub` units; it counts the raw rows of every unit before its own
+// by reading their rowmasks again (4 bytes a unit, from the L2s the page kernel left them in),
+// so all blocks start at once and need neither tickets nor a workspace. The counter's value
+// before the call comes from the rowoff slot of the call's first unit, where the page kernel
+// put it and whose final value it is; the last block, which has counted every unit, writes the
+// counter back. The blocks are small (64 units up to 16,384, so that a 4,096-token slot of 8
+// heads runs 32 of them instead of the chain's 2 of 1,024) and their 16 wavefronts take 4 to
+// 16 units each, which is what the raw-row copies need: their loads are a dependent round
+// trip after the masks. The masks read grow with the square of the units (33 MB at 65,536, in
+// 256 blocks), hence the limit.
+constexpr int kDirectUnits = 65536;
+
+static int direct_block_units(int64_t n) { return n <= 16384 ? 64 : n <= 32768 ? 128 : 256; }
+
+// Raw rows of units [0, u0), this thread's share (1,024 threads, all of them calling). u0 is a
+// multiple of 64.
+template <bool PAGED>
+__device__ inline int raw_rows_before(const EncArgs& a, int u0) {
+    int sum = 0;
+    if (!PAGED) {
+        const int L = a.npg * a.H;                     // a sequence's masks: L words in a row, every S words
+        const int64_t S = (int64_t)(a.TS / kPage) * a.H;
+        const int32_t* p0 = a.rowmask + (int64_t)a.b0 * S + (int64_t)a.pg0 * a.H;
+        const bool one = a.nb == 1;
+        if ((uintptr_t)p0 % 16 == 0 && (one || (L % 4 == 0 && S % 4 == 0))) {   // uniform
+            for (int v0 = 4 * (int)threadIdx.x; v0 < u0; v0 += 4 * 4096) {
+                uint4 m[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int v = v0 + 4096 * k;
+                    m[k] = make_uint4(0u, 0u, 0u, 0u);
+                    if (v < u0) {
+                        const int bi = one ? 0 : v / L;
+                        m[k] = *reinterpret_cast<const uint4*>(p0 + bi * S + (v - bi * L));
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) sum += popc32(m[k].x) + popc32(m[k].y) + popc32(m[k].z) + popc32(m[k].w);
+            }
+            return sum;
+        }
+    }
+    for (int v0 = threadIdx.x; v0 < u0; v0 += 4 * 1024) {
+        uint32_t m[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int v = v0 + 1024 * k;
+            int bi, pg, hk;
+            m[k] = v < u0 ? (uint32_t)a.rowmask[unit_page32<PAGED>(a, v, bi, pg, hk)] : 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sum += popc32(m[k]);
+    }
+    return sum;
+}
+
+template <bool PAGED, bool VEC16, int D>
+__global__ void __launch_bounds__(1024) scan_direct_kernel(EncArgs a, int nunits, int ub) {
+    __shared__ int s_before[16], s_own[16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, per = ub >> 4;   // units per wavefront
+    const int u0 = (int)blockIdx.x * ub, u = u0 + w * per + lane;
+    int bi = 0, pg = 0, hk = 0;
+    const int cnt0 = a.rowoff[unit_page32<PAGED>(a, 0, bi, pg, hk)];
+    int64_t page = 0;
+    uint32_t m = 0;
+    const bool mine = lane < per && u < nunits;
+    if (mine) {
+        page = unit_page32<PAGED>(a, u, bi, pg, hk);
+        m = (uint32_t)a.rowmask[page];
+    }
+    const int before = wave_incl_scan(raw_rows_before<PAGED>(a, u0));
+    const int own = wave_incl_scan(popc32(m));
+    if (lane == 63) {
+        s_before[w] = before;
+        s_own[w] = own;
+    }
+    __syncthreads();
+    int pre = cnt0, total = 0;                         // rows before this wavefront's units; the block's
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        pre += s_before[i] + (i < w ? s_own[i] : 0);
+        total += s_before[i] + s_own[i];
+    }
+    const int off = pre + own - popc32(m);
+    if (mine) a.rowoff[page] = off;
+    if (threadIdx.x == 0) {
+        if (blockIdx.x == 0 && a.before != nullptr) *a.before = cnt0;
+        if (blockIdx.x == gridDim.x - 1) *a.cnt = cnt0 + total;
+    }
+    copy_escaped_rows<VEC16, D>(a, m, off, a.src + bi * a.s_b + pg * a.s_pg + hk * a.s_h, lane);
+}
+
+template <int D>
+static void launch_direct(const EncArgs& a, int64_t n, bool paged, bool vec16, hipStream_t stream) {
+    const int ub = direct_block_units(n);
+    auto k = paged ? (vec16 ? scan_direct_kernel<true, true, D> : scan_direct_kernel<true, false, D>)
+                   : (vec16 ? scan_direct_kernel<false, true, D> : scan_direct_kernel<false, false, D>);
+    hipLaunchKernelGGL(k, dim3((unsigned)((n + ub - 1) / ub)), dim3(1024), 0, stream, a, (int)n, ub);
+}
+
+// Encode n units: the page kernel, then the direct scan up to kDirectUnits units; above, the
+// chained scan when the workspace has at least 2 + ceil(n / kScanUnits) words, else the
+// three-launch scan.
 template <int D>
 static void launch_encode_d(const EncArgs& a, int64_t n, uint64_t* ws, int64_t ws_words, hipStream_t stream) {
     hipLaunchKernelGGL(enc_pages_kernel<D>, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream, a, (int)n);
+    const bool paged = a.dst_pages != nullptr;
+    const bool vec16 = (uintptr_t)a.src % 16 == 0 && a.s_b % 8 == 0 && a.s_pg % 8 == 0 && a.s_p % 8 == 0 &&
+                       a.s_h % 8 == 0;
+    if (n <= kDirectUnits) {
+        launch_direct<D>(a, n, paged, vec16, stream);
+        return;
+    }
     const int64_t nb = (n + kScanUnits - 1) / kScanUnits;
     if (ws == nullptr || ws_words < 2 + nb) {
         launch_scan<D>(a, n, stream);
         return;
     }
-    const bool paged = a.dst_pages != nullptr;
-    const bool vec16 = (uintptr_t)a.src % 16 == 0 && a.s_b % 8 == 0 && a.s_pg % 8 == 0 && a.s_p % 8 == 0 &&
-                       a.s_h % 8 == 0;
     auto k = paged ? (vec16 ? scan_chain_kernel<true, true, D> : scan_chain_kernel<true, false, D>)
                    : (vec16 ? scan_chain_kernel<false, true, D> : scan_chain_kernel<false, false, D>);
     hipLaunchKernelGGL(k, dim3((unsigned)nb), dim3(kScanUnits), 0, stream, a, (int)n, (int)nb, ws);

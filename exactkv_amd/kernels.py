@@ -368,9 +368,9 @@ def encode_pages(src, strides, buf, b0, pg0, nb, npg, *, chained=True):
     of cache sequence b0 + i. buf is a cache's encoder view (CompressedKV._buf()): the six
     arrays, the raw-row counter cnt, cap, TS, H, D and optionally 'before', which receives
     the counter's value before the call. Escaped rows take pool slots from the counter on,
-    in (sequence, page, head, token) order. Two launches: the page kernel, then one chained
-    slot scan (in a per-stream workspace); chained=False: the page kernel, then a
-    three-launch scan (same bytes)."""
+    in (sequence, page, head, token) order. Two launches: the page kernel, then the slot scan
+    (above 65,536 pages x heads a chained one, in a per-stream workspace; there
+    chained=False makes it three launches: same bytes)."""
     H, TS, D = buf["H"], buf["TS"], buf["D"]
     _check_source(src, strides, nb, npg, H, D)
     raw = buf["raw"]

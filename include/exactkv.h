@@ -76,10 +76,10 @@ const char* exkv_last_error(void);
  * are not written, and *cnt advances by the call's total (overflow = *cnt > cap).
  * *before (may be NULL) receives the counter's value before the call.
  * scan_ws (8-byte aligned, may be NULL): a workspace of scan_ws_words 64-bit words, all zero
- * when first used and reserved for this library's encodes on one stream; with at least
- * 2 + ceil(nb*npg*H / 1024) words the encode is two launches (the page kernel, then one
- * chained slot scan), else four (the page kernel, then a three-launch scan). Same bytes
- * either way.
+ * when first used and reserved for this library's encodes on one stream. Up to 65,536 pages x
+ * heads the encode is two launches and does not use it; above, with at least
+ * 2 + ceil(nb*npg*H / 1024) words it is two launches (the page kernel, then one chained slot
+ * scan), else four (the page kernel, then a three-launch scan). Same bytes either way.
  * Replaces: kernels.py:340-346 encode_pages (launch of _encode_pages_kernel :233-268),
  * byte-identical to codec.py:31-55 encode_reference. */
 int exkv_encode_pages(const void* src, int64_t s_b, int64_t s_pg, int64_t s_p, int64_t s_h,

@@ -203,3 +203,52 @@ def test_encoder_chained_equals_multi_launch():
         if i == 2:
             assert int(b.rowmask[0, 1, 1].item()) == 0xFFFF
             assert same_bits(kernels.decode_to_bf16(b.buffers(), T), x)
+
+
+@pytest.mark.parametrize("B,npg,H,b0,pg0,D,paged", [
+    (1, 1, 1, 0, 0, 64, False),         # one unit
+    (1, 8, 8, 0, 0, 128, False),        # 64 units: one block full
+    (1, 13, 5, 0, 1, 128, False),       # 65 units, masks not 16-byte aligned
+    (3, 41, 8, 1, 2, 64, False),        # masks of several sequences, aligned
+    (3, 41, 3, 1, 1, 64, False),        # and not
+    (2, 37, 3, 0, 0, 256, True),
+    (4, 512, 8, 0, 0, 64, False),       # 16,384 units: the last size of 64-unit blocks
+    (1, 5462, 3, 0, 0, 64, False),      # 16,386: 128-unit blocks
+    (8, 512, 8, 0, 0, 64, False),       # 32,768
+    (3, 3641, 3, 0, 0, 64, False),      # 32,769: 256-unit blocks
+    (8, 1024, 8, 0, 0, 64, False),      # 65,536: the last direct scan
+    (1, 65537, 1, 0, 0, 64, False),     # the first chained one
+    (1, 65536, 1, 0, 0, 64, True),
+])
+def test_encoder_slot_scan_block_edges(B, npg, H, b0, pg0, D, paged):
+    """Raw-row slots at the edges of the slot scan's block sizes and mask layouts: every unit's
+    rowoff is the counter plus the raw rows of the units before it, the raw rows are in their
+    slots, and the counter and its value before are right."""
+    _say("slot scan edges", B, npg, H, b0, pg0, D, paged)
+    g = torch.Generator(device=DEV).manual_seed(B * npg + H)
+    x = torch.randn(B, npg * 16, H, D, generator=g, device=DEV).bfloat16()
+    rows = torch.rand(B, npg * 16, H, generator=g, device=DEV) < 0.02
+    x[rows, 3] *= 2.0 ** -30
+    c = exactkv.CompressedKV(b0 + B, (pg0 + npg) * 16, H, D, reserve=0.2)
+    c.cnt.fill_(5)
+    c.raw.zero_()
+    st = (x.stride(0), 16 * x.stride(1), x.stride(1), x.stride(2))
+    if paged:
+        NP = c.TS // 16
+        order = torch.randperm(c.B * NP, generator=g, device=DEV)[:B * npg].view(B, npg)
+        kernels.encode_pages_paged(x, st, c._buf(), order.to(torch.int32), B, npg)
+        pick = order.reshape(-1)
+        rm, off = (t.view(-1, H)[pick].view(B, npg, H) for t in (c.rowmask, c.rowoff))
+    else:
+        kernels.encode_pages(x, st, c._buf(), b0, pg0, B, npg)
+        rm, off = (t[b0:, pg0:] for t in (c.rowmask, c.rowoff))
+    bits = ((rm[..., None] >> torch.arange(16, device=DEV)) & 1).bool()        # [B, npg, H, 16]
+    assert bool((bits.permute(0, 1, 3, 2).reshape(rows.shape) | ~rows).all())
+    per = bits.sum(-1).reshape(-1)
+    excl = torch.cumsum(per, 0) - per + 5
+    assert torch.equal(off.reshape(-1).long(), excl)
+    n = int(per.sum())
+    assert int(c.cnt.item()) == 5 + n and int(c._before.item()) == 5
+    want = x.view(B, npg, 16, H, D).permute(0, 1, 3, 2, 4)[bits]               # (sequence, page, head, token) order
+    assert 5 + n <= c.cap and torch.equal(c.raw[5:5 + n].view(torch.int16), want.view(torch.int16))
+    assert not bool(c.raw[:5].view(torch.int16).any()) and not bool(c.raw[5 + n:c.cap].view(torch.int16).any())
