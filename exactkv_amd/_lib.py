@@ -6,6 +6,7 @@ library is missing or a call fails.
 """
 import ctypes
 import os
+import threading
 
 # EXACTKV_LIB overrides the path of the library to load (default: the in-tree build)
 _PATH = os.environ.get("EXACTKV_LIB") or os.path.join(os.path.dirname(os.path.abspath(__file__)), "libexactkv_hip.so")
@@ -22,6 +23,10 @@ SIGNATURES = {
                           _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _p, _i64, _p],
     "exkv_encode_pages_paged": [_p, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64,
                                 _i32, _p, _i64, _i32, _i32, _i32, _i32, _i32, _p, _i64, _p],
+    "exkv_prefill_slot": [_p, _i64, _i64, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _i32, _i32,
+                          _i32, _i32, _p, _i64, _p, _p],
+    "exkv_prefill_slot_paged": [_p, _i64, _i64, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _p, _i32, _i32,
+                                _i32, _i32, _i32, _i32, _p, _i64, _p, _p],
     "exkv_cache_append": [_p, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _i32, _i32,
                           _i32, _p],
     "exkv_bf16_append": [_p, _i64, _i64, _p, _p, _i32, _i32, _i32, _i32, _p],
@@ -139,15 +144,44 @@ _hip_rt = None
 _ERRBUF = {}
 
 
-def _stream_device(st):
-    """Device index of a raw HIP stream handle (the null stream: the current device)."""
+def _runtime():
+    """torch's HIP runtime, for the few calls made on raw streams here."""
     global _hip_rt
     if _hip_rt is None:
         import torch
-        _hip_rt = ctypes.CDLL(os.path.join(os.path.dirname(torch.__file__), "lib", "libamdhip64.so"))
-        _hip_rt.hipStreamGetDevice.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int)]
+        rt = ctypes.CDLL(os.path.join(os.path.dirname(torch.__file__), "lib", "libamdhip64.so"))
+        rt.hipStreamGetDevice.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int)]
+        rt.hipStreamSynchronize.argtypes = [ctypes.c_void_p]
+        _hip_rt = rt
+    return _hip_rt
+
+
+def synchronize(st):
+    """Wait for the work queued on raw stream `st`."""
+    if _runtime().hipStreamSynchronize(st) != 0:
+        raise RuntimeError("hipStreamSynchronize failed")
+
+
+_host = threading.local()
+
+
+def host_word(index):
+    """An int32 in pinned host memory that kernels on device `index` can write: (its address, a
+    ctypes view of it). One per thread and device, for calls that wait for their stream before
+    they return, so no two of them have it at a time."""
+    words = _host.__dict__.setdefault("words", {})
+    w = words.get(index)
+    if w is None:
+        import torch
+        t = torch.empty(1, dtype=torch.int32, pin_memory=True)
+        w = words[index] = (t.data_ptr(), ctypes.c_int32.from_address(t.data_ptr()), t)
+    return w[0], w[1]
+
+
+def _stream_device(st):
+    """Device index of a raw HIP stream handle (the null stream: the current device)."""
     d = ctypes.c_int(-1)
-    if _hip_rt.hipStreamGetDevice(st, ctypes.byref(d)) != 0:
+    if _runtime().hipStreamGetDevice(st, ctypes.byref(d)) != 0:
         raise RuntimeError("hipStreamGetDevice failed")
     return d.value
 
@@ -163,9 +197,7 @@ def stream_error_bits(st, clear=True):
     lib = load()
     if lib.exkv_error_bits(buf.data_ptr(), int(bool(clear)), st) != 0:
         raise RuntimeError("exkv_error_bits failed: " + lib.exkv_last_error().decode(errors="replace"))
-    _hip_rt.hipStreamSynchronize.argtypes = [ctypes.c_void_p]
-    if _hip_rt.hipStreamSynchronize(st) != 0:
-        raise RuntimeError("hipStreamSynchronize failed")
+    synchronize(st)
     return int(buf.cpu().item()) & 0xFFFFFFFF
 
 

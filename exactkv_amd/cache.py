@@ -28,7 +28,7 @@ How CompressedKV is organised here:
 import torch
 
 from . import _lib
-from .kernels import encode_pages, HEAD_DIMS, P
+from .kernels import encode_pages, prefill_pages, prefill_ready, HEAD_DIMS, P
 
 _FIELDS = ("sm", "code", "base", "rowmask", "rowoff", "raw")
 
@@ -132,6 +132,14 @@ class CompressedKV:
             raise AssertionError(f"{T} prompt tokens do not fit a cache of {self.TS}")
         full = T - T % P
         self.T = T
+        if 0 <= b < self.B and prefill_ready(x, self.sm.device, self.H, self.D):
+            used = prefill_pages(x, self._buf(), state=self.state, b=b)
+            if full and used > self.cap:
+                strides = (x.stride(0), P * x.stride(1), x.stride(1), x.stride(2))
+                used = self._refit(lambda: (x, strides), b, 0, 1, full // P)
+            self._keep_headroom(used)
+            return
+        # other sources: an empty prompt, rows of another type or device (less than a page of them)
         self.state[0] = T
         used = None
         if full:

@@ -555,8 +555,80 @@ __device__ inline int raw_rows_before(const EncArgs& a, int u0) {
     return sum;
 }
 
-template <bool PAGED, bool VEC16, int D>
-__global__ void __launch_bounds__(1024) scan_direct_kernel(EncArgs a, int nunits, int ub) {
+// What a prefill does besides encoding its full pages: the rows of its last, partly filled page
+// go to the slot's open-page rows, that page is opened, the device token count is set, and the
+// raw-row counter goes to the host. One more block of the scan's launch does it beside the
+// scan, in its shadow (30 KB of rows at 8 heads of 128), instead of a fill, a strided copy, an
+// open-page launch and a copy of the counter, each with its own gap around the host's wait for
+// the counter: a layer's K and V of a 4,091-token prompt 122 -> 61 us, of which the GPU works
+// 2 x 9.
+struct PrefillEnd {
+    const uint16_t* tail = nullptr;   // token 0 of the open page, head 0 (rows s_t apart, heads s_h)
+    int64_t s_t = 0, s_h = 0;
+    int rows = 0;                     // its tokens: T % 16
+    int64_t tail0 = 0;                // raw row of its token 0, head 0 (heads 16 rows apart)
+    int32_t* state = nullptr;         // contiguous: state[0] = T
+    int T = 0;
+    int B = 0;                        // contiguous: page T / 16 of every sequence is opened
+    int open_pages = 0;               // pages per sequence: none is opened at or past it
+    const int32_t* table = nullptr;   // paged: the slot's block-table row; its page T / 16 is opened
+    int64_t pool_pages = 0;
+    int32_t* host_cnt = nullptr;      // host memory (mapped): receives the counter
+};
+
+// One block of 1,024 threads.
+template <int D>
+__device__ inline void prefill_end(const EncArgs& a, const PrefillEnd& e) {
+    const int pg = e.T / kPage, H = a.H;
+    if (pg < e.open_pages) {
+        if (e.table != nullptr) {
+            const int64_t pidx = min((uint64_t)(uint32_t)e.table[pg], (uint64_t)(e.pool_pages - 1));
+            for (int h = threadIdx.x; h < H; h += 1024) {
+                a.rowmask[pidx * H + h] = 0xFFFF;
+                a.rowoff[pidx * H + h] = (int32_t)(e.tail0 + (int64_t)h * kPage);
+            }
+        } else {
+            for (int u = threadIdx.x; u < e.B * H; u += 1024) {
+                const int64_t page = ((int64_t)(u / H) * e.open_pages + pg) * H + u % H;
+                a.rowmask[page] = 0xFFFF;
+                a.rowoff[page] = (int32_t)(a.cap + (int64_t)u * kPage);
+            }
+        }
+    }
+    if (e.state != nullptr && threadIdx.x == 0) e.state[0] = e.T;
+    uint16_t* dst = a.raw + e.tail0 * D;
+    if ((uintptr_t)e.tail % 16 == 0 && e.s_t % 8 == 0 && e.s_h % 8 == 0) {   // uniform
+        for (int i = threadIdx.x; i < e.rows * H * (D / 8); i += 1024) {
+            const int c = i % (D / 8) * 8, h = i / (D / 8) % H, r = i / (D / 8) / H;
+            *reinterpret_cast<uint4*>(dst + ((int64_t)h * kPage + r) * D + c) =
+                *reinterpret_cast<const uint4*>(e.tail + r * e.s_t + h * e.s_h + c);
+        }
+    } else {
+        for (int i = threadIdx.x; i < e.rows * H * D; i += 1024) {
+            const int c = i % D, h = i / D % H, r = i / D / H;
+            dst[((int64_t)h * kPage + r) * D + c] = e.tail[r * e.s_t + h * e.s_h + c];
+        }
+    }
+}
+
+__device__ inline void tell_host(int32_t* p, int32_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// A prefill's end by itself: a prompt of less than a page, or one too long for the direct scan.
+template <int D>
+__global__ void __launch_bounds__(1024) prefill_end_kernel(EncArgs a, PrefillEnd e) {
+    prefill_end<D>(a, e);
+    if (threadIdx.x == 0) tell_host(e.host_cnt, *a.cnt);
+}
+
+// nscan blocks of ub units; END: one more, which does a prefill's end beside them.
+template <bool PAGED, bool VEC16, bool END, int D>
+__global__ void __launch_bounds__(1024) scan_direct_kernel(EncArgs a, int nunits, int ub, int nscan, PrefillEnd e) {
+    if (END && (int)blockIdx.x == nscan) {
+        prefill_end<D>(a, e);
+        return;
+    }
     __shared__ int s_before[16], s_own[16];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, per = ub >> 4;   // units per wavefront
     const int u0 = (int)blockIdx.x * ub, u = u0 + w * per + lane;
@@ -586,49 +658,62 @@ __global__ void __launch_bounds__(1024) scan_direct_kernel(EncArgs a, int nunits
     if (mine) a.rowoff[page] = off;
     if (threadIdx.x == 0) {
         if (blockIdx.x == 0 && a.before != nullptr) *a.before = cnt0;
-        if (blockIdx.x == gridDim.x - 1) *a.cnt = cnt0 + total;
+        if ((int)blockIdx.x == nscan - 1) {
+            *a.cnt = cnt0 + total;
+            if (END) tell_host(e.host_cnt, cnt0 + total);
+        }
     }
     copy_escaped_rows<VEC16, D>(a, m, off, a.src + bi * a.s_b + pg * a.s_pg + hk * a.s_h, lane);
 }
 
-template <int D>
-static void launch_direct(const EncArgs& a, int64_t n, bool paged, bool vec16, hipStream_t stream) {
-    const int ub = direct_block_units(n);
-    auto k = paged ? (vec16 ? scan_direct_kernel<true, true, D> : scan_direct_kernel<true, false, D>)
-                   : (vec16 ? scan_direct_kernel<false, true, D> : scan_direct_kernel<false, false, D>);
-    hipLaunchKernelGGL(k, dim3((unsigned)((n + ub - 1) / ub)), dim3(1024), 0, stream, a, (int)n, ub);
+template <int D, bool END>
+static void launch_direct(const EncArgs& a, int64_t n, bool paged, bool vec16, const PrefillEnd& e, hipStream_t stream) {
+    const int ub = direct_block_units(n), nscan = (int)((n + ub - 1) / ub);
+    auto k = paged ? (vec16 ? scan_direct_kernel<true, true, END, D> : scan_direct_kernel<true, false, END, D>)
+                   : (vec16 ? scan_direct_kernel<false, true, END, D> : scan_direct_kernel<false, false, END, D>);
+    hipLaunchKernelGGL(k, dim3((unsigned)(nscan + END)), dim3(1024), 0, stream, a, (int)n, ub, nscan, e);
 }
 
 // Encode n units: the page kernel, then the direct scan up to kDirectUnits units; above, the
 // chained scan when the workspace has at least 2 + ceil(n / kScanUnits) words, else the
-// three-launch scan.
+// three-launch scan. end: a prefill's end too, in the direct scan's launch or in one of its own.
 template <int D>
-static void launch_encode_d(const EncArgs& a, int64_t n, uint64_t* ws, int64_t ws_words, hipStream_t stream) {
+static void launch_encode_d(const EncArgs& a, int64_t n, uint64_t* ws, int64_t ws_words, const PrefillEnd* end,
+                            hipStream_t stream) {
+    if (n == 0) {
+        if (end) hipLaunchKernelGGL(prefill_end_kernel<D>, dim3(1), dim3(1024), 0, stream, a, *end);
+        return;
+    }
     hipLaunchKernelGGL(enc_pages_kernel<D>, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream, a, (int)n);
     const bool paged = a.dst_pages != nullptr;
     const bool vec16 = (uintptr_t)a.src % 16 == 0 && a.s_b % 8 == 0 && a.s_pg % 8 == 0 && a.s_p % 8 == 0 &&
                        a.s_h % 8 == 0;
     if (n <= kDirectUnits) {
-        launch_direct<D>(a, n, paged, vec16, stream);
+        if (end)
+            launch_direct<D, true>(a, n, paged, vec16, *end, stream);
+        else
+            launch_direct<D, false>(a, n, paged, vec16, PrefillEnd{}, stream);
         return;
     }
     const int64_t nb = (n + kScanUnits - 1) / kScanUnits;
     if (ws == nullptr || ws_words < 2 + nb) {
         launch_scan<D>(a, n, stream);
-        return;
+    } else {
+        auto k = paged ? (vec16 ? scan_chain_kernel<true, true, D> : scan_chain_kernel<true, false, D>)
+                       : (vec16 ? scan_chain_kernel<false, true, D> : scan_chain_kernel<false, false, D>);
+        hipLaunchKernelGGL(k, dim3((unsigned)nb), dim3(kScanUnits), 0, stream, a, (int)n, (int)nb, ws);
     }
-    auto k = paged ? (vec16 ? scan_chain_kernel<true, true, D> : scan_chain_kernel<true, false, D>)
-                   : (vec16 ? scan_chain_kernel<false, true, D> : scan_chain_kernel<false, false, D>);
-    hipLaunchKernelGGL(k, dim3((unsigned)nb), dim3(kScanUnits), 0, stream, a, (int)n, (int)nb, ws);
+    if (end) hipLaunchKernelGGL(prefill_end_kernel<D>, dim3(1), dim3(1024), 0, stream, a, *end);
 }
 
-static void launch_encode(const EncArgs& a, int64_t n, uint64_t* ws, int64_t ws_words, hipStream_t stream) {
+static void launch_encode(const EncArgs& a, int64_t n, uint64_t* ws, int64_t ws_words, const PrefillEnd* end,
+                          hipStream_t stream) {
     if (a.D == 64)
-        launch_encode_d<64>(a, n, ws, ws_words, stream);
+        launch_encode_d<64>(a, n, ws, ws_words, end, stream);
     else if (a.D == 256)
-        launch_encode_d<256>(a, n, ws, ws_words, stream);
+        launch_encode_d<256>(a, n, ws, ws_words, end, stream);
     else
-        launch_encode_d<128>(a, n, ws, ws_words, stream);
+        launch_encode_d<128>(a, n, ws, ws_words, end, stream);
 }
 
 // Copy one page's raw rows (token p's row at src + p*s_p, D channels) into slots rowoff + k (< cap).
@@ -1131,7 +1216,7 @@ extern "C" int exkv_encode_pages(const void* src, int64_t s_b, int64_t s_pg, int
     EncArgs a{(const uint16_t*)src, s_b, s_pg, s_p, s_h, (uint8_t*)sm, (uint8_t*)code, (uint8_t*)base,
               rowmask, rowoff, (uint16_t*)raw, cnt, before, cap, b0, pg0, nb, npg, H, TS};
     a.D = D;
-    launch_encode(a, n, (uint64_t*)scan_ws, scan_ws_words, stream);
+    launch_encode(a, n, (uint64_t*)scan_ws, scan_ws_words, nullptr, stream);
     return launch_status("encode_pages");
 }
 
@@ -1167,8 +1252,81 @@ extern "C" int exkv_encode_pages_paged(const void* src, int64_t s_b, int64_t s_p
     a.D = D;
     EXKV_REQUIRE(scan_ws == nullptr || (uintptr_t)scan_ws % 8 == 0,
                  "encode_pages_paged: scan workspace must be 8-byte aligned");
-    launch_encode(a, n, (uint64_t*)scan_ws, scan_ws_words, stream);
+    launch_encode(a, n, (uint64_t*)scan_ws, scan_ws_words, nullptr, stream);
     return launch_status("encode_pages_paged");
+}
+
+// A prompt into sequence slot b in two launches (one below a page of tokens): its full pages as
+// exkv_encode_pages encodes them, its last rows into the slot's open page, page T / 16 of every
+// sequence opened (exkv_cache_open_page), state[0] = T, *host_cnt = the raw-row counter.
+static int prefill_slot(const char* what, EncArgs& a, PrefillEnd& e, int64_t s_t, int64_t s_h, int32_t T, int64_t slot,
+                        int64_t slots, int64_t raw_rows, int32_t D, void* scan_ws, int64_t scan_ws_words,
+                        int32_t* host_cnt, hipStream_t stream) {
+    const int64_t tail_end = a.cap + slots * a.H * kPage;
+    EXKV_REQUIRE(a.cap >= 0 && tail_end <= raw_rows && tail_end <= INT32_MAX,
+                 "%s: raw pool (%lld rows) smaller than cap + open-page rows", what, (long long)raw_rows);
+    EXKV_REQUIRE(a.src && a.sm && a.code && a.base && a.rowmask && a.rowoff && a.raw && a.cnt && host_cnt,
+                 "%s: null pointer", what);
+    EXKV_REQUIRE(s_t >= 0 && s_h >= 0, "%s: negative source strides", what);
+    const int64_t n = (int64_t)a.npg * a.H;
+    EXKV_REQUIRE(n == 0 || ((uintptr_t)a.src % 4 == 0 && s_t % 2 == 0 && s_h % 2 == 0),
+                 "%s: source rows must start at even elements (4-byte aligned)", what);
+    EXKV_REQUIRE(n <= INT32_MAX - 1024, "%s: %lld pages x heads in one call (limit 2^31 - 1025)", what, (long long)n);
+    EXKV_REQUIRE(scan_ws == nullptr || (uintptr_t)scan_ws % 8 == 0, "%s: scan workspace must be 8-byte aligned", what);
+    a.D = D;
+    e.tail = a.src + (int64_t)a.npg * kPage * s_t;
+    e.s_t = s_t;
+    e.s_h = s_h;
+    e.rows = T % kPage;
+    e.tail0 = a.cap + slot * a.H * kPage;
+    e.T = T;
+    e.host_cnt = host_cnt;
+    launch_encode(a, n, (uint64_t*)scan_ws, scan_ws_words, &e, stream);
+    return launch_status(what);
+}
+
+extern "C" int exkv_prefill_slot(const void* src, int64_t s_t, int64_t s_h, int32_t T, void* sm, void* code, void* base,
+                                 int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before,
+                                 int32_t* state, int64_t cap, int64_t raw_rows, int32_t B, int32_t b, int32_t H,
+                                 int32_t TS, int32_t D, void* scan_ws, int64_t scan_ws_words, int32_t* host_cnt,
+                                 hipStream_t stream) {
+    EXKV_REQUIRE(head_dim_ok(D), "prefill_slot: head dim must be 64, 128 or 256 (got %d)", D);
+    EXKV_REQUIRE(TS > 0 && TS % kPage == 0 && B > 0 && H > 0, "prefill_slot: bad shape B=%d H=%d TS=%d", B, H, TS);
+    EXKV_REQUIRE(b >= 0 && b < B && T >= 0 && T <= TS, "prefill_slot: %d tokens into slot %d outside the cache", T, b);
+    EXKV_REQUIRE(state, "prefill_slot: null pointer");
+    EncArgs a{(const uint16_t*)src, 0, kPage * s_t, s_t, s_h, (uint8_t*)sm, (uint8_t*)code, (uint8_t*)base,
+              rowmask, rowoff, (uint16_t*)raw, cnt, before, cap, b, 0, 1, T / kPage, H, TS};
+    PrefillEnd e;
+    e.state = state;
+    e.B = B;
+    e.open_pages = TS / kPage;
+    return prefill_slot("prefill_slot", a, e, s_t, s_h, T, b, B, raw_rows, D, scan_ws, scan_ws_words, host_cnt, stream);
+}
+
+// The same into slot `slot` of a paged cache: its page p is pool page table[p] (entries clamped
+// to the pool), and page T / 16 is opened where the table has it.
+extern "C" int exkv_prefill_slot_paged(const void* src, int64_t s_t, int64_t s_h, int32_t T, void* sm, void* code,
+                                       void* base, int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt,
+                                       int32_t* before, int64_t cap, int64_t raw_rows, const int32_t* table,
+                                       int32_t slot, int32_t max_seqs, int32_t max_pages, int32_t pool_pages, int32_t H,
+                                       int32_t D, void* scan_ws, int64_t scan_ws_words, int32_t* host_cnt,
+                                       hipStream_t stream) {
+    EXKV_REQUIRE(head_dim_ok(D), "prefill_slot_paged: head dim must be 64, 128 or 256 (got %d)", D);
+    EXKV_REQUIRE(H > 0 && max_seqs > 0 && max_pages > 0 && pool_pages > 0, "prefill_slot_paged: bad shape");
+    EXKV_REQUIRE(slot >= 0 && slot < max_seqs && T >= 0 && T <= (int64_t)max_pages * kPage,
+                 "prefill_slot_paged: %d tokens into slot %d outside the cache", T, slot);
+    EXKV_REQUIRE(table, "prefill_slot_paged: null pointer");
+    EncArgs a{(const uint16_t*)src, 0, kPage * s_t, s_t, s_h, (uint8_t*)sm, (uint8_t*)code, (uint8_t*)base,
+              rowmask, rowoff, (uint16_t*)raw, cnt, before, cap, 0, 0, 1, T / kPage, H, kPage};
+    a.dst_pages = table;
+    a.dst_stride = max_pages;
+    a.all_pages = pool_pages;
+    PrefillEnd e;
+    e.open_pages = max_pages;
+    e.table = table;
+    e.pool_pages = pool_pages;
+    return prefill_slot("prefill_slot_paged", a, e, s_t, s_h, T, slot, max_seqs, raw_rows, D, scan_ws, scan_ws_words,
+                        host_cnt, stream);
 }
 
 extern "C" int exkv_cache_append(const void* x, int64_t sx_b, int64_t sx_h, void* sm, void* code, void* base,

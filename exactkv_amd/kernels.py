@@ -346,6 +346,7 @@ def _check_source(src, strides, nb, npg, H, D):
         raise ValueError(f"encode source too small: needs element {last}, has {avail}")
 
 
+DIRECT_UNITS = 65536   # pages x heads of one encode up to which its slot scan needs no workspace
 _SCAN = {}  # page-encoder scan workspaces per (device, stream)
 
 
@@ -375,7 +376,8 @@ def encode_pages(src, strides, buf, b0, pg0, nb, npg, *, chained=True):
     _check_source(src, strides, nb, npg, H, D)
     raw = buf["raw"]
     before = buf.get("before")
-    ws = _scan_ws(raw.device, int(nb) * int(npg) * H) if chained else None
+    units = int(nb) * int(npg) * H
+    ws = _scan_ws(raw.device, units) if chained and units > DIRECT_UNITS else None
     _lib.call("exkv_encode_pages", _lib.ptr(src, align=2, what="src"), *[int(s) for s in strides],
               _lib.ptr(buf["sm"]), _lib.ptr(buf["code"]), _lib.ptr(buf["base"]), _lib.ptr(buf["rowmask"]),
               _lib.ptr(buf["rowoff"]), _lib.ptr(raw), _lib.ptr(buf["cnt"], align=4),
@@ -395,13 +397,51 @@ def encode_pages_paged(src, strides, buf, dst_pages, nb, npg, *, chained=True):
         raise ValueError("dst_pages must be an int32 [nb, npg] tensor with unit column stride")
     raw = buf["raw"]
     before = buf.get("before")
-    ws = _scan_ws(raw.device, int(nb) * int(npg) * H) if chained else None
+    units = int(nb) * int(npg) * H
+    ws = _scan_ws(raw.device, units) if chained and units > DIRECT_UNITS else None
     _lib.call("exkv_encode_pages_paged", _lib.ptr(src, align=2, what="src"), *[int(s) for s in strides],
               _lib.ptr(buf["sm"]), _lib.ptr(buf["code"]), _lib.ptr(buf["base"]), _lib.ptr(buf["rowmask"]),
               _lib.ptr(buf["rowoff"]), _lib.ptr(raw), _lib.ptr(buf["cnt"], align=4),
               _lib.ptr(before, align=4) if before is not None else None, int(buf["cap"]), raw.shape[0],
               buf["sm"].shape[0], _lib.ptr(dst_pages, align=4, what="dst_pages"), dst_pages.stride(0), int(nb), int(npg), H,
               TS, D, _lib.ptr(ws), ws.numel() if ws is not None else 0, _lib.stream())
+
+
+def prefill_ready(x, dev, H, D):
+    """Whether prompt x [1, T, H, D] can go through prefill_pages as it stands: bf16 rows on the
+    cache's GPU, T > 0, and of the cache's shape where a part of a page is left over."""
+    T = x.shape[1] if x.dim() == 4 else 0
+    return (T > 0 and x.dtype == torch.bfloat16 and x.device == dev and x.stride(3) == 1
+            and (T % P == 0 or (x.shape[2] == H and x.shape[3] == D)))
+
+
+def prefill_pages(x, buf, *, state=None, b=0, table=None, slot=0, shape=None):
+    """Prompt x [1, T, H, D] (prefill_ready) into a cache, all of a prefill's device work in two
+    launches: full pages encoded, the rest into the open-page rows, that page opened, the token
+    count set. buf as for encode_pages. Contiguous: sequence b, state the device token count.
+    Paged: slot `slot`, table its row of the block table, shape (max_seqs, max_pages, pool
+    pages). Waits for the stream and returns the raw-row counter, which passes cap when the
+    pool overflowed, as after encode_pages."""
+    H, TS, D, T = buf["H"], buf["TS"], buf["D"], x.shape[1]
+    s_t, s_h = x.stride(1), x.stride(2)
+    if T >= P:
+        _check_source(x, (x.stride(0), P * s_t, s_t, s_h), 1, T // P, H, D)
+    raw, before = buf["raw"], buf["before"]
+    ws = _scan_ws(raw.device, (T // P) * H) if (T // P) * H > DIRECT_UNITS else None
+    st = _lib.stream()
+    word, count = _lib.host_word(raw.device.index)
+    args = (_lib.ptr(x, align=2, what="x"), s_t, s_h, T, _lib.ptr(buf["sm"]), _lib.ptr(buf["code"]), _lib.ptr(buf["base"]),
+            _lib.ptr(buf["rowmask"]), _lib.ptr(buf["rowoff"]), _lib.ptr(raw), _lib.ptr(buf["cnt"], align=4),
+            _lib.ptr(before, align=4))
+    scan = (_lib.ptr(ws), ws.numel() if ws is not None else 0, word, st)
+    if table is None:
+        _lib.call("exkv_prefill_slot", *args, _lib.ptr(state, align=4), int(buf["cap"]), raw.shape[0],
+                  buf["sm"].shape[0], int(b), H, TS, D, *scan)
+    else:
+        _lib.call("exkv_prefill_slot_paged", *args, int(buf["cap"]), raw.shape[0], _lib.ptr(table, align=4),
+                  int(slot), *shape, H, D, *scan)
+    _lib.synchronize(st)
+    return count.value
 
 
 def _paged_append_args(x, table, slots):

@@ -25,7 +25,8 @@ compact().
 import torch
 
 from . import _lib
-from .kernels import HEAD_DIMS, P, encode_pages_paged, append_paged, append_paged_bf16
+from .kernels import (HEAD_DIMS, P, append_paged, append_paged_bf16, encode_pages_paged, prefill_pages,
+                      prefill_ready)
 
 
 class PageTable:
@@ -234,7 +235,19 @@ class PagedCompressedKV:
         if T != self.table.length(slot):
             raise ValueError(f"prefill of {T} tokens into a slot of {self.table.length(slot)}")
         Tf = T // P * P
-        dst = self.table.block_table[slot: slot + 1]
+        t = self.table
+        dst = t.block_table[slot: slot + 1]
+        if prefill_ready(x, self.sm.device, self.H, self.D) and t.block_table.stride(0) == t.max_pages:
+            n = prefill_pages(x, self._buf(), table=dst, slot=slot, shape=(t.max_seqs, t.max_pages, t.num_pages))
+            if Tf and n > self.cap:
+                st = (x.stride(0), P * x.stride(1), x.stride(1), x.stride(2))
+                self._grow(n)
+                self.cnt.copy_(self._before)
+                self._encode_pages(x, st, dst, Tf // P)
+                n = int(self.cnt.item())
+                assert n <= self.cap
+            self._keep_headroom(n)
+            return
         if Tf:
             st = (x.stride(0), P * x.stride(1), x.stride(1), x.stride(2))
             self._encode_pages(x, st, dst, Tf // P)

@@ -88,6 +88,27 @@ int exkv_encode_pages(const void* src, int64_t s_b, int64_t s_pg, int64_t s_p, i
                       int32_t b0, int32_t pg0, int32_t nb, int32_t npg, int32_t H, int32_t TS,
                       int32_t D, void* scan_ws, int64_t scan_ws_words, hipStream_t stream);
 
+/* A prompt into sequence slot b of a cache: T tokens x H heads of `src` (bf16, element strides
+ * s_t, s_h for token and head; channels contiguous). Its T / 16 full pages are encoded as by
+ * exkv_encode_pages; the other rows go to the slot's open-page rows, raw rows
+ * cap + (b*H + h)*16 on; page T / 16 of every sequence is opened as by exkv_cache_open_page;
+ * state[0] = T; and *host_cnt (host memory that the GPU can write, such as hipHostMalloc's)
+ * receives the raw-row counter, valid once the stream has been waited for (*host_cnt > cap:
+ * overflow, as for exkv_encode_pages). Two launches up to 65,536 pages x heads.
+ * Replaces: cache.py:87-98 (encode, open-page copy) and the counter read that follows. */
+int exkv_prefill_slot(const void* src, int64_t s_t, int64_t s_h, int32_t T, void* sm, void* code, void* base,
+                      int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before, int32_t* state,
+                      int64_t cap, int64_t raw_rows, int32_t B, int32_t b, int32_t H, int32_t TS, int32_t D,
+                      void* scan_ws, int64_t scan_ws_words, int32_t* host_cnt, hipStream_t stream);
+
+/* The same into slot `slot` of a paged cache whose page p is pool page table[p] (max_pages
+ * entries, clamped to the pool); page T / 16 of the slot is opened where the table has it. */
+int exkv_prefill_slot_paged(const void* src, int64_t s_t, int64_t s_h, int32_t T, void* sm, void* code, void* base,
+                            int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before, int64_t cap,
+                            int64_t raw_rows, const int32_t* table, int32_t slot, int32_t max_seqs,
+                            int32_t max_pages, int32_t pool_pages, int32_t H, int32_t D, void* scan_ws,
+                            int64_t scan_ws_words, int32_t* host_cnt, hipStream_t stream);
+
 /* The page encoder into a paged cache: page pg of source sequence bi goes to page
  * dst_pages[bi*dst_stride + pg] of the B x TS arrays read as a list of B*TS/16 pages (entries
  * clamped to it). Same bytes and raw-slot order as exkv_encode_pages, and the same scan

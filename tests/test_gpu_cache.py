@@ -113,3 +113,57 @@ def test_append_page_ends_with_many_units_and_raw_rows(B, H, T0, TS, rate):
             _state_equal(c, m, t)
             ends += 1
     assert ends >= 2
+
+
+def _layout(x, kind):
+    """x [1, T, H, D] with other strides or alignment, same values."""
+    if kind == "heads":                                  # [1, H, T, D] as the attention modules give it
+        return x.transpose(1, 2).contiguous().transpose(1, 2)
+    if kind == "pairs":                                  # rows 4-byte aligned
+        flat = torch.empty(x.numel() + 2, dtype=x.dtype, device=x.device)[2:].view(x.shape)
+        return flat.copy_(x)
+    if kind == "odd":                                    # rows 2-byte aligned (less than a page only)
+        flat = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)[1:].view(x.shape)
+        return flat.copy_(x)
+    if kind == "wide":                                   # a slice of more heads and channels
+        big = torch.zeros(1, x.shape[1], x.shape[2] + 3, x.shape[3] + 8, dtype=x.dtype, device=x.device)
+        big[:, :, 1:1 + x.shape[2], :x.shape[3]] = x
+        return big[:, :, 1:1 + x.shape[2], :x.shape[3]]
+    return x
+
+
+@pytest.mark.parametrize("T,H,D,kind,reserve", [
+    (1, 8, 128, "plain", 0.5), (15, 3, 64, "odd", 0.5), (16, 8, 128, "plain", 0.5), (17, 5, 256, "heads", 0.5),
+    (95, 8, 128, "heads", 0.5), (96, 8, 128, "plain", 0.5), (250, 3, 64, "pairs", 0.5), (333, 2, 128, "wide", 0.5),
+    (8191, 9, 64, "heads", 0.3),                         # 4,599 units
+    (1000, 8, 128, "heads", 0.0),                        # the pool overflows and grows
+])
+@pytest.mark.parametrize("paged", [False, True])
+def test_prefill_in_one_call_equals_its_parts(T, H, D, kind, reserve, paged, monkeypatch):
+    """prefill_slot's one call (pages, open page, token count, counter) leaves every array as
+    the encoder, the page opening and the row copy leave it one after the other."""
+    from exactkv_amd import cache as mcache, paged as mpaged
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn(1, T, H, D, generator=g, device=DEV).bfloat16()
+    x[0, torch.rand(T, H, generator=g, device=DEV) < 0.1, 5] *= 2.0 ** -30
+    x = _layout(x, kind)
+    got = []
+    for parts in (False, True):
+        if parts:
+            monkeypatch.setattr(mcache, "prefill_ready", lambda *a: False)
+            monkeypatch.setattr(mpaged, "prefill_ready", lambda *a: False)
+        if paged:
+            table = exactkv.PageTable(3 * (T // 16 + 2), 3, T // 16 + (1 if T % 16 else 0) or 1)
+            c = exactkv.PagedCompressedKV(table, H, D=D, reserve=reserve)
+            for other in (40, T):
+                c.prefill(table.add(min(other, T)), x[:, :min(other, T)])
+        else:
+            c = exactkv.CompressedKV(2, -(-T // 16) * 16, H, D, reserve=reserve)
+            c.prefill_slot(0, x)
+            c.prefill_slot(1, x.flip(1) if kind == "plain" else x)
+            got.append((c.T, c.state))
+        got.append((c.cap, c.grows, c.sm, c.code, c.base, c.rowmask, c.rowoff, c.cnt, c._before,
+                    c.raw.view(torch.int16)))
+    half = len(got) // 2
+    for a, b in zip(sum(got[:half], ()), sum(got[half:], ())):
+        assert torch.equal(a, b) if isinstance(a, torch.Tensor) else a == b
