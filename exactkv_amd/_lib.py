@@ -23,6 +23,8 @@ SIGNATURES = {
                           _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _p, _i64, _p],
     "exkv_encode_pages_paged": [_p, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64,
                                 _i32, _p, _i64, _i32, _i32, _i32, _i32, _i32, _p, _i64, _p],
+    "exkv_store_raw_rows": [_p, _i64, _i64, _i64, _i64, _p, _p, _p, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32,
+                            _i32, _i32, _p],
     "exkv_prefill_slot": [_p, _i64, _i64, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _i32, _i32,
                           _i32, _i32, _p, _i64, _p, _p],
     "exkv_prefill_slot_paged": [_p, _i64, _i64, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _p, _i32, _i32,

@@ -21,7 +21,7 @@ CPU implementation in this package.
 """
 import torch
 
-from .kernels import encode_pages, decode_to_bf16, HEAD_DIMS, P
+from .kernels import encode_pages, store_raw_rows, decode_to_bf16, HEAD_DIMS, P
 
 
 def _gpu(dev):
@@ -49,13 +49,12 @@ def encode_reference(x):
                rowoff=torch.empty(B, NP, H, **i32), cnt=torch.zeros(1, **i32), cap=0, TS=T, H=H, D=D,
                raw=torch.empty(1, D, dtype=torch.bfloat16, device=dev))
     st = (xd.stride(0), P * xd.stride(1), xd.stride(1), xd.stride(2))
-    encode_pages(xd, st, buf, 0, 0, B, NP)                 # pass 1: layout and raw-row count
+    encode_pages(xd, st, buf, 0, 0, B, NP)                 # the layout and the raw rows' number (none stored)
     n = int(buf["cnt"].item())
     if n:
         buf["raw"] = torch.empty(n, D, dtype=torch.bfloat16, device=dev)
         buf["cap"] = n
-        buf["cnt"].zero_()
-        encode_pages(xd, st, buf, 0, 0, B, NP)             # pass 2: same bytes, raw rows stored
+        store_raw_rows(xd, st, buf, 0, 0, B, NP)           # into slots that the layout already has
     raw = buf["raw"][:n]
     out = dict(shape=(B, T, H, D), sm=buf["sm"], code=buf["code"], base=buf["base"], rowmask=buf["rowmask"],
                rowoff=buf["rowoff"], raw=raw)

@@ -371,12 +371,15 @@ __global__ void __launch_bounds__(1024) scan_write_kernel(EncArgs a, int nunits)
     copy_escaped_rows<VEC16, D>(a, m, off, a.src + bi * a.s_b + pg * a.s_pg + hk * a.s_h, threadIdx.x & 63);
 }
 
+// Whether every source row starts at a multiple of 16 bytes.
+static bool rows_of_16_bytes(const EncArgs& a) {
+    return (uintptr_t)a.src % 16 == 0 && a.s_b % 8 == 0 && a.s_pg % 8 == 0 && a.s_p % 8 == 0 && a.s_h % 8 == 0;
+}
+
 template <int D>
 static void launch_scan(const EncArgs& a, int64_t n, hipStream_t stream) {
     const unsigned nb = (unsigned)((n + kScanUnits - 1) / kScanUnits);
-    const bool paged = a.dst_pages != nullptr;
-    const bool vec16 = (uintptr_t)a.src % 16 == 0 && a.s_b % 8 == 0 && a.s_pg % 8 == 0 && a.s_p % 8 == 0 &&
-                       a.s_h % 8 == 0;
+    const bool paged = a.dst_pages != nullptr, vec16 = rows_of_16_bytes(a);
     if (paged)
         hipLaunchKernelGGL(scan_count_kernel<true>, dim3(nb), dim3(1024), 0, stream, a, (int)n);
     else
@@ -663,7 +666,7 @@ __global__ void __launch_bounds__(1024) scan_direct_kernel(EncArgs a, int nunits
             if (END) tell_host(e.host_cnt, cnt0 + total);
         }
     }
-    copy_escaped_rows<VEC16, D>(a, m, off, a.src + bi * a.s_b + pg * a.s_pg + hk * a.s_h, lane);
+    if (a.cap > 0) copy_escaped_rows<VEC16, D>(a, m, off, a.src + bi * a.s_b + pg * a.s_pg + hk * a.s_h, lane);
 }
 
 template <int D, bool END>
@@ -685,9 +688,7 @@ static void launch_encode_d(const EncArgs& a, int64_t n, uint64_t* ws, int64_t w
         return;
     }
     hipLaunchKernelGGL(enc_pages_kernel<D>, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream, a, (int)n);
-    const bool paged = a.dst_pages != nullptr;
-    const bool vec16 = (uintptr_t)a.src % 16 == 0 && a.s_b % 8 == 0 && a.s_pg % 8 == 0 && a.s_p % 8 == 0 &&
-                       a.s_h % 8 == 0;
+    const bool paged = a.dst_pages != nullptr, vec16 = rows_of_16_bytes(a);
     if (n <= kDirectUnits) {
         if (end)
             launch_direct<D, true>(a, n, paged, vec16, *end, stream);
@@ -714,6 +715,29 @@ static void launch_encode(const EncArgs& a, int64_t n, uint64_t* ws, int64_t ws_
         launch_encode_d<256>(a, n, ws, ws_words, end, stream);
     else
         launch_encode_d<128>(a, n, ws, ws_words, end, stream);
+}
+
+// The raw rows of pages that are already encoded (rowmask and rowoff in place) into their slots:
+// what a call whose pool was too small, or of size 0 to count the rows first, has left to do. A
+// wavefront takes kStoreUnits units, so that the copies, each a dependent round trip after the
+// masks, spread over the chip; encoding the pages again for it was as long as the first time
+// (16 x 4096 tokens x 8 heads: 49 us against 4.7).
+constexpr int kStoreUnits = 16;
+
+template <bool VEC16, int D>
+__global__ void __launch_bounds__(256) store_raw_kernel(EncArgs a, int nunits) {
+    const int lane = threadIdx.x & 63;
+    const int u = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * kStoreUnits + lane;
+    int bi = 0, pg = 0, hk = 0;
+    uint32_t m = 0;
+    int32_t off = 0;
+    if (lane < kStoreUnits && u < nunits) {
+        const int64_t page = unit_page32<false>(a, u, bi, pg, hk);
+        m = (uint32_t)a.rowmask[page];
+        off = a.rowoff[page];
+        if (off < 0) m = 0;                            // not this encoder's: outside the pool
+    }
+    copy_escaped_rows<VEC16, D>(a, m & 0xFFFFu, off, a.src + bi * a.s_b + pg * a.s_pg + hk * a.s_h, lane);
 }
 
 // Copy one page's raw rows (token p's row at src + p*s_p, D channels) into slots rowoff + k (< cap).
@@ -1191,33 +1215,70 @@ static int launch_status(const char* what) { return hip_status(hipGetLastError()
 // The instance of kernel template K for head dim D (64, 128 or 256; checked by the caller).
 #define EXKV_FOR_D(K, D) ((D) == 64 ? K<64> : (D) == 256 ? K<256> : K<128>)
 
+static int check_encode(const char* what, const void* src, int64_t s_b, int64_t s_pg, int64_t s_p, int64_t s_h,
+                        bool pointers, int64_t cap, int64_t raw_rows, int32_t B, int32_t b0, int32_t pg0, int32_t nb,
+                        int32_t npg, int32_t H, int32_t TS, int32_t D) {
+    EXKV_REQUIRE(head_dim_ok(D), "%s: head dim must be 64, 128 or 256 (got %d)", what, D);
+    EXKV_REQUIRE(TS > 0 && TS % kPage == 0, "%s: TS must be a positive multiple of 16 (got %d)", what, TS);
+    EXKV_REQUIRE(H > 0 && B > 0, "%s: bad H=%d or B=%d", what, H, B);
+    EXKV_REQUIRE(nb >= 0 && npg >= 0 && b0 >= 0 && pg0 >= 0, "%s: negative range", what);
+    EXKV_REQUIRE(b0 + nb <= B, "%s: sequences [%d, %d) outside the cache (B=%d)", what, b0, b0 + nb, B);
+    EXKV_REQUIRE(pg0 + npg <= TS / kPage, "%s: pages [%d, %d) outside the cache (%d pages)", what, pg0, pg0 + npg,
+                 TS / kPage);
+    EXKV_REQUIRE(cap >= 0 && cap <= raw_rows, "%s: cap %lld exceeds the raw pool (%lld rows)", what, (long long)cap,
+                 (long long)raw_rows);
+    EXKV_REQUIRE(src && pointers, "%s: null pointer", what);
+    EXKV_REQUIRE((uintptr_t)src % 4 == 0 && s_b % 2 == 0 && s_pg % 2 == 0 && s_p % 2 == 0 && s_h % 2 == 0,
+                 "%s: source rows must start at even elements (4-byte aligned)", what);
+    const int64_t n = (int64_t)nb * npg * H;
+    EXKV_REQUIRE(n <= INT32_MAX - 1024, "%s: %lld pages x heads in one call (limit 2^31 - 1025)", what, (long long)n);
+    return EXKV_OK;
+}
+
 extern "C" int exkv_encode_pages(const void* src, int64_t s_b, int64_t s_pg, int64_t s_p, int64_t s_h,
                                  void* sm, void* code, void* base, int32_t* rowmask, int32_t* rowoff, void* raw,
                                  int32_t* cnt, int32_t* before, int64_t cap, int64_t raw_rows, int32_t B,
                                  int32_t b0, int32_t pg0, int32_t nb, int32_t npg, int32_t H, int32_t TS,
                                  int32_t D, void* scan_ws, int64_t scan_ws_words, hipStream_t stream) {
-    EXKV_REQUIRE(head_dim_ok(D), "encode_pages: head dim must be 64, 128 or 256 (got %d)", D);
-    EXKV_REQUIRE(TS > 0 && TS % kPage == 0, "encode_pages: TS must be a positive multiple of 16 (got %d)", TS);
-    EXKV_REQUIRE(H > 0 && B > 0, "encode_pages: bad H=%d or B=%d", H, B);
-    EXKV_REQUIRE(nb >= 0 && npg >= 0 && b0 >= 0 && pg0 >= 0, "encode_pages: negative range");
-    EXKV_REQUIRE(b0 + nb <= B, "encode_pages: sequences [%d, %d) outside the cache (B=%d)", b0, b0 + nb, B);
-    EXKV_REQUIRE(pg0 + npg <= TS / kPage, "encode_pages: pages [%d, %d) outside the cache (%d pages)", pg0,
-                 pg0 + npg, TS / kPage);
-    EXKV_REQUIRE(cap >= 0 && cap <= raw_rows, "encode_pages: cap %lld exceeds the raw pool (%lld rows)",
-                 (long long)cap, (long long)raw_rows);
-    EXKV_REQUIRE(src && sm && code && base && rowmask && rowoff && raw && cnt, "encode_pages: null pointer");
-    EXKV_REQUIRE((uintptr_t)src % 4 == 0 && s_b % 2 == 0 && s_pg % 2 == 0 && s_p % 2 == 0 && s_h % 2 == 0,
-                 "encode_pages: source rows must start at even elements (4-byte aligned)");
+    const int rc = check_encode("encode_pages", src, s_b, s_pg, s_p, s_h,
+                                sm && code && base && rowmask && rowoff && raw && cnt, cap, raw_rows, B, b0, pg0, nb, npg,
+                                H, TS, D);
+    if (rc != EXKV_OK) return rc;
     const int64_t n = (int64_t)nb * npg * H;
     if (n == 0) return EXKV_OK;
-    EXKV_REQUIRE(n <= INT32_MAX - 1024, "encode_pages: %lld pages x heads in one call (limit 2^31 - 1025)",
-                 (long long)n);
     EXKV_REQUIRE(scan_ws == nullptr || (uintptr_t)scan_ws % 8 == 0, "encode_pages: scan workspace must be 8-byte aligned");
     EncArgs a{(const uint16_t*)src, s_b, s_pg, s_p, s_h, (uint8_t*)sm, (uint8_t*)code, (uint8_t*)base,
               rowmask, rowoff, (uint16_t*)raw, cnt, before, cap, b0, pg0, nb, npg, H, TS};
     a.D = D;
     launch_encode(a, n, (uint64_t*)scan_ws, scan_ws_words, nullptr, stream);
     return launch_status("encode_pages");
+}
+
+template <int D>
+static void launch_store_raw(const EncArgs& a, int64_t n, hipStream_t stream) {
+    const unsigned grid = (unsigned)((n + 4 * kStoreUnits - 1) / (4 * kStoreUnits));
+    auto k = rows_of_16_bytes(a) ? store_raw_kernel<true, D> : store_raw_kernel<false, D>;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, stream, a, (int)n);
+}
+
+extern "C" int exkv_store_raw_rows(const void* src, int64_t s_b, int64_t s_pg, int64_t s_p, int64_t s_h,
+                                   const int32_t* rowmask, const int32_t* rowoff, void* raw, int64_t cap,
+                                   int64_t raw_rows, int32_t B, int32_t b0, int32_t pg0, int32_t nb, int32_t npg,
+                                   int32_t H, int32_t TS, int32_t D, hipStream_t stream) {
+    const int rc = check_encode("store_raw_rows", src, s_b, s_pg, s_p, s_h, rowmask && rowoff && raw, cap, raw_rows, B,
+                                b0, pg0, nb, npg, H, TS, D);
+    if (rc != EXKV_OK) return rc;
+    const int64_t n = (int64_t)nb * npg * H;
+    if (n == 0) return EXKV_OK;
+    EncArgs a{(const uint16_t*)src, s_b, s_pg, s_p, s_h, nullptr, nullptr, nullptr, const_cast<int32_t*>(rowmask),
+              const_cast<int32_t*>(rowoff), (uint16_t*)raw, nullptr, nullptr, cap, b0, pg0, nb, npg, H, TS};
+    if (D == 64)
+        launch_store_raw<64>(a, n, stream);
+    else if (D == 256)
+        launch_store_raw<256>(a, n, stream);
+    else
+        launch_store_raw<128>(a, n, stream);
+    return launch_status("store_raw_rows");
 }
 
 // Pages of nb source sequences x npg pages into arbitrary pages of B x TS caches read as a

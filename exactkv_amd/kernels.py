@@ -386,6 +386,17 @@ def encode_pages(src, strides, buf, b0, pg0, nb, npg, *, chained=True):
               ws.numel() if ws is not None else 0, _lib.stream())
 
 
+def store_raw_rows(src, strides, buf, b0, pg0, nb, npg):
+    """The raw rows of pages that encode_pages has encoded with the same arguments, into their
+    slots of buf's raw pool (of rows below cap): for a pool that was sized after the encode."""
+    H, TS, D = buf["H"], buf["TS"], buf["D"]
+    _check_source(src, strides, nb, npg, H, D)
+    raw = buf["raw"]
+    _lib.call("exkv_store_raw_rows", _lib.ptr(src, align=2, what="src"), *[int(s) for s in strides],
+              _lib.ptr(buf["rowmask"]), _lib.ptr(buf["rowoff"]), _lib.ptr(raw), int(buf["cap"]), raw.shape[0],
+              buf["sm"].shape[0], int(b0), int(pg0), int(nb), int(npg), H, TS, D, _lib.stream())
+
+
 def encode_pages_paged(src, strides, buf, dst_pages, nb, npg, *, chained=True):
     """encode_pages into a paged cache: page pg of source sequence bi (strides as in
     encode_pages) goes to page dst_pages[bi, pg] of the cache's arrays read as a list of

@@ -88,6 +88,15 @@ int exkv_encode_pages(const void* src, int64_t s_b, int64_t s_pg, int64_t s_p, i
                       int32_t b0, int32_t pg0, int32_t nb, int32_t npg, int32_t H, int32_t TS,
                       int32_t D, void* scan_ws, int64_t scan_ws_words, hipStream_t stream);
 
+/* The raw rows of pages that exkv_encode_pages has encoded from the same source (rowmask and
+ * rowoff in place) into raw, in their slots below cap: after a call whose pool was too small,
+ * or of capacity 0 to learn the count. One launch.
+ * Part of what replaces: codec.py:50-53. */
+int exkv_store_raw_rows(const void* src, int64_t s_b, int64_t s_pg, int64_t s_p, int64_t s_h,
+                        const int32_t* rowmask, const int32_t* rowoff, void* raw, int64_t cap, int64_t raw_rows,
+                        int32_t B, int32_t b0, int32_t pg0, int32_t nb, int32_t npg, int32_t H, int32_t TS,
+                        int32_t D, hipStream_t stream);
+
 /* A prompt into sequence slot b of a cache: T tokens x H heads of `src` (bf16, element strides
  * s_t, s_h for token and head; channels contiguous). Its T / 16 full pages are encoded as by
  * exkv_encode_pages; the other rows go to the slot's open-page rows, raw rows

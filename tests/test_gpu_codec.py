@@ -252,3 +252,23 @@ def test_encoder_slot_scan_block_edges(B, npg, H, b0, pg0, D, paged):
     want = x.view(B, npg, 16, H, D).permute(0, 1, 3, 2, 4)[bits]               # (sequence, page, head, token) order
     assert 5 + n <= c.cap and torch.equal(c.raw[5:5 + n].view(torch.int16), want.view(torch.int16))
     assert not bool(c.raw[:5].view(torch.int16).any()) and not bool(c.raw[5 + n:c.cap].view(torch.int16).any())
+
+
+@pytest.mark.parametrize("B,T,H,D,rate", [(1, 16, 1, 64, 1.0), (2, 160, 3, 128, 0.2), (3, 1040, 5, 256, 0.02),
+                                          (1, 4096, 8, 128, 1.0), (4, 2048, 8, 64, 0.0)])
+@pytest.mark.parametrize("shift", [0, 2])
+def test_store_raw_rows_equals_a_second_encode(B, T, H, D, rate, shift):
+    """Raw rows stored after an encode that had no room for them are those of an encode that
+    had; the ones past cap are left out."""
+    g = torch.Generator(device=DEV).manual_seed(T + H)
+    x = torch.empty(B * T * H * D + shift, dtype=torch.bfloat16, device=DEV)[shift:].view(B, T, H, D)
+    x.copy_(torch.randn(B, T, H, D, generator=g, device=DEV))
+    x[torch.rand(B, T, H, generator=g, device=DEV) < rate, 1] *= 2.0 ** -30
+    st = (x.stride(0), 16 * x.stride(1), x.stride(1), x.stride(2))
+    c = exactkv.CompressedKV(B, T, H, D, reserve=1.0)
+    kernels.encode_pages(x, st, c._buf(), 0, 0, B, T // 16)
+    n = int(c.cnt.item())
+    for cap in {n, n // 2}:
+        buf = dict(c._buf(), cap=cap, raw=torch.zeros(n + 1, D, dtype=torch.bfloat16, device=DEV))
+        kernels.store_raw_rows(x, st, buf, 0, 0, B, T // 16)
+        assert same_bits(buf["raw"][:cap], c.raw[:cap]) and not bool(buf["raw"][cap:].view(torch.int16).any())
