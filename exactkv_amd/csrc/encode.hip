@@ -16,9 +16,9 @@
 //                          kernels.py:262), then the raw rows into their slots, skipping
 //                          slots >= cap (kernels.py:265-268), so an overflow is seen from
 //                          the counter.
-// The append path (cache.py:100-112) runs a write (+ page encode), a one-workgroup slot
-// scan and a raw-row copy with the token count read from device memory, so a decode step
-// can be captured in a HIP graph. Every kernel that touches rows is a template on the
+// The append path (cache.py:100-112) is one launch (row writes; at page ends the page encode,
+// the slot scan and the raw-row copies) with the token count read from device memory, so a
+// decode step can be captured in a HIP graph. Every kernel that touches rows is a template on the
 // head dim (64, 128 or 256); the entry points pick the instance.
 #include "tile.hpp"
 #include "../../include/exactkv.h"
@@ -740,22 +740,6 @@ __global__ void __launch_bounds__(256) store_raw_kernel(EncArgs a, int nunits) {
     copy_escaped_rows<VEC16, D>(a, m & 0xFFFFu, off, a.src + bi * a.s_b + pg * a.s_pg + hk * a.s_h, lane);
 }
 
-// Copy one page's raw rows (token p's row at src + p*s_p, D channels) into slots rowoff + k (< cap).
-template <int D>
-__device__ inline void copy_raw_rows(const uint16_t* src, int64_t s_p, uint32_t m, int32_t off, int64_t cap,
-                                     uint16_t* raw, int lane) {
-    int k = 0;
-    for (int p = 0; p < kPage; ++p) {
-        if (!((m >> p) & 1u)) continue;
-        const int64_t slot = (int64_t)off + k++;
-        if (slot >= cap) continue;
-        const uint16_t* s = src + p * s_p;
-        uint16_t* d = raw + slot * D;
-#pragma unroll
-        for (int c = 0; c < D; c += 64) d[c + lane] = s[c + lane];
-    }
-}
-
 // Row of D channels: d[c] = s[c], lanes striding by 64.
 template <int D>
 __device__ inline void copy_row(uint16_t* d, const uint16_t* s, int lane) {
@@ -792,12 +776,20 @@ struct AppendArgs {
 // (tokens 0-14 from the tail area, written by earlier appends; token 15 from x), sets
 // *before and *cnt, and advances state[0]. Replaces three launches (write and encode, slot
 // scan, raw-row copy), measured 0.87 ms of a c4 decode step for 64 caches.
+//
+// ONE: a grid of one block, up to kAppendOne units, where nothing is counted in. An ordinary step
+// is then one round trip (the token count and the rows, loaded together) and its stores, and
+// is bound by those and the launch. Back-to-back launches, one wavefront per row of 2-byte
+// lanes and a count in every step / now: 8 units 3.6 / 2.0 us, 64 4.4 / 2.35, 128 4.8 / 3.2 (8
+// blocks), 4,960 5.7 / 4.0. At a page end a block's 16 wavefronts encode its pages in turn (64
+// units 10-13 us in four blocks, 15-17 in one, one step in 16), hence the limit.
 constexpr int kAppendThreads = 1024;
+constexpr int kAppendWaves = kAppendThreads / 64;
 // At most this many blocks: every block's arrival is an atomic on one word, and those
 // serialise (measured at c4, 64 caches per step: 256 blocks 10.2 us per launch); the
 // waves loop over the units instead.
 constexpr int kAppendBlocks = 64;
-constexpr int kAppendBatch = 8;                     // token rows a wave has in flight
+constexpr int kAppendOne = 64;
 
 __device__ inline void st_dev_i32(int32_t* p, int32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -833,48 +825,51 @@ __device__ inline void copy_row_thread(uint16_t* dst, const uint16_t* src) {
     }
 }
 
-// The last block's share of a page end (all kAppendThreads threads call it). Thread t takes
+// Raw-row slots and rows of n units whose pages have just been encoded (all kAppendThreads
+// threads of one block call it), in unit order from slot cnt0 on: `units` gives the index of a
+// unit's page and the source of its row r. Thread t takes
 // units [t * per, (t + 1) * per): their rowmasks (device-coherent loads, eight in flight),
-// the block's exclusive scan of their raw-row counts from *cnt (the codec's slot order),
+// the block's exclusive scan of their raw-row counts (the codec's slot order),
 // rowoff. Then the raw rows (rows 0-14 from the unit's tail area, written by earlier
-// appends; row 15 from x): with up to kAppendLdsUnits units, spread over the threads one row
+// appends; row 15 from x): with up to LDSU units, spread over the threads one row
 // each -- the units' first raw-row ranks go to LDS and the thread holding raw row g finds its
 // unit by binary search -- so that a page end costs about one round trip; with more units,
 // each thread moves its own units' rows. Rows at or past cap are not written (the counter
-// shows the overflow).
+// shows the overflow). Returns the number of raw rows.
 constexpr int kAppendLdsUnits = 8192;
 
-template <int D>
-__device__ inline void append_slots(const AppendArgs& a, int T) {
-    __shared__ int s_rank[kAppendLdsUnits + 1];
-    __shared__ uint16_t s_mask[kAppendLdsUnits];
-    const int n = a.B * a.H, NP = a.TS / kPage, pg = T / kPage;
+struct RawPool {
+    const int32_t* rowmask;
+    int32_t* rowoff;
+    uint16_t* raw;
+    int64_t cap;
+};
+
+template <int D, int LDSU, class Units>
+__device__ inline int place_raw_rows(const Units& units, int n, int cnt0, const RawPool& pool) {
+    __shared__ int s_rank[LDSU + 1];
+    __shared__ uint16_t s_mask[LDSU];
     const int per = (n + kAppendThreads - 1) / kAppendThreads;
     const int u0 = min((int)threadIdx.x * per, n), u1 = min(u0 + per, n);
-    auto page_of = [&](int u) { return ((int64_t)(u / a.H) * NP + pg) * a.H + u % a.H; };
-    auto src_row = [&](int u, int r) -> const uint16_t* {
-        return r == kPage - 1 ? a.x + (u / a.H) * a.sx_b + (u % a.H) * a.sx_h
-                              : a.raw + (a.cap + (int64_t)u * kPage + r) * D;
-    };
-    const bool table = n <= kAppendLdsUnits;          // uniform
-    const int cnt0 = *a.cnt;
+    const bool table = n <= LDSU;                     // uniform
     int local = 0;
-    for (int c0 = u0; c0 < u1; c0 += 8) {
-        uint32_t m[8];
+    uint32_t m[8];
+    auto masks = [&](int c0) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k) m[k] = c0 + k < u1 ? (uint32_t)ld_dev_i32(a.rowmask + page_of(c0 + k)) : 0u;
+        for (int k = 0; k < 8; ++k) m[k] = c0 + k < u1 ? (uint32_t)ld_dev_i32(pool.rowmask + units.page(c0 + k)) : 0u;
+    };
+    for (int c0 = u0; c0 < u1; c0 += 8) {
+        masks(c0);
 #pragma unroll
         for (int k = 0; k < 8; ++k) local += popc32(m[k]);
     }
     int total;
     int run = block_excl_scan(local, total);
     for (int c0 = u0; c0 < u1; c0 += 8) {
-        uint32_t m[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) m[k] = c0 + k < u1 ? (uint32_t)ld_dev_i32(a.rowmask + page_of(c0 + k)) : 0u;
+        if (per > 8) masks(c0);                        // else still held
         for (int k = 0; k < 8 && c0 + k < u1; ++k) {
             const int u = c0 + k;
-            a.rowoff[page_of(u)] = cnt0 + run;
+            pool.rowoff[units.page(u)] = cnt0 + run;
             if (table) {
                 s_rank[u] = run;
                 s_mask[u] = (uint16_t)m[k];
@@ -883,7 +878,7 @@ __device__ inline void append_slots(const AppendArgs& a, int T) {
                 for (int r = 0; r < kPage; ++r)
                     if ((m[k] >> r) & 1u) {
                         const int64_t slot = (int64_t)cnt0 + run + j++;
-                        if (slot < a.cap) copy_row_thread<D>(a.raw + slot * D, src_row(u, r));
+                        if (slot < pool.cap) copy_row_thread<D>(pool.raw + slot * D, units.src_row(u, r));
                     }
             }
             run += popc32(m[k]);
@@ -892,60 +887,95 @@ __device__ inline void append_slots(const AppendArgs& a, int T) {
     if (table) {
         if (threadIdx.x == 0) s_rank[n] = total;
         __syncthreads();
-        for (int g = threadIdx.x; g < total && (int64_t)cnt0 + g < a.cap; g += kAppendThreads) {
+        for (int g = threadIdx.x; g < total && (int64_t)cnt0 + g < pool.cap; g += kAppendThreads) {
             int lo = 0, hi = n - 1;                    // the unit u with s_rank[u] <= g < s_rank[u + 1]
             while (lo < hi) {
                 const int mid = (lo + hi + 1) >> 1;
                 if (s_rank[mid] <= g) lo = mid; else hi = mid - 1;
             }
-            const uint32_t m = s_mask[lo];
+            const uint32_t mk = s_mask[lo];
             int k = g - s_rank[lo], r = 0;             // g is the k-th raw row of unit lo's page
             for (; r < kPage - 1; ++r)
-                if (((m >> r) & 1u) && k-- == 0) break;
-            copy_row_thread<D>(a.raw + ((int64_t)cnt0 + g) * D, src_row(lo, r));
+                if (((mk >> r) & 1u) && k-- == 0) break;
+            copy_row_thread<D>(pool.raw + ((int64_t)cnt0 + g) * D, units.src_row(lo, r));
         }
     }
-    if (threadIdx.x == 0) {
-        *a.before = cnt0;
-        *a.cnt = cnt0 + total;
+    return total;
+}
+
+// The token rows of n units into their open pages: 16-byte pieces (4-byte ones where the rows of x
+// are not 16-byte aligned), one per thread of the grid, up to four with all their loads in
+// flight. units: x(u), tail(u) and token(u), the token's index or -1.
+template <int D, int E, class Units>
+__device__ inline void write_rows(const Units& units, int n, int tid, int nthreads) {
+    constexpr int CH = D / E;                          // pieces of E channels per row
+    const int total = n * CH;
+    for (int i0 = tid; i0 < total; i0 += 4 * nthreads) {
+        uint32_t v[4][E / 2];
+        int tok[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int i = min(i0 + k * nthreads, total - 1), u = i / CH;
+            if (k > 0 && i0 + k * nthreads >= total) continue;
+            ld_words<E / 2>(units.x(u) + i % CH * E, v[k]);
+            tok[k] = units.token(u);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int i = i0 + k * nthreads, u = i / CH;
+            if (i < total && tok[k] >= 0) st_words<E / 2>(units.tail(u) + tok[k] % kPage * D + i % CH * E, v[k]);
+        }
     }
 }
 
-template <int D>
-__global__ void __launch_bounds__(kAppendThreads) append_kernel(AppendArgs a) {
-    const int T = a.state[0];
-    if (T < 0 || T >= a.TS) return;                   // full cache: nothing is written (no block counts in)
-    const int n = a.B * a.H, p = T % kPage, NP = a.TS / kPage, pg = T / kPage;
-    const int lane = threadIdx.x & 63, wpb = kAppendThreads / 64;
-    const int u0 = blockIdx.x * wpb + (int)(threadIdx.x >> 6), nw = (int)gridDim.x * wpb;
-    // the token rows, kAppendBatch units at a time with all their loads in flight
-    for (int ub = u0; ub < n; ub += kAppendBatch * nw) {
-        uint16_t v[kAppendBatch][D / 64];
-#pragma unroll
-        for (int i = 0; i < kAppendBatch; ++i) {
-            const int u = min(ub + i * nw, n - 1);
-            const uint16_t* x = a.x + (u / a.H) * a.sx_b + (u % a.H) * a.sx_h;
-#pragma unroll
-            for (int c = 0; c < D / 64; ++c) v[i][c] = x[64 * c + lane];
-        }
-#pragma unroll
-        for (int i = 0; i < kAppendBatch; ++i) {
-            const int u = ub + i * nw;
-            if (u >= n) break;
-            uint16_t* tail = a.raw + (a.cap + (int64_t)u * kPage + p) * D;
-#pragma unroll
-            for (int c = 0; c < D / 64; ++c) tail[64 * c + lane] = v[i][c];
-        }
+// Count this block in on *arrivals (zero between calls): true for the last of the grid's. Every
+// thread calls it; a wave's stores are complete first (stores: it waits for them).
+__device__ inline bool last_block(int32_t* arrivals, bool stores) {
+    __shared__ int s_last;
+    if (stores) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int old = __hip_atomic_fetch_add(arrivals, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = old == (int)gridDim.x - 1;
     }
+    __syncthreads();
+    return s_last != 0;
+}
+
+// Units of a contiguous cache's append at token T (-1: a full cache): every page fills at once
+template <int D>
+struct AppendUnits {
+    const AppendArgs& a;
+    int T;
+    __device__ int token(int) const { return T; }
+    __device__ int64_t page(int u) const {
+        return ((int64_t)(u / a.H) * (a.TS / kPage) + T / kPage) * a.H + u % a.H;
+    }
+    __device__ const uint16_t* x(int u) const { return a.x + (u / a.H) * a.sx_b + (u % a.H) * a.sx_h; }
+    __device__ uint16_t* tail(int u) const { return a.raw + (a.cap + (int64_t)u * kPage) * D; }
+    __device__ const uint16_t* src_row(int u, int r) const { return r == kPage - 1 ? x(u) : tail(u) + r * D; }
+};
+
+template <int D, bool ONE>
+__global__ void __launch_bounds__(kAppendThreads) append_kernel(AppendArgs a, bool vec16) {
+    const int n = a.B * a.H, lane = threadIdx.x & 63;
+    const int u0 = (int)blockIdx.x * kAppendWaves + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nw = (int)gridDim.x * kAppendWaves;
+    const int T = a.state[0];
+    const AppendUnits<D> units{a, T < a.TS ? T : -1};
+    const int tid = (int)blockIdx.x * kAppendThreads + (int)threadIdx.x, nthreads = (int)gridDim.x * kAppendThreads;
+    if (vec16)                                         // uniform
+        write_rows<D, 8>(units, n, tid, nthreads);
+    else
+        write_rows<D, 2>(units, n, tid, nthreads);
+    if (units.T < 0) return;                           // full cache: nothing is written (no block counts in)
+    const int p = T % kPage, NP = a.TS / kPage, pg = T / kPage;
     // a page end: the page of every unit
     for (int u = u0; p == kPage - 1 && u < n; u += nw) {
         const int b = u / a.H, h = u % a.H;
-        uint16_t* tail = a.raw + (a.cap + (int64_t)u * kPage) * D;
-        const uint16_t* x = a.x + b * a.sx_b + h * a.sx_h;
-        const int64_t row0 = ((int64_t)b * a.TS + (int64_t)pg * kPage) * a.H + h;
-        const int64_t page = ((int64_t)b * NP + pg) * a.H + h;
-        const uint32_t rm = encode_page<D>(tail, D, x, lane, a.sm + row0 * D, a.code + row0 * (D / 2), a.H,
-                                           a.base + page * D, nullptr);
+        const int64_t row0 = ((int64_t)b * a.TS + (int64_t)pg * kPage) * a.H + h, page = units.page(u);
+        const uint32_t rm = encode_page<D>(units.tail(u), D, units.x(u), lane, a.sm + row0 * D, a.code + row0 * (D / 2),
+                                           a.H, a.base + page * D, nullptr);
         if (lane == 0) {
             st_dev_i32(a.rowmask + page, (int32_t)rm);
             if (pg + 1 < NP) {
@@ -954,22 +984,25 @@ __global__ void __launch_bounds__(kAppendThreads) append_kernel(AppendArgs a) {
             }
         }
     }
-    __shared__ int s_last;
     // at a page end the last block reads every unit's rowmask: this wave's stores are
     // complete before the block counts itself in; otherwise the count only orders every
     // block's read of state[0] before the last block's write of it
-    if (p == kPage - 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int old = __hip_atomic_fetch_add(a.state + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = old == (int)gridDim.x - 1;
+    if (ONE) {
+        if (p == kPage - 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    } else if (!last_block(a.state + 1, p == kPage - 1)) {
+        return;
     }
-    __syncthreads();
-    if (!s_last) return;
-    if (p == kPage - 1) append_slots<D>(a, T);
-    __syncthreads();
+    if (p == kPage - 1) {
+        const RawPool pool{a.rowmask, a.rowoff, a.raw, a.cap};
+        const int cnt0 = *a.cnt, rows = place_raw_rows<D, ONE ? kAppendOne : kAppendLdsUnits>(units, n, cnt0, pool);
+        if (threadIdx.x == 0) {
+            *a.before = cnt0;
+            *a.cnt = cnt0 + rows;
+        }
+    }
     if (threadIdx.x == 0) {
-        st_dev_i32(a.state + 1, 0);
+        if (!ONE) st_dev_i32(a.state + 1, 0);
         a.state[0] = T + 1;
     }
 }
@@ -1062,80 +1095,133 @@ __device__ inline int paged_new_token(const PagedAppendArgs& a, int s) {
     return (T >= 0 && T < a.max_pages * kPage) ? T : -1;
 }
 
+// Units of a paged append: row i's head h is unit i * H + h, each at its own token
 template <int D>
-__global__ void __launch_bounds__(256) paged_append_write_kernel(PagedAppendArgs a) {
-    const int lane = threadIdx.x & 63;
-    const int u = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (u >= a.n * a.H) return;
-    const int i = u / a.H, h = u % a.H;
-    const int s = paged_slot(a, i);
-    const int T = paged_new_token(a, s);
-    if (T < 0) return;
-    const int p = T % kPage;
-    const int64_t tslot = a.cap + ((int64_t)s * a.H + h) * kPage;
-    uint16_t* tail = a.raw + tslot * D;
-    const uint16_t* x = a.x + i * a.sx_b + h * a.sx_h;
-    copy_row<D>(tail + p * D, x, lane);
-    if (p != kPage - 1) return;
-    const int pg = T / kPage;
-    const int64_t pidx = paged_pidx(a, s, pg);
-    const int64_t row0 = pidx * kPage * a.H + h;
-    const int64_t page = pidx * a.H + h;
-    encode_page<D>(tail, D, x, lane, a.sm + row0 * D, a.code + row0 * (D / 2), a.H, a.base + page * D,
-                   a.rowmask + page);
-    if (pg + 1 < a.max_pages && lane == 0) {
-        const int64_t next = paged_pidx(a, s, pg + 1) * a.H + h;
-        a.rowmask[next] = 0xFFFF;
-        a.rowoff[next] = (int32_t)tslot;
+struct PagedUnits {
+    const PagedAppendArgs& a;
+    __device__ int token(int u) const { return paged_new_token(a, paged_slot(a, u / a.H)); }
+    __device__ const uint16_t* x(int u) const { return a.x + (u / a.H) * a.sx_b + (u % a.H) * a.sx_h; }
+    __device__ int64_t tail_row(int u) const {
+        return a.cap + ((int64_t)paged_slot(a, u / a.H) * a.H + u % a.H) * kPage;
     }
+    __device__ uint16_t* tail(int u) const { return a.raw + tail_row(u) * D; }
+};
+
+// The units whose page fills in this step, of the rows c0 .. c0 + 1023: listed row k's head h is
+// unit k * H + h, and its page goes to pool page pidx[k].
+constexpr int kFillRows = kAppendThreads;
+template <int D>
+struct FilledUnits {
+    const PagedUnits<D>& all;
+    const int* row;
+    const int* pidx;
+    __device__ int64_t page(int u) const { return (int64_t)pidx[u / all.a.H] * all.a.H + u % all.a.H; }
+    __device__ int unit(int u) const { return row[u / all.a.H] * all.a.H + u % all.a.H; }
+    __device__ const uint16_t* src_row(int u, int r) const {
+        return r == kPage - 1 ? all.x(unit(u)) : all.tail(unit(u)) + r * D;
+    }
+};
+
+// The pool page that row i's token fills in this step, or -1.
+__device__ inline int fill_page(const PagedAppendArgs& a, int i) {
+    if (i >= a.n) return -1;
+    const int s = paged_slot(a, i), T = paged_new_token(a, s);
+    return T >= 0 && T % kPage == kPage - 1 ? (int)paged_pidx(a, s, T / kPage) : -1;
+}
+// Lists the rows c0 .. c0 + 1023 of the step whose token fills a page, in order, from every
+// thread's p = fill_page of row c0 + threadIdx.x; returns their number.
+__device__ inline int list_fills(int c0, int p, int* row, int* pidx) {
+    int nf;
+    const int at = block_excl_scan(p >= 0 ? 1 : 0, nf);
+    if (p >= 0) {
+        row[at] = c0 + (int)threadIdx.x;
+        pidx[at] = p;
+    }
+    __syncthreads();
+    return nf;
 }
 
-// Raw slots for the pages filled by this append, in (batch row, head, token) order.
-__global__ void __launch_bounds__(1024) paged_append_scan_kernel(PagedAppendArgs a) {
-    const int n = a.n * a.H;
-    const int per = (n + 1023) / 1024;
-    const int u0 = threadIdx.x * per, u1 = min(u0 + per, n);
-    const int cnt0 = *a.cnt;
-    int local = 0, filled = 0;
-    for (int u = u0; u < u1; ++u) {
-        const int s = paged_slot(a, u / a.H);
-        const int T = paged_new_token(a, s);
-        if (T < 0 || T % kPage != kPage - 1) continue;
-        filled = 1;
-        local += popc32((uint32_t)a.rowmask[paged_pidx(a, s, T / kPage) * a.H + u % a.H]);
+// Raw-row slots and rows of the pages that the step fills, by one block; listed: the number that
+// row / pidx list already, or -1.
+template <int D, int LDSU>
+__device__ inline void paged_place(const PagedAppendArgs& a, int* row, int* pidx, int listed) {
+    const PagedUnits<D> units{a};
+    int cnt0 = 0, cnt = 0;
+    bool any = false;
+    for (int c0 = 0; c0 < a.n; c0 += kFillRows) {
+        const int nf = listed >= 0 ? listed : list_fills(c0, fill_page(a, c0 + (int)threadIdx.x), row, pidx);
+        if (nf == 0) continue;                         // uniform
+        if (!any) cnt0 = cnt = *a.cnt;
+        any = true;
+        cnt += place_raw_rows<D, LDSU>(FilledUnits<D>{units, row, pidx}, nf * a.H, cnt,
+                                       RawPool{a.rowmask, a.rowoff, a.raw, a.cap});
+        __syncthreads();                               // the lists are read; the counter's value too
     }
-    const int any = __syncthreads_or(filled);
-    if (!any) return;                                  // uniform: no page filled, counter untouched
-    int total;
-    int run = cnt0 + block_excl_scan(local, total);
-    for (int u = u0; u < u1; ++u) {
-        const int s = paged_slot(a, u / a.H);
-        const int T = paged_new_token(a, s);
-        if (T < 0 || T % kPage != kPage - 1) continue;
-        const int64_t page = paged_pidx(a, s, T / kPage) * a.H + u % a.H;
-        a.rowoff[page] = run;
-        run += popc32((uint32_t)a.rowmask[page]);
-    }
-    if (threadIdx.x == 0) {
+    if (any && threadIdx.x == 0) {
         *a.before = cnt0;
-        *a.cnt = cnt0 + total;
+        *a.cnt = cnt;
     }
 }
 
+// The paged append in one launch, as append_kernel: token rows into the open pages; where
+// sequences fill a page in this step, those pages encoded, the next ones opened, and their raw
+// rows placed in (row, head, token) order by the last block to arrive. Every block lists the
+// filling sequences from lens, which no kernel writes, 1,024 rows at a time; in a step without
+// any none counts itself in. Three launches / this one, back to back, 8 KV heads of 128: 8
+// sequences none of which fills a page 5.8 / 3.3 us, 16 of which one does 8.5 / 8.1, 620 of which
+// 39 do 17.3 / 12.2. `arrivals`: an int32 word, zero between calls; nullptr: the raw
+// rows are left to paged_place_kernel (ONE: not used).
+template <int D, bool ONE>
+__global__ void __launch_bounds__(kAppendThreads) paged_append_kernel(PagedAppendArgs a, int32_t* arrivals, bool vec16) {
+    __shared__ int s_row[kFillRows], s_pidx[kFillRows];
+    const int n = a.n * a.H, lane = threadIdx.x & 63;
+    const int w0 = (int)blockIdx.x * kAppendWaves + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nw = (int)gridDim.x * kAppendWaves;
+    const PagedUnits<D> units{a};
+    const int tid = (int)blockIdx.x * kAppendThreads + (int)threadIdx.x, nthreads = (int)gridDim.x * kAppendThreads;
+    const int p0 = fill_page(a, (int)threadIdx.x);     // its loads beside the rows'
+    if (vec16)                                         // uniform
+        write_rows<D, 8>(units, n, tid, nthreads);
+    else
+        write_rows<D, 2>(units, n, tid, nthreads);
+    int nf = 0, any = 0;
+    for (int c0 = 0; c0 < a.n; c0 += kFillRows) {
+        if (c0 > 0) __syncthreads();                   // the lists are read
+        nf = list_fills(c0, c0 > 0 ? fill_page(a, c0 + (int)threadIdx.x) : p0, s_row, s_pidx);
+        any += nf;
+        const FilledUnits<D> filled{units, s_row, s_pidx};
+        for (int k = w0; k < nf * a.H; k += nw) {
+            const int u = __builtin_amdgcn_readfirstlane(filled.unit(k)), i = u / a.H, h = u % a.H;
+            const int s = paged_slot(a, i), pg = paged_new_token(a, s) / kPage;
+            const int64_t page = filled.page(k), row0 = (page - h) * kPage + h;
+            const uint32_t rm = encode_page<D>(units.tail(u), D, units.x(u), lane, a.sm + row0 * D,
+                                               a.code + row0 * (D / 2), a.H, a.base + page * D, nullptr);
+            if (lane == 0) {
+                st_dev_i32(a.rowmask + page, (int32_t)rm);
+                if (pg + 1 < a.max_pages) {
+                    const int64_t next = paged_pidx(a, s, pg + 1) * a.H + h;
+                    a.rowmask[next] = 0xFFFF;
+                    a.rowoff[next] = (int32_t)units.tail_row(u);
+                }
+            }
+        }
+    }
+    if (any == 0) return;                              // uniform over the grid
+    if (ONE) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    } else if (arrivals == nullptr || !last_block(arrivals, true)) {
+        return;
+    }
+    paged_place<D, ONE ? kAppendOne : kAppendLdsUnits>(a, s_row, s_pidx, a.n <= kFillRows ? nf : -1);
+    if (!ONE && threadIdx.x == 0) st_dev_i32(arrivals, 0);
+}
+
+// The end of a paged append whose caller gives no arrival word: one block, after the stores.
 template <int D>
-__global__ void __launch_bounds__(256) paged_append_rawcopy_kernel(PagedAppendArgs a) {
-    const int lane = threadIdx.x & 63;
-    const int u = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (u >= a.n * a.H) return;
-    const int h = u % a.H;
-    const int s = paged_slot(a, u / a.H);
-    const int T = paged_new_token(a, s);
-    if (T < 0 || T % kPage != kPage - 1) return;
-    const int64_t page = paged_pidx(a, s, T / kPage) * a.H + h;
-    const uint32_t m = (uint32_t)a.rowmask[page];
-    if (m == 0) return;
-    copy_raw_rows<D>(a.raw + (a.cap + ((int64_t)s * a.H + h) * kPage) * D, D, m, a.rowoff[page], a.cap, a.raw,
-                     lane);
+__global__ void __launch_bounds__(kAppendThreads) paged_place_kernel(PagedAppendArgs a) {
+    __shared__ int s_row[kFillRows], s_pidx[kFillRows];
+    paged_place<D, kAppendLdsUnits>(a, s_row, s_pidx, -1);
 }
 
 // bf16 twin: pool[(page * 16 + T % 16) * H + h] = x[i, h], page = bt[s, T / 16].
@@ -1214,6 +1300,19 @@ static int launch_status(const char* what) { return hip_status(hipGetLastError()
 
 // The instance of kernel template K for head dim D (64, 128 or 256; checked by the caller).
 #define EXKV_FOR_D(K, D) ((D) == 64 ? K<64> : (D) == 256 ? K<256> : K<128>)
+#define EXKV_FOR_D2(K, D, X) ((D) == 64 ? K<64, X> : (D) == 256 ? K<256, X> : K<128, X>)
+
+static bool rows_of_16_bytes(const void* x, int64_t sx_b, int64_t sx_h) {
+    return (uintptr_t)x % 16 == 0 && sx_b % 8 == 0 && sx_h % 8 == 0;
+}
+
+// Blocks of an append over n units: one (the ONE kernels) up to kAppendOne, then a unit per wave
+// up to kAppendBlocks.
+static unsigned append_grid(int64_t n) {
+    if (n <= kAppendOne) return 1;
+    const int64_t blocks = (n + kAppendWaves - 1) / kAppendWaves;
+    return (unsigned)(blocks < kAppendBlocks ? blocks : kAppendBlocks);
+}
 
 static int check_encode(const char* what, const void* src, int64_t s_b, int64_t s_pg, int64_t s_p, int64_t s_h,
                         bool pointers, int64_t cap, int64_t raw_rows, int32_t B, int32_t b0, int32_t pg0, int32_t nb,
@@ -1404,9 +1503,9 @@ extern "C" int exkv_cache_append(const void* x, int64_t sx_b, int64_t sx_h, void
                  "append: token rows must start at even elements (4-byte aligned)");
     AppendArgs a{(const uint16_t*)x, sx_b, sx_h, (uint8_t*)sm, (uint8_t*)code, (uint8_t*)base, rowmask, rowoff,
                  (uint16_t*)raw, cnt, before, state, cap, B, H, TS};
-    const int64_t blocks = ((int64_t)B * H + kAppendThreads / 64 - 1) / (kAppendThreads / 64);   // a unit per wave
-    const unsigned grid = (unsigned)(blocks < kAppendBlocks ? blocks : kAppendBlocks);
-    hipLaunchKernelGGL(EXKV_FOR_D(append_kernel, D), dim3(grid), dim3(kAppendThreads), 0, stream, a);
+    const unsigned grid = append_grid((int64_t)B * H);
+    auto k = grid == 1 ? EXKV_FOR_D2(append_kernel, D, true) : EXKV_FOR_D2(append_kernel, D, false);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(kAppendThreads), 0, stream, a, rows_of_16_bytes(x, sx_b, sx_h));
     return launch_status("cache_append");
 }
 
@@ -1460,29 +1559,49 @@ static int check_paged_append(const char* what, int32_t n, int32_t H, int32_t D,
     return EXKV_OK;
 }
 
+static int append_paged(const char* what, const PagedAppendArgs& a, int64_t raw_rows, int32_t D, int32_t* arrivals,
+                        hipStream_t stream) {
+    const int rc = check_paged_append(what, a.n, a.H, D, a.max_seqs, a.max_pages, a.bt_stride, a.pool_pages);
+    if (rc != EXKV_OK) return rc;
+    EXKV_REQUIRE(a.cap >= 0 && a.cap + (int64_t)a.max_seqs * a.H * kPage <= raw_rows,
+                 "%s: raw pool (%lld rows) smaller than cap + tail area", what, (long long)raw_rows);
+    EXKV_REQUIRE(a.x && a.sm && a.code && a.base && a.rowmask && a.rowoff && a.raw && a.cnt && a.before && a.lens && a.bt,
+                 "%s: null pointer", what);
+    EXKV_REQUIRE((uintptr_t)a.x % 4 == 0 && a.sx_b % 2 == 0 && a.sx_h % 2 == 0,
+                 "%s: token rows must start at even elements (4-byte aligned)", what);
+    if (a.n == 0) return EXKV_OK;
+    const unsigned grid = append_grid((int64_t)a.n * a.H);
+    auto k = grid == 1 ? EXKV_FOR_D2(paged_append_kernel, D, true) : EXKV_FOR_D2(paged_append_kernel, D, false);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(kAppendThreads), 0, stream, a, arrivals,
+                       rows_of_16_bytes(a.x, a.sx_b, a.sx_h));
+    if (grid > 1 && arrivals == nullptr)
+        hipLaunchKernelGGL(EXKV_FOR_D(paged_place_kernel, D), dim3(1), dim3(kAppendThreads), 0, stream, a);
+    return launch_status(what);
+}
+
 extern "C" int exkv_cache_append_paged(const void* x, int64_t sx_b, int64_t sx_h, void* sm, void* code, void* base,
                                        int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before,
                                        int64_t cap, int64_t raw_rows, const int32_t* slots, const int32_t* lens,
                                        const int32_t* block_table, int64_t bt_stride, int32_t n, int32_t H,
                                        int32_t max_seqs, int32_t max_pages, int32_t pool_pages, int32_t D,
                                        hipStream_t stream) {
-    const int rc = check_paged_append("append_paged", n, H, D, max_seqs, max_pages, bt_stride, pool_pages);
-    if (rc != EXKV_OK) return rc;
-    EXKV_REQUIRE(cap >= 0 && cap + (int64_t)max_seqs * H * kPage <= raw_rows,
-                 "append_paged: raw pool (%lld rows) smaller than cap + tail area", (long long)raw_rows);
-    EXKV_REQUIRE(x && sm && code && base && rowmask && rowoff && raw && cnt && before && lens && block_table,
-                 "append_paged: null pointer");
-    EXKV_REQUIRE((uintptr_t)x % 4 == 0 && sx_b % 2 == 0 && sx_h % 2 == 0,
-                 "append_paged: token rows must start at even elements (4-byte aligned)");
-    if (n == 0) return EXKV_OK;
-    PagedAppendArgs a{(const uint16_t*)x, sx_b, sx_h, (uint8_t*)sm, (uint8_t*)code, (uint8_t*)base, rowmask,
-                      rowoff, (uint16_t*)raw, cnt, before, slots, lens, block_table, bt_stride, cap, n, H,
-                      max_seqs, max_pages, pool_pages};
-    const unsigned grid = (unsigned)((n * H + 3) / 4);
-    hipLaunchKernelGGL(EXKV_FOR_D(paged_append_write_kernel, D), dim3(grid), dim3(256), 0, stream, a);
-    hipLaunchKernelGGL(paged_append_scan_kernel, dim3(1), dim3(1024), 0, stream, a);
-    hipLaunchKernelGGL(EXKV_FOR_D(paged_append_rawcopy_kernel, D), dim3(grid), dim3(256), 0, stream, a);
-    return launch_status("cache_append_paged");
+    const PagedAppendArgs a{(const uint16_t*)x, sx_b, sx_h, (uint8_t*)sm, (uint8_t*)code, (uint8_t*)base, rowmask,
+                            rowoff, (uint16_t*)raw, cnt, before, slots, lens, block_table, bt_stride, cap, n, H,
+                            max_seqs, max_pages, pool_pages};
+    return append_paged("append_paged", a, raw_rows, D, nullptr, stream);
+}
+
+extern "C" int exkv_cache_append_paged_counted(const void* x, int64_t sx_b, int64_t sx_h, void* sm, void* code,
+                                               void* base, int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt,
+                                               int32_t* before, int32_t* arrivals, int64_t cap, int64_t raw_rows,
+                                               const int32_t* slots, const int32_t* lens, const int32_t* block_table,
+                                               int64_t bt_stride, int32_t n, int32_t H, int32_t max_seqs,
+                                               int32_t max_pages, int32_t pool_pages, int32_t D, hipStream_t stream) {
+    EXKV_REQUIRE(arrivals, "append_paged: null pointer");
+    const PagedAppendArgs a{(const uint16_t*)x, sx_b, sx_h, (uint8_t*)sm, (uint8_t*)code, (uint8_t*)base, rowmask,
+                            rowoff, (uint16_t*)raw, cnt, before, slots, lens, block_table, bt_stride, cap, n, H,
+                            max_seqs, max_pages, pool_pages};
+    return append_paged("append_paged", a, raw_rows, D, arrivals, stream);
 }
 
 extern "C" int exkv_bf16_append_paged(const void* x, int64_t sx_b, int64_t sx_h, void* buf, const int32_t* slots,

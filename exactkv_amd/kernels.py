@@ -469,13 +469,17 @@ def _paged_append_args(x, table, slots):
 def append_paged(x, buf, table, slots=None):
     """One token per row of x [n, H, D] into a paged compressed cache (buf as for
     encode_pages, arrays of a [1, 16 * pool_pages, H, D] cache) whose slots, lengths and
-    block table are those of `table` (lens already counting the new token)."""
+    block table are those of `table` (lens already counting the new token). buf's 'arrivals', an
+    int32 word that is zero between calls, makes it one launch at every size."""
     sp, lp, bp, bts, n, H, ms, mp = _paged_append_args(x, table, slots)
-    raw = buf["raw"]
-    _lib.call("exkv_cache_append_paged", _lib.ptr(x, align=2, what="x"), x.stride(0), x.stride(1),
+    raw, arrivals = buf["raw"], buf.get("arrivals")
+    words = [_lib.ptr(buf["cnt"], align=4), _lib.ptr(buf["before"], align=4)]
+    if arrivals is not None:
+        words.append(_lib.ptr(arrivals, align=4))
+    _lib.call("exkv_cache_append_paged" if arrivals is None else "exkv_cache_append_paged_counted",
+              _lib.ptr(x, align=2, what="x"), x.stride(0), x.stride(1),
               _lib.ptr(buf["sm"]), _lib.ptr(buf["code"]), _lib.ptr(buf["base"]), _lib.ptr(buf["rowmask"]),
-              _lib.ptr(buf["rowoff"]), _lib.ptr(raw), _lib.ptr(buf["cnt"], align=4), _lib.ptr(buf["before"], align=4),
-              int(buf["cap"]), raw.shape[0], sp, lp, bp, bts, n, H, ms, mp, buf["TS"] // P, buf["D"], _lib.stream())
+              _lib.ptr(buf["rowoff"]), _lib.ptr(raw), *words, int(buf["cap"]), raw.shape[0], sp, lp, bp, bts, n, H, ms, mp, buf["TS"] // P, buf["D"], _lib.stream())
 
 
 def append_paged_bf16(x, pool, table, slots=None):

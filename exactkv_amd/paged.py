@@ -175,6 +175,7 @@ class PagedCompressedKV:
         self.rowoff = torch.zeros(1, NPg, H, dtype=torch.int32, device=dev)
         self.cnt = torch.zeros(1, dtype=torch.int32, device=dev)
         self._before = torch.zeros(1, dtype=torch.int32, device=dev)
+        self._arrivals = torch.zeros(1, dtype=torch.int32, device=dev)   # the append kernel's, zero between calls
         self._step_room = table.max_seqs * H * P                  # rows one step can add at most
         self.cap = max(64, int(self.TS * H * reserve), self._step_room)
         self.raw = torch.zeros(self.cap + self._step_room, D, dtype=torch.bfloat16, device=dev)
@@ -191,7 +192,8 @@ class PagedCompressedKV:
     def _buf(self):
         """The encoder's view (kernels.encode_pages_paged): arrays, counters and sizes."""
         d = {k: getattr(self, k) for k in ("sm", "code", "base", "rowmask", "rowoff", "raw")}
-        d.update(cnt=self.cnt, before=self._before, cap=self.cap, TS=self.TS, H=self.H, D=self.D)
+        d.update(cnt=self.cnt, before=self._before, cap=self.cap, TS=self.TS, H=self.H, D=self.D,
+                 arrivals=self._arrivals)
         return d
 
     def _open(self, slots):

@@ -166,6 +166,16 @@ int exkv_cache_append_paged(const void* x, int64_t sx_b, int64_t sx_h, void* sm,
                             int32_t max_seqs, int32_t max_pages, int32_t pool_pages, int32_t D,
                             hipStream_t stream);
 
+/* The same with an int32 word *arrivals of the caller's, zero when first used and reserved for
+ * this cache's appends on one stream: one launch at every size (without it more than 128
+ * sequences x heads take two). */
+int exkv_cache_append_paged_counted(const void* x, int64_t sx_b, int64_t sx_h, void* sm, void* code, void* base,
+                                    int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before,
+                                    int32_t* arrivals, int64_t cap, int64_t raw_rows, const int32_t* slots,
+                                    const int32_t* lens, const int32_t* block_table, int64_t bt_stride, int32_t n,
+                                    int32_t H, int32_t max_seqs, int32_t max_pages, int32_t pool_pages, int32_t D,
+                                    hipStream_t stream);
+
 /* bf16 twin of exkv_cache_append_paged over a pool buf [16 * pool_pages, H, D]: token
  * lens[s] - 1 of slot s goes to row (block_table[s, t / 16] * 16 + t % 16).
  * No counterpart in the reference (see exkv_cache_append_paged). */

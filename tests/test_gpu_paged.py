@@ -282,3 +282,62 @@ def test_paged_table_errors():
         table.begin_step([s, s])
     with pytest.raises(RuntimeError, match="exhausted"):
         table.add(40)                                   # 3 pages, 2 free
+
+
+@pytest.mark.parametrize("n,H,D,kind", [
+    (1, 1, 64, "plain"), (8, 8, 128, "plain"), (9, 8, 128, "pairs"), (64, 1, 256, "plain"), (65, 1, 64, "pairs"),
+    (40, 3, 128, "plain"),
+    (1024, 2, 64, "plain"),                              # one list of filled rows, and two
+    (1300, 1, 64, "plain"),
+    (1030, 8, 64, "plain"),                              # more units than one LDS table of ranks holds, all filling
+])
+def test_paged_append_one_launch(n, H, D, kind):
+    """Paged appends with and without an arrival word, at the edges of the one-block form and of the
+    lists of filled rows: pages encoded as the page encoder encodes them, raw rows in (row, head,
+    token) order, next pages opened, nothing else touched."""
+    g = torch.Generator(device=DEV).manual_seed(n + H)
+    all_fill = n == 1030
+    lens = [15 if all_fill or (i + 1) % 3 else 7 + i % 5 for i in range(n)]
+    table = exactkv.PageTable(n * 2, n + 2, 2)
+    order = torch.randperm(n, generator=torch.Generator().manual_seed(n)).tolist()
+    x0 = torch.randn(n, 15, H, D, generator=g, device=DEV).bfloat16()
+    x0[torch.rand(n, 15, H, generator=g, device=DEV) < 0.1, 3] *= 2.0 ** -30
+    x = torch.empty(n * H * D + 2, dtype=torch.bfloat16, device=DEV)[2 if kind == "pairs" else 0:][:n * H * D].view(n, H, D)
+    x.copy_(torch.randn(n, H, D, generator=g, device=DEV))
+    caches = [exactkv.PagedCompressedKV(table, H, D=D, reserve=1.0) for _ in range(2)]
+    for i in range(n):
+        table.add(lens[i])
+    slots = list(range(n)) if n < 9 else order
+    for c in caches:
+        c._open(list(range(n)))
+        rows = c.raw[c.cap:].view(n + 2, H, 16, D)
+        rows[:n, :, :15] = x0.transpose(1, 2)
+    table.begin_step(slots)
+    sd = table.step_rows()[0]
+    for c, counted in zip(caches, (True, False)):
+        buf = c._buf()
+        if not counted:
+            del buf["arrivals"]
+        c.cnt.fill_(3)
+        kernels.append_paged(x, buf, table, sd)
+        assert int(c._arrivals.item()) == 0
+    a, b = caches
+    for f in ("sm", "code", "base", "rowmask", "rowoff", "cnt", "_before"):
+        assert torch.equal(getattr(a, f), getattr(b, f)), f
+    assert same_bits(a.raw, b.raw)
+    # the page encoder on the filled pages, in the step's order
+    fill = [(r, s) for r, s in enumerate(slots) if lens[s] == 15]
+    src = torch.stack([torch.cat([x0[s], x[r:r + 1]]) for r, s in fill])        # [f, 16, H, D]
+    ref = exactkv.PagedCompressedKV(table, H, D=D, reserve=1.0)
+    ref.cnt.fill_(3)
+    pages = torch.tensor([[table.pages(s)[0]] for _, s in fill], dtype=torch.int32, device=DEV)
+    kernels.encode_pages_paged(src, (src.stride(0), 0, src.stride(1), src.stride(2)), ref._buf(), pages, len(fill), 1)
+    assert torch.equal(a.cnt, ref.cnt) and int(a._before.item()) == 3
+    for f in ("sm", "code"):
+        assert torch.equal(getattr(a, f).view(n * 2, 16, -1)[pages[:, 0]], getattr(ref, f).view(n * 2, 16, -1)[pages[:, 0]])
+    for f in ("base", "rowmask", "rowoff"):
+        assert torch.equal(getattr(a, f)[0][pages[:, 0]], getattr(ref, f)[0][pages[:, 0]]), f
+    assert same_bits(a.raw[3:int(a.cnt.item())], ref.raw[3:int(a.cnt.item())])
+    nxt = torch.tensor([table.pages(s)[1] for _, s in fill], device=DEV)
+    tail = torch.tensor([s for _, s in fill], device=DEV)[:, None] * H + torch.arange(H, device=DEV)
+    assert bool((a.rowmask[0][nxt] == 0xFFFF).all()) and torch.equal(a.rowoff[0][nxt].long(), a.cap + tail * 16)
