@@ -58,6 +58,8 @@ SIGNATURES = {
     "exkv_attn_bf16_paged": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _i32,
                              _p, _i64, _i32, _i32, _i32, _f32, _p],
     "exkv_wire_bytes": [_i32, _i32, _i64],
+    "exkv_wire_count": [_p, _i64, _i32, _p, _i64, _p, _i32, _i32, _p, _p],
+    "exkv_wire_check": [_i32, _p, _p, _i32, _p, _p, _p],
     "exkv_wire_pack": [_p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _p, _i64, _p, _p, _p, _p, _i32, _i32, _i32, _p,
                        _i64, _p],
     "exkv_wire_unpack": [_p, _p, _p, _p, _p, _p, _i64, _i64, _p, _p, _i64, _i32, _p, _i64, _p, _p, _p, _p, _p, _i32,
@@ -169,17 +171,19 @@ def synchronize(st):
 _host = threading.local()
 
 
-def host_word(index):
-    """An int32 in pinned host memory that kernels on device `index` can write: (its address, a
-    ctypes view of it). One per thread and device, for calls that wait for their stream before
-    they return, so no two of them have it at a time."""
-    words = _host.__dict__.setdefault("words", {})
-    w = words.get(index)
-    if w is None:
+def host_words(index, n=1):
+    """At least n int32 words in pinned host memory that kernels on device `index` can write:
+    (their address, a ctypes array of them). One buffer per thread and device, grown on demand,
+    for calls that wait for their stream before they return and have read the words by then, so
+    no two of them use it at a time."""
+    bufs = _host.__dict__.setdefault("bufs", {})
+    b = bufs.get(index)
+    if b is None or b[2] < n:
         import torch
-        t = torch.empty(1, dtype=torch.int32, pin_memory=True)
-        w = words[index] = (t.data_ptr(), ctypes.c_int32.from_address(t.data_ptr()), t)
-    return w[0], w[1]
+        size = max(n, 64 if b is None else 2 * b[2])
+        t = torch.empty(size, dtype=torch.int32, pin_memory=True)
+        b = bufs[index] = (t.data_ptr(), (ctypes.c_int32 * size).from_address(t.data_ptr()), size, t)
+    return b[0], b[1]
 
 
 def _stream_device(st):

@@ -440,7 +440,7 @@ def prefill_pages(x, buf, *, state=None, b=0, table=None, slot=0, shape=None):
     raw, before = buf["raw"], buf["before"]
     ws = _scan_ws(raw.device, (T // P) * H) if (T // P) * H > DIRECT_UNITS else None
     st = _lib.stream()
-    word, count = _lib.host_word(raw.device.index)
+    word, count = _lib.host_words(raw.device.index)
     args = (_lib.ptr(x, align=2, what="x"), s_t, s_h, T, _lib.ptr(buf["sm"]), _lib.ptr(buf["code"]), _lib.ptr(buf["base"]),
             _lib.ptr(buf["rowmask"]), _lib.ptr(buf["rowoff"]), _lib.ptr(raw), _lib.ptr(buf["cnt"], align=4),
             _lib.ptr(before, align=4))
@@ -452,7 +452,7 @@ def prefill_pages(x, buf, *, state=None, b=0, table=None, slot=0, shape=None):
         _lib.call("exkv_prefill_slot_paged", *args, int(buf["cap"]), raw.shape[0], _lib.ptr(table, align=4),
                   int(slot), *shape, H, D, *scan)
     _lib.synchronize(st)
-    return count.value
+    return count[0]
 
 
 def _paged_append_args(x, table, slots):

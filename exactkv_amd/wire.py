@@ -23,6 +23,7 @@ does not depend on where its rows sat in the source pool.
 """
 import struct
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -45,10 +46,28 @@ def nbytes(H, T, raw_rows):
     return n
 
 
-def header(blob):
-    """The header fields of a blob (a uint8 tensor on any device) as a dict."""
+class _Read:
+    """A blob on the GPU with its header and the raw rows of its rowmask section, as
+    exkv_wire_check has read them."""
+    __slots__ = ("blob", "head", "rows")
+
+    def __init__(self, blob, head, rows):
+        self.blob, self.head, self.rows = blob, head, rows
+
+    def numel(self):
+        return self.blob.numel()
+
+
+def _blob_shape(blob):
     if blob.dtype != torch.uint8 or blob.dim() != 1 or blob.numel() < HEADER:
         raise ValueError("a wire blob is a 1-D uint8 tensor of at least 256 bytes")
+
+
+def header(blob):
+    """The header fields of a blob (a uint8 tensor on any device) as a dict."""
+    if isinstance(blob, _Read):
+        return dict(zip(_KEYS, struct.unpack_from("<8I7Q", blob.head)))
+    _blob_shape(blob)
     vals = struct.unpack_from("<8I7Q", bytes(blob[:HEADER].cpu().numpy()))
     return dict(zip(_KEYS, vals))
 
@@ -61,32 +80,70 @@ def _sequence(cache, seq):
         if not 0 <= seq < t.max_seqs or t._pages[seq] is None:
             raise ValueError(f"slot {seq} is not in use")
         T = t.length(seq)
-        return T, list(t._pages[seq]), cache.cap + seq * H * P, t.num_pages, T // P < t.max_pages
+        return T, t._pages[seq], cache.cap + seq * H * P, t.num_pages, T // P < t.max_pages
     if isinstance(cache, CompressedKV):
         if not 0 <= seq < cache.B:
             raise ValueError(f"sequence {seq} outside the cache's {cache.B}")
         NP = cache.TS // P
         T = cache.T
-        return T, list(range(seq * NP, seq * NP + NP)), cache.cap + seq * H * P, cache.B * NP, T < cache.TS
+        return T, range(seq * NP, seq * NP + NP), cache.cap + seq * H * P, cache.B * NP, T < cache.TS
     raise TypeError(type(cache))
+
+
+class _Part:
+    """A part of a device buffer, by its address."""
+    __slots__ = ("buf", "off")
+
+    def __init__(self, buf, off):
+        self.buf, self.off = buf, off
+
+    def data_ptr(self):
+        return self.buf.data_ptr() + self.off
+
+
+def _upload(host, dev):
+    """Numpy arrays (a dict) on the GPU, in one buffer and one copy that waits for nothing."""
+    offs, size = {}, 0
+    for k, v in host.items():
+        offs[k] = size
+        size += -(-v.nbytes // 16) * 16
+    pin = torch.empty(size, dtype=torch.uint8, pin_memory=True)
+    view = pin.numpy()
+    for k, v in host.items():
+        view[offs[k]:offs[k] + v.nbytes] = v.reshape(-1).view(np.uint8)
+    buf = torch.empty(size, dtype=torch.uint8, device=dev)
+    buf.copy_(pin, non_blocking=True)
+    return {k: _Part(buf, o) for k, o in offs.items()}
+
+
+def _host_pages(cache, infos):
+    """The sequences' page lists, token counts, first tail rows and open flags as arrays."""
+    width = max(max(len(i[1]) for i in infos), 1)
+    pages = np.zeros((len(infos), width), np.int32)
+    for row, i in zip(pages, infos):
+        row[:len(i[1])] = np.arange(i[1].start, i[1].stop) if isinstance(i[1], range) else i[1]
+    return dict(pages=pages, tokens=np.array([i[0] for i in infos], np.int32),
+                tails=np.array([i[2] for i in infos], np.int64), open=np.array([int(i[4]) for i in infos], np.int32))
+
+
+def _host_blobs(blobs):
+    return dict(blobs=np.array([_lib.ptr(b, align=256, what="blob") for b in blobs], np.int64),
+                sizes=np.array([b.numel() for b in blobs], np.int64))
+
+
+def _scratch(cache, infos, dev):
+    """(ws, its row stride, the most tokens) of a pack or unpack call."""
+    max_t = max(i[0] for i in infos)
+    ws_stride = (max_t // P) * cache.H + 3
+    return torch.empty(len(infos), ws_stride, dtype=torch.int32, device=dev), ws_stride, max_t
 
 
 def _batch_args(cache, seqs, infos, blobs, dev):
     """Device arrays of one pack / unpack call."""
-    width = max(max(len(i[1]) for i in infos), 1)
-    pages = torch.zeros(len(seqs), width, dtype=torch.int32)
-    for r, i in enumerate(infos):
-        pages[r, :len(i[1])] = torch.tensor(i[1], dtype=torch.int32)
-    max_t = max(i[0] for i in infos)
-    ws_stride = (max_t // P) * cache.H + 3
-    host = dict(pages=pages, tokens=torch.tensor([i[0] for i in infos], dtype=torch.int32),
-                tails=torch.tensor([i[2] for i in infos], dtype=torch.int64),
-                blobs=torch.tensor([_lib.ptr(b, align=256, what="blob") for b in blobs], dtype=torch.int64),
-                sizes=torch.tensor([b.numel() for b in blobs], dtype=torch.int64),
-                open=torch.tensor([int(i[4]) for i in infos], dtype=torch.int32))
-    d = {k: v.to(dev) for k, v in host.items()}
-    d["ws"] = torch.empty(len(seqs), ws_stride, dtype=torch.int32, device=dev)
-    return d, width, max_t, ws_stride
+    host = _host_pages(cache, infos)
+    d = _upload(dict(host, **_host_blobs(blobs)), dev)
+    d["ws"], ws_stride, max_t = _scratch(cache, infos, dev)
+    return d, host["pages"].shape[1], max_t, ws_stride
 
 
 def pack(cache, seq):
@@ -104,23 +161,20 @@ def pack_many(cache, seqs):
         return []
     H, dev = cache.H, cache.sm.device
     infos = [_sequence(cache, s) for s in seqs]
-    full = [p for i in infos for p in i[1][:i[0] // P]]
-    counts = [0] * len(seqs)
-    if full:
-        rm = cache.rowmask.view(-1, H).index_select(0, torch.tensor(full, dtype=torch.int64, device=dev))
-        per_page = _popc16(rm & 0xFFFF).sum(1).cpu().tolist()
-        k = 0
-        for r, i in enumerate(infos):
-            n = i[0] // P
-            counts[r] = int(sum(per_page[k:k + n]))
-            k += n
-    blobs = [torch.empty(nbytes(H, i[0], n), dtype=torch.uint8, device=dev) for i, n in zip(infos, counts)]
-    d, width, max_t, ws_stride = _batch_args(cache, seqs, infos, blobs, dev)
+    host, n = _host_pages(cache, infos), len(seqs)
+    d, width = _upload(host, dev), host["pages"].shape[1]
+    d["ws"], ws_stride, max_t = _scratch(cache, infos, dev)
+    st = _lib.stream()
+    addr, counts = _lib.host_words(dev.index, n)
+    _lib.call("exkv_wire_count", _lib.ptr(cache.rowmask), infos[0][3], n, d["pages"].data_ptr(), width,
+              d["tokens"].data_ptr(), max_t, H, addr, st)
+    _lib.synchronize(st)
+    blobs = [torch.empty(nbytes(H, i[0], c), dtype=torch.uint8, device=dev) for i, c in zip(infos, counts)]
+    d.update(_upload(_host_blobs(blobs), dev))
     _lib.call("exkv_wire_pack", _lib.ptr(cache.sm), _lib.ptr(cache.code), _lib.ptr(cache.base),
               _lib.ptr(cache.rowmask), _lib.ptr(cache.rowoff), _lib.ptr(cache.raw), cache.raw.shape[0], infos[0][3],
               len(seqs), d["pages"].data_ptr(), width, d["tokens"].data_ptr(), d["tails"].data_ptr(),
-              d["blobs"].data_ptr(), d["sizes"].data_ptr(), max_t, H, cache.D, d["ws"].data_ptr(), ws_stride,
-              _lib.stream())
+              d["blobs"].data_ptr(), d["sizes"].data_ptr(), max_t, H, cache.D, d["ws"].data_ptr(), ws_stride, st)
     return blobs
 
 
@@ -137,8 +191,11 @@ def _check_blob(blob, cache):
         raise ValueError(f"blob of {blob.numel()} bytes is shorter than its header's {h['total']}")
     npf = h["full_pages"] * cache.H
     if npf:
-        rm = blob[h["off_rowmask"]: h["off_rowmask"] + 4 * npf].view(torch.int32)
-        rows = int(_popc16(rm & 0xFFFF).sum().item())
+        if isinstance(blob, _Read):
+            rows = blob.rows
+        else:
+            rm = blob[h["off_rowmask"]: h["off_rowmask"] + 4 * npf].view(torch.int32)
+            rows = int(_popc16(rm & 0xFFFF).sum().item())
         if rows != N:
             raise ValueError(f"blob's rowmask marks {rows} raw rows, its header declares {N}")
     return h
@@ -158,9 +215,19 @@ def unpack_many(blobs, cache, seqs):
         raise ValueError("one distinct sequence per blob")
     if not seqs:
         return
-    heads = [_check_blob(b, cache) for b in blobs]
-    dev = cache.sm.device
+    for b in blobs:
+        _blob_shape(b)
+    dev, n = cache.sm.device, len(seqs)
     blobs = [b if b.device == dev else b.to(dev) for b in blobs]
+    up = _upload(_host_blobs(blobs), dev)
+    st = _lib.stream()
+    addr, facts = _lib.host_words(dev.index, 65 * n + 1)
+    _lib.call("exkv_wire_check", n, up["blobs"].data_ptr(), up["sizes"].data_ptr(), cache.H, _lib.ptr(cache.cnt, align=4),
+              addr, st)
+    _lib.synchronize(st)
+    head, cnt = bytes(facts)[:HEADER * n], facts[65 * n]
+    rows = facts[64 * n:65 * n]
+    heads = [_check_blob(_Read(b, head[HEADER * i:HEADER * (i + 1)], rows[i]), cache) for i, b in enumerate(blobs)]
     if cache._pending is not None:
         raise RuntimeError("call check_overflow() before unpacking")
     Ts = [h["tokens"] for h in heads]
@@ -174,15 +241,15 @@ def unpack_many(blobs, cache, seqs):
             if cache.table.length(s) != T:
                 raise ValueError(f"blob of {T} tokens into a slot of {cache.table.length(s)}")
     N = sum(h["raw_rows"] for h in heads)
-    cnt = int(cache.cnt.item())
     if cnt + N > cache.cap:
         cache._grow(cnt + N)
     infos = [_sequence(cache, s) for s in seqs]                 # tail rows after any growth
-    d, width, max_t, ws_stride = _batch_args(cache, seqs, infos, blobs, dev)
+    host = _host_pages(cache, infos)
+    d, width = _upload(host, dev), host["pages"].shape[1]
+    d["ws"], ws_stride, max_t = _scratch(cache, infos, dev)
     _lib.call("exkv_wire_unpack", _lib.ptr(cache.sm), _lib.ptr(cache.code), _lib.ptr(cache.base),
               _lib.ptr(cache.rowmask), _lib.ptr(cache.rowoff), _lib.ptr(cache.raw), cache.raw.shape[0], cache.cap,
               _lib.ptr(cache.cnt, align=4), _lib.ptr(cache._before, align=4), infos[0][3], len(seqs),
               d["pages"].data_ptr(), width, d["tokens"].data_ptr(), d["open"].data_ptr(), d["tails"].data_ptr(),
-              d["blobs"].data_ptr(), d["sizes"].data_ptr(), max_t, cache.H, cache.D, d["ws"].data_ptr(), ws_stride,
-              _lib.stream())
+              up["blobs"].data_ptr(), up["sizes"].data_ptr(), max_t, cache.H, cache.D, d["ws"].data_ptr(), ws_stride, st)
     cache._keep_headroom(cnt + N)

@@ -230,6 +230,20 @@ int exkv_time_next_split(hipEvent_t start, hipEvent_t stop);
 /* Blob size for H heads, T tokens and N raw rows (-1 for bad arguments). */
 int64_t exkv_wire_bytes(int32_t H, int32_t T, int64_t raw_rows);
 
+/* Raw rows of the full pages of nseq sequences (arguments as for exkv_wire_pack), which size
+ * their blobs: sequence s's to host_counts[s] (host memory that the GPU can write; valid once
+ * the stream has been waited for). One launch. */
+int exkv_wire_count(const int32_t* rowmask, int64_t pool_pages, int32_t nseq, const int32_t* pages,
+                    int64_t page_stride, const int32_t* tokens, int32_t max_tokens, int32_t H,
+                    uint32_t* host_counts, hipStream_t stream);
+
+/* What a check of nseq blobs for a cache of H heads reads, to host memory (as above): blob s's
+ * 256-byte header to host_facts[64 s ..], the raw rows its rowmask section marks to
+ * host_facts[64 nseq + s] (0xFFFFFFFF where the section is not inside the blob), and the raw-row
+ * counter *cnt to host_facts[65 nseq]. Only the blobs' blob_bytes[s] bytes are read. One launch. */
+int exkv_wire_check(int32_t nseq, const uint64_t* blobs, const int64_t* blob_bytes, int32_t H,
+                    const int32_t* cnt, uint32_t* host_facts, hipStream_t stream);
+
 /* Pack nseq sequences of one compressed cache (arrays as above, pool_pages pages of
  * 16 tokens) into one blob each. Sequence s has tokens[s] (<= max_tokens) tokens; its page
  * p is pool page pages[s * page_stride + p] (entries clamped to the pool); its open page's

@@ -7,6 +7,8 @@ build's own). Gates:
     bit-identical attention, and decoding can go on from there;
   * a raw pool too small for the blob grows first.
 """
+import struct
+
 import numpy as np
 import pytest
 import torch
@@ -158,3 +160,39 @@ def test_unpack_skips_a_blob_whose_rowmask_disagrees_with_its_header(monkeypatch
     assert int(dst.cnt.item()) == cnt0 + wire.header(good)["raw_rows"] + h["raw_rows"]
     assert same_bits(kernels.decode_to_bf16(dst.buffers(), 64)[0], x[0].to(DEV))
     assert int(dst.sm[1].sum().item()) == 0 and int(dst.code[1].sum().item()) == 0
+
+
+def _sealed(blob, **fields):
+    """A copy of a blob with header fields replaced."""
+    out = blob.clone()
+    head = wire.header(blob)
+    head.update(fields)
+    raw = struct.pack("<8I7Q", *[head[k] for k in wire._KEYS])
+    out[:len(raw)] = torch.frombuffer(bytearray(raw), dtype=torch.uint8).to(blob.device)
+    return out
+
+
+@pytest.mark.parametrize("H,T", [(1, 5), (2, 16), (3, 37), (8, 4101), (5, 33000)])
+def test_batch_facts_equal_the_blobs(H, T):
+    """The one-launch count and check: a pack's sizes and an unpack's header fields and rowmask
+    counts are the blobs' own; sections that a header puts outside its blob are not read."""
+    x = synthetic.make_kv(2, T, H, kind="k", seed=T, raw_row_rate=0.05)
+    c = _cache(x)
+    blobs = wire.pack_many(c, [1, 0])
+    for b, s in zip(blobs, (1, 0)):
+        h = wire.header(b)
+        marks = c.rowmask[s, :T // 16].reshape(-1).tolist()
+        assert h["raw_rows"] == sum(bin(m & 0xFFFF).count("1") for m in marks) and h["total"] == b.numel()
+        wire._check_blob(b, c)                          # and by the tensor's own reads
+    dst = exactkv.CompressedKV(2, c.TS, H, 128, reserve=0.2)
+    wire.unpack_many([blobs[1], blobs[0].cpu()], dst, [0, 1])
+    assert same_bits(kernels.decode_to_bf16(dst.buffers(), T), x.to(DEV))
+    if T >= 16:
+        for fields in (dict(off_rowmask=blobs[0].numel() - 2), dict(off_rowmask=1 << 62), dict(off_rowmask=3),
+                       dict(raw_rows=wire.header(blobs[0])["raw_rows"] + 1)):
+            with pytest.raises(ValueError):
+                wire.unpack(_sealed(blobs[0], **fields), dst, 0)
+    with pytest.raises(ValueError):
+        wire.unpack(_sealed(blobs[0], full_pages=0xFFFFFFFF), dst, 0)
+    with pytest.raises(ValueError):
+        wire.unpack(blobs[0][:100], dst, 0)
