@@ -57,6 +57,8 @@ SIGNATURES = {
                                          _i32, _i32, _f32, _p],
     "exkv_attn_bf16_paged": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _i32,
                              _p, _i64, _i32, _i32, _i32, _f32, _p],
+    "exkv_table_write": [_p, _i64, _p, _i64, _p, _p, _i32, _i32, _p],
+    "exkv_gather_words": [_p, _i32, _p, _p],
     "exkv_wire_bytes": [_i32, _i32, _i64],
     "exkv_wire_count": [_p, _i64, _i32, _p, _i64, _p, _i32, _i32, _p, _p],
     "exkv_wire_check": [_i32, _p, _p, _i32, _p, _p, _p],

@@ -28,7 +28,7 @@ How CompressedKV is organised here:
 import torch
 
 from . import _lib
-from .kernels import encode_pages, prefill_pages, prefill_ready, HEAD_DIMS, P
+from .kernels import encode_pages, prefill_pages, prefill_ready, read_words, HEAD_DIMS, P
 
 _FIELDS = ("sm", "code", "base", "rowmask", "rowoff", "raw")
 
@@ -252,11 +252,13 @@ class BF16KV:
 
 
 def check_overflow(caches):
-    """After a step whose token filled a page: one device-to-host transfer of the counters of
+    """After a step whose token filled a page: one device-to-host read of the counters of
     every compressed cache (contiguous or paged) with a page waiting, then each repairs an
     overflow and tops up its headroom. Returns the number of pools that grew."""
     waiting = [c for c in caches if hasattr(c, "finish_page") and c._pending is not None]
     if not waiting:
         return 0
-    counts = torch.cat([c.cnt for c in waiting]).tolist()
+    words = [c.cnt for c in waiting]
+    one_gpu = words[0].is_cuda and all(w.device == words[0].device for w in words)
+    counts = read_words(words) if one_gpu else torch.cat(words).tolist()
     return sum(int(c.finish_page(n > c.cap, n)) for c, n in zip(waiting, counts))

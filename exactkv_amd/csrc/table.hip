@@ -1,0 +1,77 @@
+// Small host values to the device and device words to the host, through kernel arguments and
+// mapped host memory: the page table's updates and the overflow check's counters. A copy from
+// pageable memory waits for the whole stream before it returns, so each of them drained the
+// GPU (and cost a copy and a scatter launch); a launch with the values in its arguments does
+// neither. Twelve paged sequences joining, 24 steps and leaving: 4,060 -> 3,000 us.
+//
+// No counterpart in the reference (its token count and counters are read and written by torch
+// calls, cache.py:57-60,149-158; paged KV is in its future work, README.md:121-123).
+#include "common.hpp"
+#include "../../include/exactkv.h"
+
+namespace exkv {
+
+constexpr int kPairs = 448;          // (index, value) pairs per launch (whole wavefronts; 3,584 of the 4,096 argument bytes)
+constexpr int kWords = 448;          // word addresses per launch
+
+struct Pairs {
+    int32_t at[kPairs];
+    int32_t val[kPairs];
+};
+
+// Pairs [0, nl) into lens, [nl, n) into table.
+__global__ void __launch_bounds__(kPairs) table_write_kernel(int32_t* lens, int32_t* table, int nl, int n, Pairs p) {
+    const int i = threadIdx.x;
+    if (i < n) (i < nl ? lens : table)[p.at[i]] = p.val[i];
+}
+
+struct Words {
+    const int32_t* p[kWords];
+};
+__global__ void __launch_bounds__(kWords) gather_words_kernel(Words w, int n, int32_t* out) {
+    const int i = threadIdx.x;
+    if (i < n) __hip_atomic_store(out + i, *w.p[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+}  // namespace exkv
+
+using namespace exkv;
+
+extern "C" int exkv_table_write(int32_t* lens, int64_t lens_size, int32_t* table, int64_t table_size, const int32_t* at,
+                                const int32_t* val, int32_t n_lens, int32_t n, hipStream_t stream) {
+    EXKV_REQUIRE(n >= 0 && n_lens >= 0 && n_lens <= n, "table_write: bad counts %d of %d", n_lens, n);
+    EXKV_REQUIRE(n == 0 || (lens && table && at && val), "table_write: null pointer");
+    for (int32_t i = 0; i < n; ++i)
+        EXKV_REQUIRE(at[i] >= 0 && at[i] < (i < n_lens ? lens_size : table_size), "table_write: index %d of pair %d", at[i],
+                     i);
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(stream, &capturing);
+    if (e != hipSuccess) return hip_status(e, "table_write");
+    // a replay would write this call's values again, over later ones
+    EXKV_REQUIRE(capturing == hipStreamCaptureStatusNone, "table_write: the stream is being captured");
+    Pairs p;
+    for (int32_t i0 = 0; i0 < n; i0 += kPairs) {
+        const int32_t m = n - i0 < kPairs ? n - i0 : kPairs;
+        for (int32_t i = 0; i < m; ++i) {
+            p.at[i] = at[i0 + i];
+            p.val[i] = val[i0 + i];
+        }
+        const int32_t nl = n_lens - i0 < 0 ? 0 : n_lens - i0;
+        hipLaunchKernelGGL(table_write_kernel, dim3(1), dim3((m + 63) / 64 * 64), 0, stream, lens, table, nl, m, p);
+    }
+    return hip_status(hipGetLastError(), "table_write");
+}
+
+extern "C" int exkv_gather_words(const int32_t* const* words, int32_t n, int32_t* host_out, hipStream_t stream) {
+    EXKV_REQUIRE(n >= 0 && (n == 0 || (words && host_out)), "gather_words: null pointer");
+    Words w;
+    for (int32_t i0 = 0; i0 < n; i0 += kWords) {
+        const int32_t m = n - i0 < kWords ? n - i0 : kWords;
+        for (int32_t i = 0; i < m; ++i) {
+            EXKV_REQUIRE(words[i0 + i], "gather_words: null word %d", i0 + i);
+            w.p[i] = words[i0 + i];
+        }
+        hipLaunchKernelGGL(gather_words_kernel, dim3(1), dim3((m + 63) / 64 * 64), 0, stream, w, m, host_out + i0);
+    }
+    return hip_status(hipGetLastError(), "gather_words");
+}

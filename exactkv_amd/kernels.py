@@ -15,6 +15,7 @@ split plan), out (output tensor).
 """
 import ctypes
 import math
+from array import array
 
 import torch
 
@@ -453,6 +454,32 @@ def prefill_pages(x, buf, *, state=None, b=0, table=None, slot=0, shape=None):
                   int(slot), *shape, H, D, *scan)
     _lib.synchronize(st)
     return count[0]
+
+
+def table_write(lens, block_table, lens_at, lens_val, table_at, table_val):
+    """Host ints into a page table on the GPU: lens[lens_at] = lens_val and, row-major,
+    block_table[table_at] = table_val (any sequences), in stream order, waiting for nothing."""
+    at, val = array("i", lens_at), array("i", lens_val)
+    n_lens = len(at)
+    at.extend(table_at)
+    val.extend(table_val)
+    if len(at) != len(val):
+        raise ValueError("as many values as indices")
+    _lib.call("exkv_table_write", _lib.ptr(lens, align=4), lens.numel(), _lib.ptr(block_table, align=4),
+              block_table.numel(), at.buffer_info()[0], val.buffer_info()[0], n_lens, len(at),
+              _lib.stream(lens.device.index))
+
+
+def read_words(words):
+    """The values of one-element int32 tensors of one GPU, after the work queued on its current
+    stream: one launch and a wait."""
+    dev = words[0].device.index
+    st = _lib.stream(dev)
+    addr, out = _lib.host_words(dev, len(words))
+    at = array("Q", [_lib.ptr(w, align=4) for w in words])
+    _lib.call("exkv_gather_words", at.buffer_info()[0], len(at), addr, st)
+    _lib.synchronize(st)
+    return out[:len(at)]
 
 
 def _paged_append_args(x, table, slots):

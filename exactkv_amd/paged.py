@@ -26,7 +26,7 @@ import torch
 
 from . import _lib
 from .kernels import (HEAD_DIMS, P, append_paged, append_paged_bf16, encode_pages_paged, prefill_pages,
-                      prefill_ready)
+                      prefill_ready, table_write)
 
 
 class PageTable:
@@ -82,11 +82,18 @@ class PageTable:
         pages = self._claim(self._npages(T))
         self._pages[slot] = pages
         self._len[slot] = T
-        row = torch.tensor(pages, dtype=torch.int32)
-        self.block_table[slot, : len(pages)] = row.to(self.dev)
-        self.lens[slot] = T
+        first = slot * self.max_pages
+        self._write([slot], [T], range(first, first + len(pages)), pages)
         self._rows = None
         return slot
+
+    def _write(self, slots, lens, at, pages):
+        """lens of the slots and row-major block-table entries, on the device."""
+        if self.dev.type == "cuda":
+            table_write(self.lens, self.block_table, slots, lens, at, pages)
+            return
+        self.lens[torch.tensor(list(slots), dtype=torch.int64)] = torch.tensor(list(lens), dtype=torch.int32)
+        self.block_table.view(-1)[torch.tensor(list(at), dtype=torch.int64)] = torch.tensor(list(pages), dtype=torch.int32)
 
     def release(self, slot):
         """Give a slot's pages back to the pool."""
@@ -114,19 +121,16 @@ class PageTable:
             need += L % P == 0 and L // P < self.max_pages
         if need > len(self._free):
             raise RuntimeError(f"page pool exhausted: need {need} pages, {len(self._free)} free")
-        new_cols, new_pages = [], []
+        new_at, new_pages = [], []
         for s in slots:
             L = self._len[s] + 1
             if L % P == 0 and L // P < self.max_pages:          # the token fills a page: open the next
                 pg = self._claim(1)[0]
                 self._pages[s].append(pg)
-                new_cols.append((s, L // P))
+                new_at.append(s * self.max_pages + L // P)
                 new_pages.append(pg)
             self._len[s] = L
-        if new_cols:
-            idx = torch.tensor([s * self.max_pages + c for s, c in new_cols], dtype=torch.int64)
-            self.block_table.view(-1)[idx.to(self.dev)] = torch.tensor(new_pages, dtype=torch.int32).to(self.dev)
-        self.lens.copy_(torch.tensor(self._len, dtype=torch.int32))
+        self._write(slots, [self._len[s] for s in slots], new_at, new_pages)
         self.step += 1
         self._step_slots = slots
         if slots == list(range(len(slots))):

@@ -147,6 +147,18 @@ int exkv_cache_append(const void* x, int64_t sx_b, int64_t sx_h, void* sm, void*
 int exkv_bf16_append(const void* x, int64_t sx_b, int64_t sx_h, void* buf, int32_t* state, int32_t B,
                      int32_t H, int32_t TS, int32_t D, hipStream_t stream);
 
+/* Values of a paged cache's table through kernel arguments: of the n (index, value) pairs
+ * at[i], val[i] in host memory, the first n_lens go to lens (lens_size entries), the others to
+ * the table (table_size entries, row-major). Copied by the call; nothing is waited for.
+ * No counterpart in the reference (contiguous caches only). */
+int exkv_table_write(int32_t* lens, int64_t lens_size, int32_t* table, int64_t table_size, const int32_t* at,
+                     const int32_t* val, int32_t n_lens, int32_t n, hipStream_t stream);
+
+/* The device words at n addresses (a host array) to host_out[0 .. n) (host memory that the GPU
+ * can write; valid once the stream has been waited for): the overflow check's counters.
+ * Part of what replaces: cache.py:149-158. */
+int exkv_gather_words(const int32_t* const* words, int32_t n, int32_t* host_out, hipStream_t stream);
+
 /* Append one token for each of n sequences of a paged cache: a pool of pool_pages pages
  * (arrays as a [1, 16 * pool_pages, H, D] cache) shared by max_seqs sequence slots.
  * Batch row i is slot slots[i] (slots == NULL: slot i; the slots must differ); slot s owns

@@ -341,3 +341,28 @@ def test_paged_append_one_launch(n, H, D, kind):
     nxt = torch.tensor([table.pages(s)[1] for _, s in fill], device=DEV)
     tail = torch.tensor([s for _, s in fill], device=DEV)[:, None] * H + torch.arange(H, device=DEV)
     assert bool((a.rowmask[0][nxt] == 0xFFFF).all()) and torch.equal(a.rowoff[0][nxt].long(), a.cap + tail * 16)
+
+
+@pytest.mark.parametrize("n_lens,n_table", [(0, 0), (1, 0), (0, 1), (3, 445), (3, 446), (448, 448), (449, 1), (700, 2000)])
+def test_table_write(n_lens, n_table):
+    """Page-table values through kernel arguments, at the edges of a launch's pairs: each at its
+    place, nothing else written; an index outside either tensor is refused before any launch."""
+    g = torch.Generator().manual_seed(n_lens + n_table)
+    lens, table = torch.full((1000,), -1, dtype=torch.int32), torch.full((50, 60), -1, dtype=torch.int32)
+    la, ta = torch.randperm(1000, generator=g)[:n_lens], torch.randperm(3000, generator=g)[:n_table]
+    lv, tv = torch.arange(n_lens, dtype=torch.int32), 5000 + torch.arange(n_table, dtype=torch.int32)
+    dl, dt = lens.to(DEV), table.to(DEV)
+    kernels.table_write(dl, dt, la.tolist(), lv.tolist(), ta.tolist(), tv.tolist())
+    lens[la] = lv
+    table.view(-1)[ta] = tv
+    assert torch.equal(dl.cpu(), lens) and torch.equal(dt.cpu(), table)
+    for bad in (([1000], [1], [], []), ([-1], [1], [], []), ([], [], [3000], [1])):
+        with pytest.raises(RuntimeError, match="index"):
+            kernels.table_write(dl, dt, *bad)
+    assert torch.equal(dl.cpu(), lens) and torch.equal(dt.cpu(), table)
+
+
+def test_read_words():
+    words = [torch.full((1,), i * 7 - 3, dtype=torch.int32, device=DEV) for i in range(1003)]
+    for n in (1, 64, 448, 449, 1003):
+        assert kernels.read_words(words[:n]) == [i * 7 - 3 for i in range(n)]
