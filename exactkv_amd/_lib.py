@@ -135,12 +135,17 @@ def describe_errors(bits):
     return "; ".join(names + ([f"unknown bits {rest:#x}"] if rest else [])) or "none"
 
 
+_bound = {}      # entry point name -> its function, once the library is loaded
+
+
 def call(name, *args):
     """Call entry point `name`; raise RuntimeError with the library's message on failure."""
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    f = _bound.get(name)
+    if f is None:
+        f = _bound[name] = getattr(load(), name)
+    rc = f(*args)
     if rc != 0:
-        msg = lib.exkv_last_error().decode(errors="replace")
+        msg = load().exkv_last_error().decode(errors="replace")
         raise RuntimeError(f"{name} failed ({rc}): {msg}")
     if _CHECK and name not in _NO_STREAM:
         bits = stream_error_bits(args[-1], clear=True)
@@ -211,19 +216,21 @@ def stream_error_bits(st, clear=True):
     return int(buf.cpu().item()) & 0xFFFFFFFF
 
 
-_raw_stream = None
+_raw_stream = _current_device = None
 
 
 def stream(index=None):
     """The current HIP stream of device `index` (default: the current device) as an integer,
     through torch's raw-stream query when it has one (a few µs cheaper per call than
     building a torch Stream object)."""
-    global _raw_stream
-    import torch
+    global _raw_stream, _current_device
     if _raw_stream is None:
+        import torch
         _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", False)
+        _current_device = torch.cuda.current_device
     if _raw_stream:
-        return _raw_stream(torch.cuda.current_device() if index is None else index)
+        return _raw_stream(_current_device() if index is None else index)
+    import torch
     return torch.cuda.current_stream(index).cuda_stream
 
 

@@ -19,7 +19,7 @@ def decode_attention(q, k_cache, v_cache, **kw):
     if isinstance(k_cache, (PagedCompressedKV, PagedBF16KV)):
         _, bt, lens = k_cache.table.step_rows()
         if isinstance(k_cache, PagedCompressedKV):
-            return attention_compressed(q, k_cache.buffers(), v_cache.buffers(), 0, lens=lens, block_table=bt, **kw)
+            return attention_compressed(q, k_cache, v_cache, 0, lens=lens, block_table=bt, **kw)
         return attention_reference(q, k_cache.buf, v_cache.buf, 0, lens=lens, block_table=bt, **kw)
     if isinstance(k_cache, CompressedKV):
         return attention_compressed(q, k_cache, v_cache, k_cache.T, **kw)

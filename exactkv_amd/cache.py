@@ -28,7 +28,7 @@ How CompressedKV is organised here:
 import torch
 
 from . import _lib
-from .kernels import encode_pages, prefill_pages, prefill_ready, read_words, HEAD_DIMS, P
+from .kernels import array_ptrs, encode_pages, prefill_pages, prefill_ready, read_words, HEAD_DIMS, P
 
 _FIELDS = ("sm", "code", "base", "rowmask", "rowoff", "raw")
 
@@ -62,7 +62,7 @@ class CompressedKV:
         self.T = 0
         self.grows = 0
         self._pending = None                           # page filled by the last append, until checked
-        self._abi = None
+        self._abi = self._ptr_memo = None
         self._open_page()                              # appends may start from an empty cache
 
     # ---------------------------------------------------------------- device-side upkeep
@@ -82,6 +82,12 @@ class CompressedKV:
         if self._abi is None or self._abi[5] is not self.raw:
             self._abi = (self.sm, self.code, self.base, self.rowmask, self.rowoff, self.raw)
         return self._abi
+
+    def _ptrs(self):
+        """Addresses of the six arrays, cnt, _before and state."""
+        self._ptr_memo = array_ptrs(self._ptr_memo, (self.sm, self.code, self.base, self.rowmask, self.rowoff, self.raw,
+                                                     self.cnt, self._before, self.state), 3)
+        return self._ptr_memo[1]
 
     def _buf(self):
         """The encoder's view (kernels.encode_pages): arrays, counters and sizes."""
@@ -133,7 +139,7 @@ class CompressedKV:
         full = T - T % P
         self.T = T
         if 0 <= b < self.B and prefill_ready(x, self.sm.device, self.H, self.D):
-            used = prefill_pages(x, self._buf(), state=self.state, b=b)
+            used = prefill_pages(x, self, b=b)
             if full and used > self.cap:
                 strides = (x.stride(0), P * x.stride(1), x.stride(1), x.stride(2))
                 used = self._refit(lambda: (x, strides), b, 0, 1, full // P)
@@ -172,11 +178,8 @@ class CompressedKV:
     def _launch_append(self, x):
         """Tail write (+ at a page end: page encode, slot scan, raw-row copy, next page
         opened): one kernel that reads the token count from state[0] and advances it."""
-        _lib.call("exkv_cache_append", _lib.ptr(x, align=2, what="x"), x.stride(0), x.stride(1),
-                  _lib.ptr(self.sm), _lib.ptr(self.code), _lib.ptr(self.base), _lib.ptr(self.rowmask),
-                  _lib.ptr(self.rowoff), _lib.ptr(self.raw), _lib.ptr(self.cnt, 4), _lib.ptr(self._before, 4),
-                  _lib.ptr(self.state, 4), self.cap, self.raw.shape[0], self.B, self.H, self.TS, self.D,
-                  _lib.stream())
+        _lib.call("exkv_cache_append", _lib.ptr(x, 2, "x"), x.stride(0), x.stride(1), *self._ptrs(), self.cap,
+                  self.raw.shape[0], self.B, self.H, self.TS, self.D, _lib.stream())
 
     def _advance(self):
         """Host mirror of an append whose kernels ran (eagerly or in a graph replay)."""

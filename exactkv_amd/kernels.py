@@ -14,7 +14,9 @@ ignored and splits are planned over the buffer length), nsplit / split_len (expl
 split plan), out (output tensor).
 """
 import ctypes
+import functools
 import math
+import operator
 from array import array
 
 import torch
@@ -24,6 +26,7 @@ from . import _lib
 LOG2E = 1.4426950408889634
 P = 16
 HEAD_DIMS = (64, 128, 256)   # head dims the kernels are built for (128: the tuned attention kernels)
+_QK_SCALE = {D: D ** -0.5 * LOG2E for D in HEAD_DIMS}   # scores in log2 units
 
 
 def choose_split(B, Hkv, T, BLOCK_N, target=512):
@@ -81,14 +84,21 @@ _WS = {}  # split partials, reused per (device, stream, rows, nsplit): kernels o
 _CNT = {}  # merge arrival counters per (device, stream, units): zero between calls
 
 
-def _workspace(dev, rows, ns, D, st=None):
-    key = (dev.index, _lib.stream(dev.index) if st is None else st, rows, ns, D)
+def _partials(dev, rows, ns, D, st):
+    """A call's split partials on device dev, stream st: the addresses of o, m and l, then the
+    tensors, which the caller holds until it has launched."""
+    key = (dev.index, st, rows, ns, D)
     ws = _WS.get(key)
     if ws is None:
         f32 = dict(device=dev, dtype=torch.float32)
-        ws = _WS[key] = (torch.empty(rows, ns, D, **f32), torch.empty(rows, ns, **f32),
-                         torch.empty(rows, ns, **f32))
+        held = (torch.empty(rows, ns, D, **f32), torch.empty(rows, ns, **f32), torch.empty(rows, ns, **f32))
+        ws = _WS[key] = (*(t.data_ptr() for t in held), held)
     return ws
+
+
+def _workspace(dev, rows, ns, D):
+    """The split partials (o, m, l) of calls on dev's current stream."""
+    return _partials(dev, rows, ns, D, _lib.stream(dev.index))[3]
 
 
 def merge_units(B, Hkv, Hq):
@@ -136,14 +146,18 @@ def _fused_counters(dev, B, Hkv, Hq, ns, fused_merge):
 
 
 def _check_q(q):
-    if q.dim() != 3 or q.shape[2] not in HEAD_DIMS:
-        raise ValueError(f"q must be [B, Hq, D], D in {HEAD_DIMS} (got {tuple(q.shape)})")
+    """q's (B, Hq, D), checked."""
+    shape = q.shape
+    if len(shape) != 3 or shape[2] not in HEAD_DIMS:
+        raise ValueError(f"q must be [B, Hq, D], D in {HEAD_DIMS} (got {tuple(shape)})")
     if q.dtype != torch.bfloat16 or not q.is_contiguous() or not q.is_cuda:
         raise ValueError("q must be a contiguous bf16 GPU tensor")
+    return shape
 
 
 def _cache_args(c):
-    """(seven compressed-cache arguments, TS, Hkv, B) from a CompressedKV or its buffers() dict."""
+    """(seven compressed-cache arguments, TS, Hkv, B) from a CompressedKV, a PagedCompressedKV
+    (its pool as one sequence) or a buffers() dict."""
     if isinstance(c, dict):
         B, TS, H, D = c["shape"]
         raw = c["raw"]
@@ -172,13 +186,19 @@ def _cache_dim(c):
     return (c["sm"] if isinstance(c, dict) else c.sm).shape[-1]
 
 
+@functools.lru_cache(maxsize=4096)
+def _default_plan(B, Hkv, Hq, T, D):
+    """The default split plan, which the sizes alone determine."""
+    return plan_splits(B, Hkv, Hq, T) if D == 128 else plan_splits_hd(B, Hkv, Hq, T, D)
+
+
 def _plan(B, Hkv, Hq, T, TS, lens, nsplit, split_len, window=0, D=128):
     if nsplit is not None and split_len is not None:
         return nsplit, split_len
     reach = TS if lens is not None else T
     if window:                                 # the splits start at the window's first page
         reach = min(reach, window + P - 1)
-    return plan_splits(B, Hkv, Hq, reach) if D == 128 else plan_splits_hd(B, Hkv, Hq, reach, D)
+    return _default_plan(B, Hkv, Hq, reach, D)
 
 
 def _window_arg(window):
@@ -220,11 +240,10 @@ def attention_compressed(q, kc, vc, T, BLOCK_N=64, num_warps=4, num_stages=1, *,
 
     window > 0 (sliding-window attention; not in the reference, engine.py:26-28 rejects
     it): each sequence attends to its last `window` tokens only."""
-    _check_q(q)
+    B, Hq, D = _check_q(q)
     ka, TS, Hkv, Bc = _cache_args(kc)
     va, TSv, Hv, Bv = _cache_args(vc)
-    B, Hq, D = q.shape
-    if (TSv, Hv) != (TS, Hkv) or (Bc < B or Bv < B if block_table is None else Bc != Bv):
+    if TSv != TS or Hv != Hkv or (Bc < B or Bv < B if block_table is None else Bc != Bv):
         raise ValueError("k and v caches differ in shape or hold fewer sequences than q")
     if _cache_dim(kc) != D or _cache_dim(vc) != D:
         raise ValueError(f"cache head dim {_cache_dim(kc)} / {_cache_dim(vc)} differs from q's {D}")
@@ -232,21 +251,21 @@ def attention_compressed(q, kc, vc, T, BLOCK_N=64, num_warps=4, num_stages=1, *,
         bt, bts, cap = _block_table_arg(block_table, B)
         pool_pages = Bc * TS // P
         TS = cap
-    window = _window_arg(window)
+    window = _window_arg(window) if window else 0
     ns, sl = _plan(B, Hkv, Hq, T, TS, lens, nsplit, split_len, window, D)
-    lp, lstride = _lens_arg(lens, B)
-    st = _lib.stream(q.device.index)
-    wo, wm, wl = _workspace(q.device, B * Hq, ns, D, st)
-    cnt = _fused_counters(q.device, B, Hkv, Hq, ns, fused_merge)
+    lp, lstride = (None, 0) if lens is None else _lens_arg(lens, B)
+    dev = q.device
+    st = _lib.stream(dev.index)
+    wo, wm, wl, held = _partials(dev, B * Hq, ns, D, st)
+    cnt = _fused_counters(dev, B, Hkv, Hq, ns, True) if fused_merge else None
+    cnt = cnt.data_ptr() if cnt is not None else None
     out = torch.empty_like(q) if out is None else out
     if block_table is not None:
-        _lib.call("exkv_attn_compressed_paged", _lib.ptr(q), *ka, *va, wo.data_ptr(), wm.data_ptr(), wl.data_ptr(),
-                  cnt.data_ptr() if cnt is not None else None, _lib.ptr(out), bt, bts, pool_pages, B, Hq, Hkv, D,
-                  int(T), TS, lp, lstride, ns, sl, window, D ** -0.5 * LOG2E, st)
+        _lib.call("exkv_attn_compressed_paged", _lib.ptr(q), *ka, *va, wo, wm, wl, cnt, _lib.ptr(out), bt, bts,
+                  pool_pages, B, Hq, Hkv, D, int(T), TS, lp, lstride, ns, sl, window, _QK_SCALE[D], st)
         return out
-    _lib.call("exkv_attn_compressed", _lib.ptr(q), *ka, *va, wo.data_ptr(), wm.data_ptr(), wl.data_ptr(),
-              cnt.data_ptr() if cnt is not None else None, _lib.ptr(out), B, Hq, Hkv, D, int(T), TS, lp, lstride, ns, sl, window, D ** -0.5 * LOG2E,
-              st)
+    _lib.call("exkv_attn_compressed", _lib.ptr(q), *ka, *va, wo, wm, wl, cnt, _lib.ptr(out), B, Hq, Hkv, D, int(T), TS,
+              lp, lstride, ns, sl, window, _QK_SCALE[D], st)
     return out
 
 
@@ -283,10 +302,9 @@ def attention_reference(q, k, v, T, BLOCK_N=64, num_warps=4, num_stages=1, *, le
                         split_len=None, out=None, fused_merge=False, block_table=None, window=0):
     """Same computation on uncompressed bf16 K, V of shape [B, TS, Hkv, D] (contiguous);
     with block_table, k and v are pools of pages as in attention_compressed."""
-    _check_q(q)
+    B, Hq, D = _check_q(q)
     if k.shape != v.shape or k.dim() != 4 or k.dtype != torch.bfloat16 or not (k.is_contiguous() and v.is_contiguous()):
         raise ValueError("k and v must be contiguous bf16 [B, TS, Hkv, D] tensors of one shape")
-    B, Hq, D = q.shape
     TS, Hkv = k.shape[1], k.shape[2]
     if (block_table is None and k.shape[0] < B) or k.shape[3] != D:
         raise ValueError("k/v hold fewer sequences than q or have the wrong head dim")
@@ -296,21 +314,21 @@ def attention_reference(q, k, v, T, BLOCK_N=64, num_warps=4, num_stages=1, *, le
         bt, bts, cap = _block_table_arg(block_table, B)
         pool_pages = k.shape[0] * TS // P
         TS = cap
-    window = _window_arg(window)
+    window = _window_arg(window) if window else 0
     ns, sl = _plan(B, Hkv, Hq, T, TS, lens, nsplit, split_len, window, D)
-    lp, lstride = _lens_arg(lens, B)
-    st = _lib.stream(q.device.index)
-    wo, wm, wl = _workspace(q.device, B * Hq, ns, D, st)
-    cnt = _fused_counters(q.device, B, Hkv, Hq, ns, fused_merge)
+    lp, lstride = (None, 0) if lens is None else _lens_arg(lens, B)
+    dev = q.device
+    st = _lib.stream(dev.index)
+    wo, wm, wl, held = _partials(dev, B * Hq, ns, D, st)
+    cnt = _fused_counters(dev, B, Hkv, Hq, ns, True) if fused_merge else None
+    cnt = cnt.data_ptr() if cnt is not None else None
     out = torch.empty_like(q) if out is None else out
     if block_table is not None:
-        _lib.call("exkv_attn_bf16_paged", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), wo.data_ptr(), wm.data_ptr(),
-                  wl.data_ptr(), cnt.data_ptr() if cnt is not None else None, _lib.ptr(out), bt, bts, pool_pages, B,
-                  Hq, Hkv, D, int(T), TS, lp, lstride, ns, sl, window, D ** -0.5 * LOG2E, st)
+        _lib.call("exkv_attn_bf16_paged", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), wo, wm, wl, cnt, _lib.ptr(out), bt, bts,
+                  pool_pages, B, Hq, Hkv, D, int(T), TS, lp, lstride, ns, sl, window, _QK_SCALE[D], st)
         return out
-    _lib.call("exkv_attn_bf16", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), wo.data_ptr(), wm.data_ptr(),
-              wl.data_ptr(), cnt.data_ptr() if cnt is not None else None, _lib.ptr(out), B, Hq, Hkv, D, int(T), TS, lp, lstride, ns, sl, window,
-              D ** -0.5 * LOG2E, st)
+    _lib.call("exkv_attn_bf16", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), wo, wm, wl, cnt, _lib.ptr(out), B, Hq, Hkv, D,
+              int(T), TS, lp, lstride, ns, sl, window, _QK_SCALE[D], st)
     return out
 
 
@@ -427,31 +445,29 @@ def prefill_ready(x, dev, H, D):
             and (T % P == 0 or (x.shape[2] == H and x.shape[3] == D)))
 
 
-def prefill_pages(x, buf, *, state=None, b=0, table=None, slot=0, shape=None):
-    """Prompt x [1, T, H, D] (prefill_ready) into a cache, all of a prefill's device work in two
-    launches: full pages encoded, the rest into the open-page rows, that page opened, the token
-    count set. buf as for encode_pages. Contiguous: sequence b, state the device token count.
-    Paged: slot `slot`, table its row of the block table, shape (max_seqs, max_pages, pool
-    pages). Waits for the stream and returns the raw-row counter, which passes cap when the
-    pool overflowed, as after encode_pages."""
-    H, TS, D, T = buf["H"], buf["TS"], buf["D"], x.shape[1]
+def prefill_pages(x, c, *, b=0, table=None):
+    """Prompt x [1, T, H, D] (prefill_ready) into slot b of a cache, all of a prefill's device work in
+    two launches: full pages encoded, the rest into the open-page rows, that page opened, the
+    token count set. c: a CompressedKV, or a PagedCompressedKV with its PageTable. Waits for the
+    stream and returns the raw-row counter, which passes cap when the pool overflowed, as after
+    encode_pages."""
+    H, D, T = c.H, c.D, x.shape[1]
     s_t, s_h = x.stride(1), x.stride(2)
     if T >= P:
         _check_source(x, (x.stride(0), P * s_t, s_t, s_h), 1, T // P, H, D)
-    raw, before = buf["raw"], buf["before"]
-    ws = _scan_ws(raw.device, (T // P) * H) if (T // P) * H > DIRECT_UNITS else None
+    ptrs = c._ptrs()
+    units = (T // P) * H
+    ws = _scan_ws(c.raw.device, units) if units > DIRECT_UNITS else None
     st = _lib.stream()
-    word, count = _lib.host_words(raw.device.index)
-    args = (_lib.ptr(x, align=2, what="x"), s_t, s_h, T, _lib.ptr(buf["sm"]), _lib.ptr(buf["code"]), _lib.ptr(buf["base"]),
-            _lib.ptr(buf["rowmask"]), _lib.ptr(buf["rowoff"]), _lib.ptr(raw), _lib.ptr(buf["cnt"], align=4),
-            _lib.ptr(before, align=4))
+    word, count = _lib.host_words(c.raw.device.index)
     scan = (_lib.ptr(ws), ws.numel() if ws is not None else 0, word, st)
     if table is None:
-        _lib.call("exkv_prefill_slot", *args, _lib.ptr(state, align=4), int(buf["cap"]), raw.shape[0],
-                  buf["sm"].shape[0], int(b), H, TS, D, *scan)
+        _lib.call("exkv_prefill_slot", _lib.ptr(x, 2, "x"), s_t, s_h, T, *ptrs, c.cap, c.raw.shape[0], c.B, b, H, c.TS, D,
+                  *scan)
     else:
-        _lib.call("exkv_prefill_slot_paged", *args, int(buf["cap"]), raw.shape[0], _lib.ptr(table, align=4),
-                  int(slot), *shape, H, D, *scan)
+        row = table.block_table.data_ptr() + 4 * b * table.max_pages
+        _lib.call("exkv_prefill_slot_paged", _lib.ptr(x, 2, "x"), s_t, s_h, T, *ptrs[:8], c.cap, c.raw.shape[0], row, b,
+                  table.max_seqs, table.max_pages, table.num_pages, H, D, *scan)
     _lib.synchronize(st)
     return count[0]
 
@@ -493,20 +509,31 @@ def _paged_append_args(x, table, slots):
             _lib.ptr(bt, what="block_table"), bt.stride(0), n, H, bt.shape[0], bt.shape[1])
 
 
+def array_ptrs(memo, arrays, words):
+    """(arrays, their pointers): `memo` again while it holds the very same tensors, so that a cache
+    checks its buffers once and not in every append. arrays first (16-byte aligned), then words."""
+    if memo is not None and all(map(operator.is_, memo[0], arrays)):
+        return memo
+    n = len(arrays) - words
+    return arrays, tuple(_lib.ptr(t, 16 if i < n else 4) for i, t in enumerate(arrays))
+
+
 def append_paged(x, buf, table, slots=None):
     """One token per row of x [n, H, D] into a paged compressed cache (buf as for
     encode_pages, arrays of a [1, 16 * pool_pages, H, D] cache) whose slots, lengths and
     block table are those of `table` (lens already counting the new token). buf's 'arrivals', an
     int32 word that is zero between calls, makes it one launch at every size."""
-    sp, lp, bp, bts, n, H, ms, mp = _paged_append_args(x, table, slots)
     raw, arrivals = buf["raw"], buf.get("arrivals")
-    words = [_lib.ptr(buf["cnt"], align=4), _lib.ptr(buf["before"], align=4)]
-    if arrivals is not None:
-        words.append(_lib.ptr(arrivals, align=4))
-    _lib.call("exkv_cache_append_paged" if arrivals is None else "exkv_cache_append_paged_counted",
-              _lib.ptr(x, align=2, what="x"), x.stride(0), x.stride(1),
-              _lib.ptr(buf["sm"]), _lib.ptr(buf["code"]), _lib.ptr(buf["base"]), _lib.ptr(buf["rowmask"]),
-              _lib.ptr(buf["rowoff"]), _lib.ptr(raw), *words, int(buf["cap"]), raw.shape[0], sp, lp, bp, bts, n, H, ms, mp, buf["TS"] // P, buf["D"], _lib.stream())
+    ptrs = [_lib.ptr(buf[k]) for k in ("sm", "code", "base", "rowmask", "rowoff", "raw")]
+    ptrs += [_lib.ptr(t, 4) for t in (buf["cnt"], buf["before"], arrivals) if t is not None]
+    launch_paged_append(x, ptrs, int(buf["cap"]), raw.shape[0], buf["TS"] // P, buf["D"], table, slots)
+
+
+def launch_paged_append(x, ptrs, cap, raw_rows, pool_pages, D, table, slots):
+    """append_paged on a cache's eight pointers, or nine with the arrival word's."""
+    sp, lp, bp, bts, n, H, ms, mp = _paged_append_args(x, table, slots)
+    _lib.call("exkv_cache_append_paged" if len(ptrs) == 8 else "exkv_cache_append_paged_counted", _lib.ptr(x, 2, "x"),
+              x.stride(0), x.stride(1), *ptrs, cap, raw_rows, sp, lp, bp, bts, n, H, ms, mp, pool_pages, D, _lib.stream())
 
 
 def append_paged_bf16(x, pool, table, slots=None):

@@ -25,8 +25,8 @@ compact().
 import torch
 
 from . import _lib
-from .kernels import (HEAD_DIMS, P, append_paged, append_paged_bf16, encode_pages_paged, prefill_pages,
-                      prefill_ready, table_write)
+from .kernels import (HEAD_DIMS, P, append_paged_bf16, array_ptrs, encode_pages_paged, launch_paged_append,
+                      prefill_pages, prefill_ready, table_write)
 
 
 class PageTable:
@@ -186,8 +186,22 @@ class PagedCompressedKV:
         self.grows = 0
         self._pending = None                                   # pages filled by the last append
         self._appended = 0                                     # table step of the last append
+        self.B = 1                                             # the pool, as the attention calls read it
+        self._abi = self._ptr_memo = None
 
     # -- internals
+    def kernel_args(self):
+        """(sm, code, base, rowmask, rowoff, raw), as CompressedKV.kernel_args."""
+        if self._abi is None or self._abi[5] is not self.raw:
+            self._abi = (self.sm, self.code, self.base, self.rowmask, self.rowoff, self.raw)
+        return self._abi
+
+    def _ptrs(self):
+        """Addresses of the six arrays, cnt, _before and _arrivals."""
+        self._ptr_memo = array_ptrs(self._ptr_memo, (self.sm, self.code, self.base, self.rowmask, self.rowoff, self.raw,
+                                                     self.cnt, self._before, self._arrivals), 3)
+        return self._ptr_memo[1]
+
     def _tail(self, slot):
         """bf16 [H, 16, D] view of a slot's open page (its rows behind cap)."""
         first = self.cap + slot * self.H * P
@@ -244,7 +258,7 @@ class PagedCompressedKV:
         t = self.table
         dst = t.block_table[slot: slot + 1]
         if prefill_ready(x, self.sm.device, self.H, self.D) and t.block_table.stride(0) == t.max_pages:
-            n = prefill_pages(x, self._buf(), table=dst, slot=slot, shape=(t.max_seqs, t.max_pages, t.num_pages))
+            n = prefill_pages(x, self, b=slot, table=t)
             if Tf and n > self.cap:
                 st = (x.stride(0), P * x.stride(1), x.stride(1), x.stride(2))
                 self._grow(n)
@@ -291,7 +305,8 @@ class PagedCompressedKV:
             raise ValueError(f"append expects [{len(t._step_slots)}, {self.H}, {self.D}] (one row per step slot)")
 
     def _launch_append(self, x):
-        append_paged(x, self._buf(), self.table, self.table.step_rows()[0])
+        launch_paged_append(x, self._ptrs(), self.cap, self.raw.shape[0], self.table.num_pages, self.D, self.table,
+                            self.table.step_rows()[0])
 
     def _advance(self):
         self._appended = self.table.step
