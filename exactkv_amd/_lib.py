@@ -26,9 +26,9 @@ SIGNATURES = {
     "exkv_store_raw_rows": [_p, _i64, _i64, _i64, _i64, _p, _p, _p, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32,
                             _i32, _i32, _p],
     "exkv_prefill_slot": [_p, _i64, _i64, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _i32, _i32,
-                          _i32, _i32, _p, _i64, _p, _p],
+                          _i32, _i32, _p, _i64, _p],
     "exkv_prefill_slot_paged": [_p, _i64, _i64, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _p, _i32, _i32,
-                                _i32, _i32, _i32, _i32, _p, _i64, _p, _p],
+                                _i32, _i32, _i32, _i32, _p, _i64, _p],
     "exkv_cache_append": [_p, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _i32, _i32,
                           _i32, _p],
     "exkv_bf16_append": [_p, _i64, _i64, _p, _p, _i32, _i32, _i32, _i32, _p],
@@ -58,7 +58,7 @@ SIGNATURES = {
     "exkv_attn_bf16_paged": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _i32,
                              _p, _i64, _i32, _i32, _i32, _f32, _p],
     "exkv_table_write": [_p, _i64, _p, _i64, _p, _p, _i32, _i32, _p],
-    "exkv_gather_words": [_p, _i32, _p, _p],
+    "exkv_fetch_words": [_p, _i32, _p, _i32, _p],
     "exkv_wire_bytes": [_i32, _i32, _i64],
     "exkv_wire_count": [_p, _i64, _i32, _p, _i64, _p, _i32, _i32, _p, _p],
     "exkv_wire_check": [_i32, _p, _p, _i32, _p, _p, _p],
@@ -178,19 +178,38 @@ def synchronize(st):
 _host = threading.local()
 
 
-def host_words(index, n=1):
-    """At least n int32 words in pinned host memory that kernels on device `index` can write:
-    (their address, a ctypes array of them). One buffer per thread and device, grown on demand,
-    for calls that wait for their stream before they return and have read the words by then, so
-    no two of them use it at a time."""
+class _HostWords:
+    """int32 words in pinned host memory that kernels can write: their address, a ctypes array of
+    them, and the tag of the last fetch."""
+
+    def __init__(self, size):
+        import torch
+        self.size = size
+        self.held = torch.zeros(size, dtype=torch.int32, pin_memory=True)
+        self.addr = self.held.data_ptr()
+        self.view = (ctypes.c_int32 * size).from_address(self.addr)
+        self.tag = 0
+
+
+def host_words(index, n):
+    """At least n pinned host words for device `index`: one buffer per thread and device, grown on
+    demand, for calls that wait for their stream before they return and have read the words by
+    then, so no two of them use it at a time. Word 0 is fetch's flag."""
     bufs = _host.__dict__.setdefault("bufs", {})
     b = bufs.get(index)
-    if b is None or b[2] < n:
-        import torch
-        size = max(n, 64 if b is None else 2 * b[2])
-        t = torch.empty(size, dtype=torch.int32, pin_memory=True)
-        b = bufs[index] = (t.data_ptr(), (ctypes.c_int32 * size).from_address(t.data_ptr()), size, t)
-    return b[0], b[1]
+    if b is None or b.size < n:
+        b = bufs[index] = _HostWords(max(n, 64 if b is None else 2 * b.size))
+    return b
+
+
+def fetch(index, ptrs, st):
+    """Wait for the work queued on raw stream `st` of device `index`; the int32 words at the device
+    addresses `ptrs` (an array('Q')), as a list."""
+    n = len(ptrs)
+    w = host_words(index, n + 1)
+    w.tag = w.tag % 0x3FFFFFFF + 1
+    call("exkv_fetch_words", ptrs.buffer_info()[0], n, w.addr, w.tag, st)
+    return w.view[1:n + 1]
 
 
 def _stream_device(st):

@@ -21,7 +21,7 @@ CPU implementation in this package.
 """
 import torch
 
-from .kernels import encode_pages, store_raw_rows, decode_to_bf16, HEAD_DIMS, P
+from .kernels import encode_pages, store_raw_rows, decode_to_bf16, read_words, HEAD_DIMS, P
 
 
 def _gpu(dev):
@@ -50,7 +50,7 @@ def encode_reference(x):
                raw=torch.empty(1, D, dtype=torch.bfloat16, device=dev))
     st = (xd.stride(0), P * xd.stride(1), xd.stride(1), xd.stride(2))
     encode_pages(xd, st, buf, 0, 0, B, NP)                 # the layout and the raw rows' number (none stored)
-    n = int(buf["cnt"].item())
+    n = read_words([buf["cnt"]])[0]
     if n:
         buf["raw"] = torch.empty(n, D, dtype=torch.bfloat16, device=dev)
         buf["cap"] = n

@@ -559,12 +559,11 @@ __device__ inline int raw_rows_before(const EncArgs& a, int u0) {
 }
 
 // What a prefill does besides encoding its full pages: the rows of its last, partly filled page
-// go to the slot's open-page rows, that page is opened, the device token count is set, and the
-// raw-row counter goes to the host. One more block of the scan's launch does it beside the
-// scan, in its shadow (30 KB of rows at 8 heads of 128), instead of a fill, a strided copy, an
-// open-page launch and a copy of the counter, each with its own gap around the host's wait for
-// the counter: a layer's K and V of a 4,091-token prompt 122 -> 61 us, of which the GPU works
-// 2 x 9.
+// go to the slot's open-page rows, that page is opened, and the device token count is set. One
+// more block of the scan's launch does it beside the scan, in its shadow (30 KB of rows at 8
+// heads of 128), instead of a fill, a strided copy and an open-page launch, the last two after
+// the host's wait for the raw-row counter: a layer's K and V of a 4,091-token prompt
+// 122 -> 61 us, of which the GPU works 2 x 9.
 struct PrefillEnd {
     const uint16_t* tail = nullptr;   // token 0 of the open page, head 0 (rows s_t apart, heads s_h)
     int64_t s_t = 0, s_h = 0;
@@ -576,7 +575,6 @@ struct PrefillEnd {
     int open_pages = 0;               // pages per sequence: none is opened at or past it
     const int32_t* table = nullptr;   // paged: the slot's block-table row; its page T / 16 is opened
     int64_t pool_pages = 0;
-    int32_t* host_cnt = nullptr;      // host memory (mapped): receives the counter
 };
 
 // One block of 1,024 threads.
@@ -614,15 +612,10 @@ __device__ inline void prefill_end(const EncArgs& a, const PrefillEnd& e) {
     }
 }
 
-__device__ inline void tell_host(int32_t* p, int32_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 // A prefill's end by itself: a prompt of less than a page, or one too long for the direct scan.
 template <int D>
 __global__ void __launch_bounds__(1024) prefill_end_kernel(EncArgs a, PrefillEnd e) {
     prefill_end<D>(a, e);
-    if (threadIdx.x == 0) tell_host(e.host_cnt, *a.cnt);
 }
 
 // nscan blocks of ub units; END: one more, which does a prefill's end beside them.
@@ -661,10 +654,7 @@ __global__ void __launch_bounds__(1024) scan_direct_kernel(EncArgs a, int nunits
     if (mine) a.rowoff[page] = off;
     if (threadIdx.x == 0) {
         if (blockIdx.x == 0 && a.before != nullptr) *a.before = cnt0;
-        if ((int)blockIdx.x == nscan - 1) {
-            *a.cnt = cnt0 + total;
-            if (END) tell_host(e.host_cnt, cnt0 + total);
-        }
+        if ((int)blockIdx.x == nscan - 1) *a.cnt = cnt0 + total;
     }
     if (a.cap > 0) copy_escaped_rows<VEC16, D>(a, m, off, a.src + bi * a.s_b + pg * a.s_pg + hk * a.s_h, lane);
 }
@@ -1418,14 +1408,14 @@ extern "C" int exkv_encode_pages_paged(const void* src, int64_t s_b, int64_t s_p
 
 // A prompt into sequence slot b in two launches (one below a page of tokens): its full pages as
 // exkv_encode_pages encodes them, its last rows into the slot's open page, page T / 16 of every
-// sequence opened (exkv_cache_open_page), state[0] = T, *host_cnt = the raw-row counter.
+// sequence opened (exkv_cache_open_page), state[0] = T.
 static int prefill_slot(const char* what, EncArgs& a, PrefillEnd& e, int64_t s_t, int64_t s_h, int32_t T, int64_t slot,
                         int64_t slots, int64_t raw_rows, int32_t D, void* scan_ws, int64_t scan_ws_words,
-                        int32_t* host_cnt, hipStream_t stream) {
+                        hipStream_t stream) {
     const int64_t tail_end = a.cap + slots * a.H * kPage;
     EXKV_REQUIRE(a.cap >= 0 && tail_end <= raw_rows && tail_end <= INT32_MAX,
                  "%s: raw pool (%lld rows) smaller than cap + open-page rows", what, (long long)raw_rows);
-    EXKV_REQUIRE(a.src && a.sm && a.code && a.base && a.rowmask && a.rowoff && a.raw && a.cnt && host_cnt,
+    EXKV_REQUIRE(a.src && a.sm && a.code && a.base && a.rowmask && a.rowoff && a.raw && a.cnt,
                  "%s: null pointer", what);
     EXKV_REQUIRE(s_t >= 0 && s_h >= 0, "%s: negative source strides", what);
     const int64_t n = (int64_t)a.npg * a.H;
@@ -1440,7 +1430,6 @@ static int prefill_slot(const char* what, EncArgs& a, PrefillEnd& e, int64_t s_t
     e.rows = T % kPage;
     e.tail0 = a.cap + slot * a.H * kPage;
     e.T = T;
-    e.host_cnt = host_cnt;
     launch_encode(a, n, (uint64_t*)scan_ws, scan_ws_words, &e, stream);
     return launch_status(what);
 }
@@ -1448,8 +1437,7 @@ static int prefill_slot(const char* what, EncArgs& a, PrefillEnd& e, int64_t s_t
 extern "C" int exkv_prefill_slot(const void* src, int64_t s_t, int64_t s_h, int32_t T, void* sm, void* code, void* base,
                                  int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before,
                                  int32_t* state, int64_t cap, int64_t raw_rows, int32_t B, int32_t b, int32_t H,
-                                 int32_t TS, int32_t D, void* scan_ws, int64_t scan_ws_words, int32_t* host_cnt,
-                                 hipStream_t stream) {
+                                 int32_t TS, int32_t D, void* scan_ws, int64_t scan_ws_words, hipStream_t stream) {
     EXKV_REQUIRE(head_dim_ok(D), "prefill_slot: head dim must be 64, 128 or 256 (got %d)", D);
     EXKV_REQUIRE(TS > 0 && TS % kPage == 0 && B > 0 && H > 0, "prefill_slot: bad shape B=%d H=%d TS=%d", B, H, TS);
     EXKV_REQUIRE(b >= 0 && b < B && T >= 0 && T <= TS, "prefill_slot: %d tokens into slot %d outside the cache", T, b);
@@ -1460,7 +1448,7 @@ extern "C" int exkv_prefill_slot(const void* src, int64_t s_t, int64_t s_h, int3
     e.state = state;
     e.B = B;
     e.open_pages = TS / kPage;
-    return prefill_slot("prefill_slot", a, e, s_t, s_h, T, b, B, raw_rows, D, scan_ws, scan_ws_words, host_cnt, stream);
+    return prefill_slot("prefill_slot", a, e, s_t, s_h, T, b, B, raw_rows, D, scan_ws, scan_ws_words, stream);
 }
 
 // The same into slot `slot` of a paged cache: its page p is pool page table[p] (entries clamped
@@ -1469,8 +1457,7 @@ extern "C" int exkv_prefill_slot_paged(const void* src, int64_t s_t, int64_t s_h
                                        void* base, int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt,
                                        int32_t* before, int64_t cap, int64_t raw_rows, const int32_t* table,
                                        int32_t slot, int32_t max_seqs, int32_t max_pages, int32_t pool_pages, int32_t H,
-                                       int32_t D, void* scan_ws, int64_t scan_ws_words, int32_t* host_cnt,
-                                       hipStream_t stream) {
+                                       int32_t D, void* scan_ws, int64_t scan_ws_words, hipStream_t stream) {
     EXKV_REQUIRE(head_dim_ok(D), "prefill_slot_paged: head dim must be 64, 128 or 256 (got %d)", D);
     EXKV_REQUIRE(H > 0 && max_seqs > 0 && max_pages > 0 && pool_pages > 0, "prefill_slot_paged: bad shape");
     EXKV_REQUIRE(slot >= 0 && slot < max_seqs && T >= 0 && T <= (int64_t)max_pages * kPage,
@@ -1486,7 +1473,7 @@ extern "C" int exkv_prefill_slot_paged(const void* src, int64_t s_t, int64_t s_h
     e.table = table;
     e.pool_pages = pool_pages;
     return prefill_slot("prefill_slot_paged", a, e, s_t, s_h, T, slot, max_seqs, raw_rows, D, scan_ws, scan_ws_words,
-                        host_cnt, stream);
+                        stream);
 }
 
 extern "C" int exkv_cache_append(const void* x, int64_t sx_b, int64_t sx_h, void* sm, void* code, void* base,

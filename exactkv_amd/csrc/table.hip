@@ -6,6 +6,8 @@
 //
 // No counterpart in the reference (its token count and counters are read and written by torch
 // calls, cache.py:57-60,149-158; paged KV is in its future work, README.md:121-123).
+#include <chrono>
+
 #include "common.hpp"
 #include "../../include/exactkv.h"
 
@@ -28,9 +30,13 @@ __global__ void __launch_bounds__(kPairs) table_write_kernel(int32_t* lens, int3
 struct Words {
     const int32_t* p[kWords];
 };
-__global__ void __launch_bounds__(kWords) gather_words_kernel(Words w, int n, int32_t* out) {
+// The words to out, then the tag to *done.
+__global__ void __launch_bounds__(kWords) fetch_words_kernel(Words w, int n, int32_t* out, int32_t* done, int32_t tag) {
     const int i = threadIdx.x;
     if (i < n) __hip_atomic_store(out + i, *w.p[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+    __syncthreads();
+    if (i == 0) __hip_atomic_store(done, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace exkv
@@ -62,16 +68,40 @@ extern "C" int exkv_table_write(int32_t* lens, int64_t lens_size, int32_t* table
     return hip_status(hipGetLastError(), "table_write");
 }
 
-extern "C" int exkv_gather_words(const int32_t* const* words, int32_t n, int32_t* host_out, hipStream_t stream) {
-    EXKV_REQUIRE(n >= 0 && (n == 0 || (words && host_out)), "gather_words: null pointer");
+// The stream's last kernel here says through mapped host memory that everything before it is
+// done, and the host polls for that: 6.4 us from the launch to the answer on an idle stream,
+// where a launch and hipStreamSynchronize take 11.9. After kPollUs without it (a long queue)
+// the stream is waited for instead.
+constexpr int kPollUs = 200;
+
+extern "C" int exkv_fetch_words(const int32_t* const* words, int32_t n, int32_t* host, int32_t tag, hipStream_t stream) {
+    EXKV_REQUIRE(n >= 0 && host && (n == 0 || words), "fetch_words: null pointer");
+    for (int32_t i = 0; i < n; ++i) EXKV_REQUIRE(words[i], "fetch_words: null word %d", i);
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(stream, &capturing);
+    if (e != hipSuccess) return hip_status(e, "fetch_words");
+    EXKV_REQUIRE(capturing == hipStreamCaptureStatusNone, "fetch_words: the stream is being captured");
     Words w;
-    for (int32_t i0 = 0; i0 < n; i0 += kWords) {
+    int32_t i0 = 0;
+    do {
         const int32_t m = n - i0 < kWords ? n - i0 : kWords;
-        for (int32_t i = 0; i < m; ++i) {
-            EXKV_REQUIRE(words[i0 + i], "gather_words: null word %d", i0 + i);
-            w.p[i] = words[i0 + i];
+        for (int32_t i = 0; i < m; ++i) w.p[i] = words[i0 + i];
+        // only the last launch's tag is the call's
+        hipLaunchKernelGGL(fetch_words_kernel, dim3(1), dim3(m < 1 ? 64 : (m + 63) / 64 * 64), 0, stream, w, m,
+                           host + 1 + i0, host, i0 + m < n ? ~tag : tag);
+        i0 += kWords;
+    } while (i0 < n);
+    e = hipGetLastError();
+    if (e != hipSuccess) return hip_status(e, "fetch_words");
+    const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(kPollUs);
+    do {
+        for (int k = 0; k < 64; ++k) {
+            if (__atomic_load_n(host, __ATOMIC_ACQUIRE) == tag) return EXKV_OK;
+            __builtin_ia32_pause();
         }
-        hipLaunchKernelGGL(gather_words_kernel, dim3(1), dim3((m + 63) / 64 * 64), 0, stream, w, m, host_out + i0);
-    }
-    return hip_status(hipGetLastError(), "gather_words");
+    } while (std::chrono::steady_clock::now() < end);
+    e = hipStreamSynchronize(stream);
+    if (e != hipSuccess) return hip_status(e, "fetch_words");
+    EXKV_REQUIRE(__atomic_load_n(host, __ATOMIC_ACQUIRE) == tag, "fetch_words: no answer from the GPU");
+    return EXKV_OK;
 }

@@ -459,8 +459,7 @@ def prefill_pages(x, c, *, b=0, table=None):
     units = (T // P) * H
     ws = _scan_ws(c.raw.device, units) if units > DIRECT_UNITS else None
     st = _lib.stream()
-    word, count = _lib.host_words(c.raw.device.index)
-    scan = (_lib.ptr(ws), ws.numel() if ws is not None else 0, word, st)
+    scan = (_lib.ptr(ws), ws.numel() if ws is not None else 0, st)
     if table is None:
         _lib.call("exkv_prefill_slot", _lib.ptr(x, 2, "x"), s_t, s_h, T, *ptrs, c.cap, c.raw.shape[0], c.B, b, H, c.TS, D,
                   *scan)
@@ -468,8 +467,7 @@ def prefill_pages(x, c, *, b=0, table=None):
         row = table.block_table.data_ptr() + 4 * b * table.max_pages
         _lib.call("exkv_prefill_slot_paged", _lib.ptr(x, 2, "x"), s_t, s_h, T, *ptrs[:8], c.cap, c.raw.shape[0], row, b,
                   table.max_seqs, table.max_pages, table.num_pages, H, D, *scan)
-    _lib.synchronize(st)
-    return count[0]
+    return _lib.fetch(c.raw.device.index, array("Q", ptrs[6:7]), st)[0]
 
 
 def table_write(lens, block_table, lens_at, lens_val, table_at, table_val):
@@ -490,12 +488,7 @@ def read_words(words):
     """The values of one-element int32 tensors of one GPU, after the work queued on its current
     stream: one launch and a wait."""
     dev = words[0].device.index
-    st = _lib.stream(dev)
-    addr, out = _lib.host_words(dev, len(words))
-    at = array("Q", [_lib.ptr(w, align=4) for w in words])
-    _lib.call("exkv_gather_words", at.buffer_info()[0], len(at), addr, st)
-    _lib.synchronize(st)
-    return out[:len(at)]
+    return _lib.fetch(dev, array("Q", [_lib.ptr(w, align=4) for w in words]), _lib.stream(dev))
 
 
 def _paged_append_args(x, table, slots):

@@ -22,6 +22,7 @@ rowoff is implicit (the running count of raw rows in (page, head) order), so a b
 does not depend on where its rows sat in the source pool.
 """
 import struct
+from array import array
 
 import numpy as np
 import torch
@@ -31,6 +32,7 @@ from .cache import CompressedKV
 from .kernels import P
 from .paged import PagedCompressedKV, _popc16
 
+_NO_WORDS = array("Q")
 HEADER = 256
 MAGIC = 0x564B5845
 VERSION = 1
@@ -165,11 +167,11 @@ def pack_many(cache, seqs):
     d, width = _upload(host, dev), host["pages"].shape[1]
     d["ws"], ws_stride, max_t = _scratch(cache, infos, dev)
     st = _lib.stream()
-    addr, counts = _lib.host_words(dev.index, n)
+    hw = _lib.host_words(dev.index, n + 1)
     _lib.call("exkv_wire_count", _lib.ptr(cache.rowmask), infos[0][3], n, d["pages"].data_ptr(), width,
-              d["tokens"].data_ptr(), max_t, H, addr, st)
-    _lib.synchronize(st)
-    blobs = [torch.empty(nbytes(H, i[0], c), dtype=torch.uint8, device=dev) for i, c in zip(infos, counts)]
+              d["tokens"].data_ptr(), max_t, H, hw.addr + 4, st)
+    _lib.fetch(dev.index, _NO_WORDS, st)
+    blobs = [torch.empty(nbytes(H, i[0], c), dtype=torch.uint8, device=dev) for i, c in zip(infos, hw.view[1:n + 1])]
     d.update(_upload(_host_blobs(blobs), dev))
     _lib.call("exkv_wire_pack", _lib.ptr(cache.sm), _lib.ptr(cache.code), _lib.ptr(cache.base),
               _lib.ptr(cache.rowmask), _lib.ptr(cache.rowoff), _lib.ptr(cache.raw), cache.raw.shape[0], infos[0][3],
@@ -221,12 +223,11 @@ def unpack_many(blobs, cache, seqs):
     blobs = [b if b.device == dev else b.to(dev) for b in blobs]
     up = _upload(_host_blobs(blobs), dev)
     st = _lib.stream()
-    addr, facts = _lib.host_words(dev.index, 65 * n + 1)
+    hw = _lib.host_words(dev.index, 65 * n + 2)
     _lib.call("exkv_wire_check", n, up["blobs"].data_ptr(), up["sizes"].data_ptr(), cache.H, _lib.ptr(cache.cnt, align=4),
-              addr, st)
-    _lib.synchronize(st)
-    head, cnt = bytes(facts)[:HEADER * n], facts[65 * n]
-    rows = facts[64 * n:65 * n]
+              hw.addr + 4, st)
+    _lib.fetch(dev.index, _NO_WORDS, st)
+    head, rows, cnt = bytes(hw.view)[4:4 + HEADER * n], hw.view[1 + 64 * n:1 + 65 * n], hw.view[1 + 65 * n]
     heads = [_check_blob(_Read(b, head[HEADER * i:HEADER * (i + 1)], rows[i]), cache) for i, b in enumerate(blobs)]
     if cache._pending is not None:
         raise RuntimeError("call check_overflow() before unpacking")

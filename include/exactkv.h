@@ -101,14 +101,13 @@ int exkv_store_raw_rows(const void* src, int64_t s_b, int64_t s_pg, int64_t s_p,
  * s_t, s_h for token and head; channels contiguous). Its T / 16 full pages are encoded as by
  * exkv_encode_pages; the other rows go to the slot's open-page rows, raw rows
  * cap + (b*H + h)*16 on; page T / 16 of every sequence is opened as by exkv_cache_open_page;
- * state[0] = T; and *host_cnt (host memory that the GPU can write, such as hipHostMalloc's)
- * receives the raw-row counter, valid once the stream has been waited for (*host_cnt > cap:
- * overflow, as for exkv_encode_pages). Two launches up to 65,536 pages x heads.
- * Replaces: cache.py:87-98 (encode, open-page copy) and the counter read that follows. */
+ * and state[0] = T. Two launches up to 65,536 pages x heads. Overflow shows in *cnt, as for
+ * exkv_encode_pages.
+ * Replaces: cache.py:87-98 (encode, open-page copy). */
 int exkv_prefill_slot(const void* src, int64_t s_t, int64_t s_h, int32_t T, void* sm, void* code, void* base,
                       int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before, int32_t* state,
                       int64_t cap, int64_t raw_rows, int32_t B, int32_t b, int32_t H, int32_t TS, int32_t D,
-                      void* scan_ws, int64_t scan_ws_words, int32_t* host_cnt, hipStream_t stream);
+                      void* scan_ws, int64_t scan_ws_words, hipStream_t stream);
 
 /* The same into slot `slot` of a paged cache whose page p is pool page table[p] (max_pages
  * entries, clamped to the pool); page T / 16 of the slot is opened where the table has it. */
@@ -116,7 +115,7 @@ int exkv_prefill_slot_paged(const void* src, int64_t s_t, int64_t s_h, int32_t T
                             int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before, int64_t cap,
                             int64_t raw_rows, const int32_t* table, int32_t slot, int32_t max_seqs,
                             int32_t max_pages, int32_t pool_pages, int32_t H, int32_t D, void* scan_ws,
-                            int64_t scan_ws_words, int32_t* host_cnt, hipStream_t stream);
+                            int64_t scan_ws_words, hipStream_t stream);
 
 /* The page encoder into a paged cache: page pg of source sequence bi goes to page
  * dst_pages[bi*dst_stride + pg] of the B x TS arrays read as a list of B*TS/16 pages (entries
@@ -154,10 +153,11 @@ int exkv_bf16_append(const void* x, int64_t sx_b, int64_t sx_h, void* buf, int32
 int exkv_table_write(int32_t* lens, int64_t lens_size, int32_t* table, int64_t table_size, const int32_t* at,
                      const int32_t* val, int32_t n_lens, int32_t n, hipStream_t stream);
 
-/* The device words at n addresses (a host array) to host_out[0 .. n) (host memory that the GPU
- * can write; valid once the stream has been waited for): the overflow check's counters.
- * Part of what replaces: cache.py:149-158. */
-int exkv_gather_words(const int32_t* const* words, int32_t n, int32_t* host_out, hipStream_t stream);
+/* Waits for the work queued on the stream, then has the device words at n addresses (a host
+ * array) in host[1 .. n]; host (n + 1 words that the GPU can write) [0] is the call's flag and
+ * must not hold `tag`, which no call still in flight on it has. Not on a capturing stream.
+ * Part of what replaces: the counter reads of cache.py:57-60,149-158. */
+int exkv_fetch_words(const int32_t* const* words, int32_t n, int32_t* host, int32_t tag, hipStream_t stream);
 
 /* Append one token for each of n sequences of a paged cache: a pool of pool_pages pages
  * (arrays as a [1, 16 * pool_pages, H, D] cache) shared by max_seqs sequence slots.

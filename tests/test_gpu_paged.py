@@ -366,3 +366,6 @@ def test_read_words():
     words = [torch.full((1,), i * 7 - 3, dtype=torch.int32, device=DEV) for i in range(1003)]
     for n in (1, 64, 448, 449, 1003):
         assert kernels.read_words(words[:n]) == [i * 7 - 3 for i in range(n)]
+    torch.cuda._sleep(20_000_000)                      # longer than the host polls
+    words[1].fill_(99)
+    assert kernels.read_words(words[:2]) == [-3, 99]
