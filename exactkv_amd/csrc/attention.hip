@@ -143,39 +143,59 @@ struct AttnArgs {
 // head) row with lane = channel pair, the sums over s in order with explicit fmas -- the
 // order of the fused merge's one-level case, so both produce the same bits.
 __device__ inline float fast_exp2(float x);
+// Over the wavefront by DPP row rotations and the row-swap permutes, all VALU: six shuffles
+// through the LDS (a merge's longest chain after its loads) cost 0.3 us of every call.
+template <int N>
+__device__ inline float row_ror(float x) {             // lane i of a 16-lane row: lane (i - N) % 16 of it
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x120 + N, 0xf, 0xf, false));
+}
+__device__ inline float group_max(float x);
+__device__ inline float group_sum(float x);
 __device__ inline float wave_max(float x) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) x = fmaxf(x, __shfl_xor(x, d));
-    return x;
+    x = fmaxf(x, row_ror<8>(x));
+    x = fmaxf(x, row_ror<4>(x));
+    x = fmaxf(x, row_ror<2>(x));
+    x = fmaxf(x, row_ror<1>(x));
+    return group_max(x);
 }
 __device__ inline uint32_t pack_bf16x2(float a, float b) {
     const __bf16 r0 = (__bf16)a, r1 = (__bf16)b;
     return (uint32_t)__builtin_bit_cast(uint16_t, r0) | ((uint32_t)__builtin_bit_cast(uint16_t, r1) << 16);
 }
-// ns <= N splits in one round trip: m, l and o loads issued together.
-template <int N>
-__device__ __attribute__((always_inline)) inline uint32_t merge_direct(const float* po, const float* m,
-                                                                        const float* l, int ns, int lane) {
-    const float2* po2 = reinterpret_cast<const float2*>(po);
+// One row of head dim D, ns <= N splits in one round trip (m, l and o loads issued together):
+// lane = D / 64 consecutive channels; the sums run over the splits in order with fmas.
+template <int N, int D>
+__device__ __attribute__((always_inline)) inline void merge_direct(const float* po, const float* m, const float* l,
+                                                                   uint16_t* out, int ns, int lane) {
+    constexpr int C = D / 64;
+    typedef float fC __attribute__((ext_vector_type(C)));
     const float mv = lane < ns ? m[lane] : -INFINITY;
     const float lv = lane < ns ? l[lane] : 0.f;
-    float2 o[N];
+    fC o[N];
 #pragma unroll
     for (int i = 0; i < N; ++i)
-        if (i < ns) o[i] = po2[(int64_t)i * (kD / 2) + lane];
+        if (i < ns) o[i] = *reinterpret_cast<const fC*>(po + (int64_t)i * D + C * lane);
     const float M = wave_max(mv);
     const float ws = fast_exp2(mv - M);
-    float n0 = 0.f, n1 = 0.f, den = 0.f;
+    float n[C], den = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) n[c] = 0.f;
 #pragma unroll
     for (int i = 0; i < N; ++i)
         if (i < ns) {
             const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ws), i));
             const float li = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lv), i));
-            n0 = __builtin_fmaf(o[i].x, w, n0);
-            n1 = __builtin_fmaf(o[i].y, w, n1);
+#pragma unroll
+            for (int c = 0; c < C; ++c) n[c] = __builtin_fmaf(o[i][c], w, n[c]);
             den = __builtin_fmaf(li, w, den);
         }
-    return pack_bf16x2(n0 / den, n1 / den);
+    uint16_t* dst = out + C * lane;
+    if constexpr (C == 1) {
+        dst[0] = __builtin_bit_cast(uint16_t, (__bf16)(n[0] / den));
+    } else {
+#pragma unroll
+        for (int c = 0; c < C; c += 2) reinterpret_cast<uint32_t*>(dst)[c / 2] = pack_bf16x2(n[c] / den, n[c + 1] / den);
+    }
 }
 __device__ inline bf16x8 as_bf16x8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
     u32x4 u = {a, b, c, d};
@@ -1270,13 +1290,13 @@ __global__ void __launch_bounds__(kThreads) attn_split_kernel<false>(AttnArgs a)
 }
 
 // Separate merge of up to 32 splits: one wavefront per (sequence, query head) row, every
-// load of the row in flight at once (the fused merge's code, so both give the same bits).
+// load of the row in flight at once (at head dim 128 the fused merge's arithmetic, so both give
+// the same bits).
+template <int D>
 __global__ void __launch_bounds__(64) attn_reduce_kernel(const float* po, const float* pm, const float* pl,
                                                          uint16_t* out, int ns) {
     const int64_t row = blockIdx.x;
-    const int lane = threadIdx.x & 63;
-    reinterpret_cast<uint32_t*>(out + row * kD)[lane] =
-        merge_direct<32>(po + row * ns * kD, pm + row * ns, pl + row * ns, ns, lane);
+    merge_direct<32, D>(po + row * ns * D, pm + row * ns, pl + row * ns, out + row * D, ns, threadIdx.x & 63);
 }
 
 // Separate merge of more than 32 splits: workgroup (row, 16-channel chunk) of four
@@ -1288,15 +1308,19 @@ __global__ void __launch_bounds__(64) attn_reduce_kernel(const float* po, const 
 // waits for a first pass over m. Empty splits (m = -inf) weigh 0, and a wavefront whose
 // splits are all empty adds 0. The sums combine over sg by shuffles, then over the
 // wavefronts in order through LDS, each rescaled to the row's largest m. Deterministic,
-// so the compressed call and its twin still agree bit for bit.
+// so the compressed call and its twin still agree bit for bit. At head dims 64 and 256, where
+// one wavefront took 32 splits of a row after another, whole calls / with this merge: 14q/2kv at
+// 64, 1 x 4093 (256 splits) 24.7 / 12.5 us, 32q/8kv 1 x 32763 32.4 / 20.3; 16q/2kv at 256,
+// 1 x 32768 38.0 / 23.7.
 constexpr int kWideWaves = 4, kWideChunk = 16;
+template <int D>
 __global__ void __launch_bounds__(64 * kWideWaves) attn_reduce_wide_kernel(const float* po, const float* pm,
                                                                             const float* pl, uint16_t* out, int ns) {
     const int64_t row = blockIdx.x;
     const int c0 = kWideChunk * (int)blockIdx.y;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int sg = lane >> 3, cp = lane & 7;
-    const float* o = po + row * ns * kD + c0 + 2 * cp;
+    const float* o = po + row * ns * D + c0 + 2 * cp;
     const float* m = pm + row * ns;
     const float* l = pl + row * ns;
     __shared__ float part[kWideWaves][4][8];
@@ -1309,7 +1333,7 @@ __global__ void __launch_bounds__(64 * kWideWaves) attn_reduce_wide_kernel(const
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int s = min(b0 + 8 * i + sg, s1 - 1);           // past the range: a valid split, weight 0
-            v[i] = *reinterpret_cast<const float2*>(o + (int64_t)s * kD);
+            v[i] = *reinterpret_cast<const float2*>(o + (int64_t)s * D);
             mv[i] = m[s];
             lv[i] = l[s];
         }
@@ -1335,12 +1359,9 @@ __global__ void __launch_bounds__(64 * kWideWaves) attn_reduce_wide_kernel(const
             den = __builtin_fmaf(lv[i], w, den);
         }
     }
-#pragma unroll
-    for (int d = 8; d < 64; d <<= 1) {
-        n0 += __shfl_xor(n0, d);
-        n1 += __shfl_xor(n1, d);
-        den += __shfl_xor(den, d);
-    }
+    n0 = group_sum(n0 + row_ror<8>(n0));               // over sg
+    n1 = group_sum(n1 + row_ror<8>(n1));
+    den = group_sum(den + row_ror<8>(den));
     if (sg == 0) {
         part[wave][0][cp] = n0;
         part[wave][1][cp] = n1;
@@ -1361,7 +1382,7 @@ __global__ void __launch_bounds__(64 * kWideWaves) attn_reduce_wide_kernel(const
             a1 = __builtin_fmaf(part[w][1][cp], f, a1);
             dn = __builtin_fmaf(part[w][2][cp], f, dn);
         }
-        reinterpret_cast<uint32_t*>(out + row * kD + c0)[cp] = pack_bf16x2(a0 / dn, a1 / dn);
+        reinterpret_cast<uint32_t*>(out + row * D + c0)[cp] = pack_bf16x2(a0 / dn, a1 / dn);
     }
 }
 
@@ -1983,58 +2004,6 @@ __global__ void __launch_bounds__(64 * (D >= 256 ? 2 : 4)) attn_dgen_kernel(Attn
     }
 }
 
-// Split merge for head dims 64 and 256: one wavefront per (sequence, query head) row, lane
-// = D/64 consecutive channels. The splits go in batches of 32 with every load of a batch in
-// flight (lane s of the batch reads m and l of split s, every lane its channels of each
-// split's o); the sums run over s in order with fmas (out = sum o_s w_s / sum l_s w_s, w_s
-// = 2^(m_s - max m)). Used by the compressed call and its twin alike.
-template <int D>
-__global__ void __launch_bounds__(64) attn_reduce_d_kernel(const float* po, const float* pm, const float* pl,
-                                                           uint16_t* out, int ns) {
-    constexpr int C = D / 64;
-    constexpr int NBATCH = 32;
-    typedef float fC __attribute__((ext_vector_type(C)));
-    const int64_t row = blockIdx.x;
-    const int lane = threadIdx.x & 63;
-    const float* m = pm + row * ns;
-    const float* l = pl + row * ns;
-    const float* o = po + row * ns * D + lane * C;
-    float M = -INFINITY;
-    for (int s = lane; s < ns; s += 64) M = fmaxf(M, m[s]);
-    M = wave_max(M);
-    fC n;
-#pragma unroll
-    for (int c = 0; c < C; ++c) n[c] = 0.f;
-    float den = 0.f;
-    for (int s0 = 0; s0 < ns; s0 += NBATCH) {
-        const int nb = min(NBATCH, ns - s0);
-        const float mv = lane < nb ? m[s0 + lane] : -INFINITY;
-        const float lv = lane < nb ? l[s0 + lane] : 0.f;
-        fC v[NBATCH];
-#pragma unroll
-        for (int i = 0; i < NBATCH; ++i)
-            if (i < nb) v[i] = *reinterpret_cast<const fC*>(o + (int64_t)(s0 + i) * D);
-        const float ws = fast_exp2(mv - M);
-#pragma unroll
-        for (int i = 0; i < NBATCH; ++i)
-            if (i < nb) {
-                const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ws), i));
-                const float li = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lv), i));
-#pragma unroll
-                for (int c = 0; c < C; ++c) n[c] = __builtin_fmaf(v[i][c], w, n[c]);
-                den = __builtin_fmaf(li, w, den);
-            }
-    }
-    uint16_t* dst = out + row * D + lane * C;
-    if constexpr (C == 1) {
-        const __bf16 r = (__bf16)(n[0] / den);
-        dst[0] = __builtin_bit_cast(uint16_t, r);
-    } else {
-#pragma unroll
-        for (int c = 0; c < C; c += 2) reinterpret_cast<uint32_t*>(dst)[c / 2] = pack_bf16x2(n[c] / den, n[c + 1] / den);
-    }
-}
-
 // ---- head dim 64 as pairs of KV heads (attn_pair_kernel)
 //
 // KV heads 2v and 2v + 1 of a token row are 64 + 64 contiguous bytes of sm, 32 + 32 of
@@ -2055,7 +2024,7 @@ __global__ void __launch_bounds__(64) attn_reduce_d_kernel(const float* po, cons
 //     head 2v+1;
 //   * metadata and raw rows per real head: up to kRawPair raw rows (128 bytes each) of a
 //     page travel through the wavefront's raw slot, in the order 2v K, 2v V, 2v+1 K, 2v+1 V;
-//   * partials per real head (64 channels), merged by attn_reduce_d_kernel<64>, or the
+//   * partials per real head (64 channels), merged by attn_reduce_kernel<64>, or the
 //     output itself for one split.
 // The compressed kernel and its bf16 twin share the per-page arithmetic: same bits.
 constexpr int kDp = 64;
@@ -2225,7 +2194,7 @@ static_assert(Ring<true>::per_wave >= 2 * kMoHeadP && Ring<false>::per_wave >= 2
               "a page phase's partials of both heads fit its wavefront's ring");
 
 // One split per row: the output with the merge's arithmetic for a single term (as
-// store_direct; attn_reduce_d_kernel<64> at ns = 1 gives the same bits)
+// store_direct; attn_reduce_kernel<64> at ns = 1 gives the same bits)
 __device__ inline void store_direct_d64(const AttnArgs& a, int64_t orow, int g, const f32x4 (&o)[4], float m,
                                         float l) {
     const float w = fast_exp2(m - m);
@@ -2773,17 +2742,24 @@ extern "C" int exkv_time_next_split(hipEvent_t start, hipEvent_t stop) {
     return EXKV_OK;
 }
 
+template <int D>
+static void launch_reduce_d(const float* o, const float* m, const float* l, uint16_t* out, int64_t rows, int ns,
+                            hipStream_t stream) {
+    if (ns <= 32)
+        hipLaunchKernelGGL(attn_reduce_kernel<D>, dim3((unsigned)rows), dim3(64), 0, stream, o, m, l, out, ns);
+    else
+        hipLaunchKernelGGL(attn_reduce_wide_kernel<D>, dim3((unsigned)rows, D / kWideChunk), dim3(64 * kWideWaves), 0,
+                           stream, o, m, l, out, ns);
+}
+
 static int launch_reduce(const float* o, const float* m, const float* l, void* out, int64_t rows, int ns, int D,
                          hipStream_t stream) {
     if (D == 64)
-        hipLaunchKernelGGL(attn_reduce_d_kernel<64>, dim3((unsigned)rows), dim3(64), 0, stream, o, m, l, (uint16_t*)out, ns);
+        launch_reduce_d<64>(o, m, l, (uint16_t*)out, rows, ns, stream);
     else if (D == 256)
-        hipLaunchKernelGGL(attn_reduce_d_kernel<256>, dim3((unsigned)rows), dim3(64), 0, stream, o, m, l, (uint16_t*)out, ns);
-    else if (ns <= 32)
-        hipLaunchKernelGGL(attn_reduce_kernel, dim3((unsigned)rows), dim3(64), 0, stream, o, m, l, (uint16_t*)out, ns);
+        launch_reduce_d<256>(o, m, l, (uint16_t*)out, rows, ns, stream);
     else
-        hipLaunchKernelGGL(attn_reduce_wide_kernel, dim3((unsigned)rows, kD / kWideChunk), dim3(64 * kWideWaves), 0,
-                           stream, o, m, l, (uint16_t*)out, ns);
+        launch_reduce_d<128>(o, m, l, (uint16_t*)out, rows, ns, stream);
     return hip_status(hipGetLastError(), "attn_reduce");
 }
 

@@ -304,3 +304,29 @@ def test_one_split_writes_the_merge_bits(B, T, Hq, Hkv, window):
     lo = T - window if window else 0
     ref = oatt.attention(u16(q), u16(k[:, lo:T]), u16(v[:, lo:T]), T - lo, np.float32)
     assert_bf16_tolerance(direct, ref)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("ns", [1, 2, 31, 32, 33, 64, 65, 255, 256, 257, 1000])
+def test_split_merge_widths(D, ns):
+    """The separate merge at the edges of its one-wavefront and wide forms, every head dim, some
+    splits empty: within bf16 rounding (2^-8 of the value) and fp32 summation (ns + 16 roundings
+    of 2^-24, of the terms' absolute sum) of float64."""
+    from exactkv_amd import _lib
+    rows = 5
+    g = torch.Generator(device="cuda").manual_seed(ns + D)
+    o = torch.randn(rows, ns, D, generator=g, device="cuda")
+    m = 8 * torch.randn(rows, ns, generator=g, device="cuda")
+    l = torch.rand(rows, ns, generator=g, device="cuda") + 0.5
+    empty = torch.rand(rows, ns, generator=g, device="cuda") < 0.3
+    empty[:, ns // 2] = False
+    m[empty], l[empty], o[empty] = -float("inf"), 0.0, 0.0
+    out = torch.empty(rows, D, dtype=torch.bfloat16, device="cuda")
+    _lib.call("exkv_attn_reduce", o.data_ptr(), m.data_ptr(), l.data_ptr(), out.data_ptr(), rows, ns, D, _lib.stream())
+    w = torch.exp2(m.double() - m.double().max(1, keepdim=True).values)
+    den = (l.double() * w).sum(1, keepdim=True)
+    ref = (o.double() * w[..., None]).sum(1) / den
+    slack = 2.0 ** -8 * ref.abs() + (ns + 16) * 2.0 ** -24 * (o.double().abs() * w[..., None]).sum(1) / den
+    # exp2 of a difference rounded to fp32: |m| up to 64 rounds to 2^-18, a weight to ln 2 * 2^-18
+    slack = slack + 2.0 ** -18 * (o.double().abs() * w[..., None]).sum(1) / den + 2.0 ** -18 * ref.abs()
+    assert bool(((out.double() - ref).abs() <= slack).all())
