@@ -174,7 +174,9 @@ extern "C" int exkv_plan_splits_hd(int32_t B, int32_t Hkv, int32_t Hq, int32_t T
     }
     const int64_t units = (int64_t)B * Hkv * ((Hq / Hkv + 15) / 16);
     if (D == 256) {
-        plan_core(units, T, 512, 64, 2, kRampD256, scratch_splits(B, Hq, D), nsplit, split_len);
+        // down to a page per phase: 1 x 1000 at 32q/8kv 32 x 32 11.8 us, 16 x 64 13.3; 1 x 4093 at
+        // 16q/2kv 128 x 32 11.3, 64 x 64 13.3, 256 x 16 12.5
+        plan_core(units, T, 512, 32, 2, kRampD256, scratch_splits(B, Hq, D), nsplit, split_len);
         return EXKV_OK;
     }
     const int64_t slots = units < 512 ? 768 : 512, cap = std::max<int64_t>(1, ((int64_t)T + 63) / 64);

@@ -127,6 +127,7 @@ def test_plan_splits_hd(B, Hkv, Hq, T, D, expect):
     (9, 8, 32, 4093, 256, 512, (7, 592)),      # 72 units, two workgroups per CU
     (65, 8, 32, 4093, 128, 256, (5, 832)),     # 130 units: three rounds, 2.5 of them filled
     (220, 8, 32, 1000, 128, 256, (1, 1008)),   # short contexts: no second workgroup ramp
+    (1, 2, 16, 4093, 256, 512, (128, 32)),     # head dim 256: a page per phase at least
     (1, 1, 1, 1, 128, 256, (1, 16)),
     (1, 8, 128, 524288, 128, 256, (256, 2048)),
 ])
