@@ -219,6 +219,8 @@ def unpack_many(blobs, cache, seqs):
         return
     for b in blobs:
         _blob_shape(b)
+        if b.stride(0) != 1:                           # the GPU reads it through its address
+            raise ValueError("a wire blob must be contiguous")
     dev, n = cache.sm.device, len(seqs)
     blobs = [b if b.device == dev else b.to(dev) for b in blobs]
     up = _upload(_host_blobs(blobs), dev)

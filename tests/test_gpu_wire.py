@@ -138,6 +138,13 @@ def test_bad_blobs_raise():
         wire.unpack(blob[:-256].clone() if blob.numel() > 512 else blob[:300].clone(), c, 0)
 
 
+def test_strided_blobs_are_refused():
+    c = _cache(synthetic.make_kv(1, 40, 2, kind="k", seed=1))
+    blob = wire.pack(c, 0)
+    with pytest.raises(ValueError, match="contiguous"):
+        wire.unpack(torch.stack([blob, blob], 1)[:, 0], c, 0)
+
+
 def test_unpack_skips_a_blob_whose_rowmask_disagrees_with_its_header(monkeypatch):
     """The kernel's own check (behind the host's): a blob whose rowmask marks more raw rows
     than its header declares is skipped on the device -- its sequence is not written and
