@@ -62,7 +62,7 @@ class CompressedKV:
         self.T = 0
         self.grows = 0
         self._pending = None                           # page filled by the last append, until checked
-        self._abi = self._ptr_memo = None
+        self._abi = None
         self._open_page()                              # appends may start from an empty cache
 
     # ---------------------------------------------------------------- device-side upkeep
@@ -85,9 +85,8 @@ class CompressedKV:
 
     def _ptrs(self):
         """Addresses of the six arrays, cnt, _before and state."""
-        self._ptr_memo = array_ptrs(self._ptr_memo, (self.sm, self.code, self.base, self.rowmask, self.rowoff, self.raw,
-                                                     self.cnt, self._before, self.state), 3)
-        return self._ptr_memo[1]
+        return array_ptrs((self.sm, self.code, self.base, self.rowmask, self.rowoff, self.raw),
+                          (self.cnt, self._before, self.state))
 
     def _buf(self):
         """The encoder's view (kernels.encode_pages): arrays, counters and sizes."""
@@ -138,14 +137,15 @@ class CompressedKV:
             raise AssertionError(f"{T} prompt tokens do not fit a cache of {self.TS}")
         full = T - T % P
         self.T = T
-        if 0 <= b < self.B and prefill_ready(x, self.sm.device, self.H, self.D):
+        if isinstance(b, int) and 0 <= b < self.B and prefill_ready(x, self.sm.device, self.H, self.D):
             used = prefill_pages(x, self, b=b)
             if full and used > self.cap:
                 strides = (x.stride(0), P * x.stride(1), x.stride(1), x.stride(2))
                 used = self._refit(lambda: (x, strides), b, 0, 1, full // P)
             self._keep_headroom(used)
             return
-        # other sources: an empty prompt, rows of another type or device (less than a page of them)
+        # other sources: an empty prompt, rows of another type or device (less than a page of them), a slot
+        # that is not a plain index
         self.state[0] = T
         used = None
         if full:

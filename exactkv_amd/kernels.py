@@ -16,7 +16,6 @@ split plan), out (output tensor).
 import ctypes
 import functools
 import math
-import operator
 from array import array
 
 import torch
@@ -50,9 +49,10 @@ def plan_splits(B, Hkv, Hq, T, target_blocks=256, min_split=16):
     """MI355X split plan (native): the split count whose rounds of `target_blocks` workgroups
     (one per CU) a cost model finds cheapest -- one round of as many splits as fit it for few
     (sequence, head-block) units, else the fewest rounds that end nearly full -- at least
-    `min_split` tokens per split, split length a multiple of 16. Returns (nsplit, split_len). Short splits cost little: a wavefront's pages follow one
-    another at about one round trip each, so few units are best served by many splits
-    (measured: B1 x 8K 36 -> 18 -> 14.3 us going from 256- to 64- to 32-token splits)."""
+    `min_split` tokens per split, split length a multiple of 16. Returns (nsplit, split_len).
+    Short splits cost little: a wavefront's pages follow one another at about one round trip
+    each, so few units are best served by many splits (measured: B1 x 8K 36 -> 18 -> 14.3 us
+    going from 256- to 64- to 32-token splits)."""
     ns, sl = ctypes.c_int32(), ctypes.c_int32()
     _lib.call("exkv_plan_splits", B, Hkv, Hq, T, target_blocks, min_split, ctypes.byref(ns), ctypes.byref(sl))
     return ns.value, sl.value
@@ -176,7 +176,7 @@ def _cache_args(c):
         raise ValueError("raw pool must have at least one row")
     ptrs = [_lib.ptr(t, what=n) for t, n in zip(args, ("sm", "code", "base", "rowmask", "rowoff", "raw"))]
     res = (*ptrs, raw.shape[0]), TS, H, B
-    if not isinstance(c, dict):
+    if not isinstance(c, dict) and getattr(c, "_abi", None) is args:
         c._abi_memo = (args, res)                      # kernel_args() is rebuilt when the pool grows
     return res
 
@@ -473,6 +473,10 @@ def prefill_pages(x, c, *, b=0, table=None):
 def table_write(lens, block_table, lens_at, lens_val, table_at, table_val):
     """Host ints into a page table on the GPU: lens[lens_at] = lens_val and, row-major,
     block_table[table_at] = table_val (any sequences), in stream order, waiting for nothing."""
+    dev = lens.device.index
+    if dev != torch.cuda.current_device():             # its stream may be the null stream, the current device's
+        with torch.cuda.device(dev):
+            return table_write(lens, block_table, lens_at, lens_val, table_at, table_val)
     at, val = array("i", lens_at), array("i", lens_val)
     n_lens = len(at)
     at.extend(table_at)
@@ -481,13 +485,16 @@ def table_write(lens, block_table, lens_at, lens_val, table_at, table_val):
         raise ValueError("as many values as indices")
     _lib.call("exkv_table_write", _lib.ptr(lens, align=4), lens.numel(), _lib.ptr(block_table, align=4),
               block_table.numel(), at.buffer_info()[0], val.buffer_info()[0], n_lens, len(at),
-              _lib.stream(lens.device.index))
+              _lib.stream(dev))
 
 
 def read_words(words):
     """The values of one-element int32 tensors of one GPU, after the work queued on its current
     stream: one launch and a wait."""
     dev = words[0].device.index
+    if dev != torch.cuda.current_device():
+        with torch.cuda.device(dev):
+            return read_words(words)
     return _lib.fetch(dev, array("Q", [_lib.ptr(w, align=4) for w in words]), _lib.stream(dev))
 
 
@@ -502,13 +509,21 @@ def _paged_append_args(x, table, slots):
             _lib.ptr(bt, what="block_table"), bt.stride(0), n, H, bt.shape[0], bt.shape[1])
 
 
-def array_ptrs(memo, arrays, words):
-    """(arrays, their pointers): `memo` again while it holds the very same tensors, so that a cache
-    checks its buffers once and not in every append. arrays first (16-byte aligned), then words."""
-    if memo is not None and all(map(operator.is_, memo[0], arrays)):
-        return memo
-    n = len(arrays) - words
-    return arrays, tuple(_lib.ptr(t, 16 if i < n else 4) for i, t in enumerate(arrays))
+def array_ptrs(arrays, words):
+    """Addresses of a cache's GPU arrays (16-byte aligned), then of its int32 words, read and checked
+    anew by each call: all at once, and one by one only to say which is at fault."""
+    a, w = [t.data_ptr() for t in arrays], [t.data_ptr() for t in words]
+    low = 0
+    for p in a:
+        low |= p
+    for p in w:
+        low |= p << 2
+    if low & 15 or not all([t.is_cuda for t in arrays]) or not all([t.is_cuda for t in words]):
+        for t in arrays:
+            _lib.ptr(t, 16)
+        for t in words:
+            _lib.ptr(t, 4)
+    return a + w
 
 
 def append_paged(x, buf, table, slots=None):

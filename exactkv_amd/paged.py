@@ -187,20 +187,16 @@ class PagedCompressedKV:
         self._pending = None                                   # pages filled by the last append
         self._appended = 0                                     # table step of the last append
         self.B = 1                                             # the pool, as the attention calls read it
-        self._abi = self._ptr_memo = None
 
     # -- internals
     def kernel_args(self):
-        """(sm, code, base, rowmask, rowoff, raw), as CompressedKV.kernel_args."""
-        if self._abi is None or self._abi[5] is not self.raw:
-            self._abi = (self.sm, self.code, self.base, self.rowmask, self.rowoff, self.raw)
-        return self._abi
+        """(sm, code, base, rowmask, rowoff, raw) for the attention and decode kernels."""
+        return self.sm, self.code, self.base, self.rowmask, self.rowoff, self.raw
 
     def _ptrs(self):
         """Addresses of the six arrays, cnt, _before and _arrivals."""
-        self._ptr_memo = array_ptrs(self._ptr_memo, (self.sm, self.code, self.base, self.rowmask, self.rowoff, self.raw,
-                                                     self.cnt, self._before, self._arrivals), 3)
-        return self._ptr_memo[1]
+        return array_ptrs((self.sm, self.code, self.base, self.rowmask, self.rowoff, self.raw),
+                          (self.cnt, self._before, self._arrivals))
 
     def _tail(self, slot):
         """bf16 [H, 16, D] view of a slot's open page (its rows behind cap)."""
@@ -257,7 +253,8 @@ class PagedCompressedKV:
         Tf = T // P * P
         t = self.table
         dst = t.block_table[slot: slot + 1]
-        if prefill_ready(x, self.sm.device, self.H, self.D) and t.block_table.stride(0) == t.max_pages:
+        if (isinstance(slot, int) and 0 <= slot < t.max_seqs and prefill_ready(x, self.sm.device, self.H, self.D)
+                and t.block_table.stride(0) == t.max_pages):
             n = prefill_pages(x, self, b=slot, table=t)
             if Tf and n > self.cap:
                 st = (x.stride(0), P * x.stride(1), x.stride(1), x.stride(2))

@@ -167,3 +167,50 @@ def test_prefill_in_one_call_equals_its_parts(T, H, D, kind, reserve, paged, mon
     half = len(got) // 2
     for a, b in zip(sum(got[:half], ()), sum(got[half:], ())):
         assert torch.equal(a, b) if isinstance(a, torch.Tensor) else a == b
+
+
+def test_appends_follow_moved_buffers():
+    """Every append and prefill reads the addresses of the cache's arrays anew: storage that moves
+    under the same tensor objects is written where it is now."""
+    g = torch.Generator().manual_seed(3)
+    B, H, D, T0 = 2, 4, 128, 20
+    x = _make(g, B, 64, H, D, 0.1).to(DEV)
+    a, c = exactkv.CompressedKV(B, 64, H, D, reserve=0.6), exactkv.CompressedKV(B, 64, H, D, reserve=0.6)
+    for k in (a, c):
+        for b in range(B):
+            k.prefill_slot(b, x[b:b + 1, :T0].contiguous())
+        k.append(x[:, T0].contiguous())
+    old = {n: getattr(c, n).data for n in ("sm", "code", "base", "rowmask", "rowoff", "raw", "cnt", "state")}
+    was = {n: t.clone() for n, t in old.items()}
+    for n in old:
+        getattr(c, n).data = old[n].clone()
+    for t in range(T0 + 1, 40):
+        for k in (a, c):
+            k.append(x[:, t].contiguous())
+        exactkv.check_overflow([a, c])
+    for n in old:
+        assert torch.equal(getattr(a, n), getattr(c, n)), n
+        assert torch.equal(old[n], was[n]), n
+
+
+@pytest.mark.parametrize("T", [7, 40])
+def test_prefill_takes_any_index_type(T):
+    """Slots as Python ints, numpy ints and one-element tensors alike."""
+    g = torch.Generator().manual_seed(4)
+    x = _make(g, 3, T, 2, 128, 0.1).to(DEV)
+    a, c = exactkv.CompressedKV(3, 64, 2, 128, reserve=0.6), exactkv.CompressedKV(3, 64, 2, 128, reserve=0.6)
+    for b, same in enumerate((0, np.int64(1), torch.tensor(2))):
+        a.prefill_slot(b, x[b:b + 1])
+        c.prefill_slot(same, x[b:b + 1])
+    for n in ("sm", "code", "base", "rowmask", "rowoff", "raw", "cnt", "state"):
+        assert torch.equal(getattr(a, n), getattr(c, n)), n
+
+
+def test_misaligned_cache_arrays_are_refused():
+    """array_ptrs names what is at fault: an array off 16 bytes, a word off 4, a tensor not on the GPU."""
+    buf = torch.zeros(64, dtype=torch.uint8, device=DEV)
+    word = torch.zeros(1, dtype=torch.int32, device=DEV)
+    assert kernels.array_ptrs((buf, buf[16:]), (word,)) == [buf.data_ptr(), buf.data_ptr() + 16, word.data_ptr()]
+    for arrays, words in (((buf[8:],), (word,)), ((buf,), (buf[2:],)), ((buf.cpu(),), (word,))):
+        with pytest.raises(ValueError):
+            kernels.array_ptrs(arrays, words)
