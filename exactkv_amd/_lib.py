@@ -26,9 +26,9 @@ SIGNATURES = {
     "exkv_store_raw_rows": [_p, _i64, _i64, _i64, _i64, _p, _p, _p, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32,
                             _i32, _i32, _p],
     "exkv_prefill_slot": [_p, _i64, _i64, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _i32, _i32,
-                          _i32, _i32, _p, _i64, _p],
-    "exkv_prefill_slot_paged": [_p, _i64, _i64, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _p, _i32, _i32,
-                                _i32, _i32, _i32, _i32, _p, _i64, _p],
+                          _i32, _i32, _p, _i64, _p, _i32, _p],
+    "exkv_prefill_slot_paged": [_p, _i64, _i64, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _p, _i32, _i32,
+                                _i32, _i32, _i32, _i32, _p, _i64, _p, _i32, _p],
     "exkv_cache_append": [_p, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i32, _i32, _i32,
                           _i32, _p],
     "exkv_bf16_append": [_p, _i64, _i64, _p, _p, _i32, _i32, _i32, _i32, _p],
@@ -202,12 +202,18 @@ def host_words(index, n):
     return b
 
 
+def tagged_words(index, n):
+    """host_words with a new tag, which word 0 does not hold."""
+    w = host_words(index, n)
+    w.tag = w.tag % 0x3FFFFFFF + 1
+    return w
+
+
 def fetch(index, ptrs, st):
     """Wait for the work queued on raw stream `st` of device `index`; the int32 words at the device
     addresses `ptrs` (an array('Q')), as a list."""
     n = len(ptrs)
-    w = host_words(index, n + 1)
-    w.tag = w.tag % 0x3FFFFFFF + 1
+    w = tagged_words(index, n + 1)
     call("exkv_fetch_words", ptrs.buffer_info()[0], n, w.addr, w.tag, st)
     return w.view[1:n + 1]
 

@@ -117,6 +117,8 @@ __device__ inline int block_excl_scan(int v, int& total) {
 namespace exkv {
 void set_error(const char* fmt, ...);
 int hip_status(hipError_t e, const char* where);
+// Wait until a kernel on `stream` has stored `tag` in the mapped host word *host (table.hip).
+int wait_for_tag(const char* what, const int32_t* host, int32_t tag, hipStream_t stream);
 // Launch the fetch of one source file's sticky error word (errors.hpp) on `stream`.
 hipError_t fetch_errors_attention(uint32_t* out, int first, int clear, hipStream_t stream);
 hipError_t fetch_errors_encode(uint32_t* out, int first, int clear, hipStream_t stream);

@@ -575,7 +575,15 @@ struct PrefillEnd {
     int open_pages = 0;               // pages per sequence: none is opened at or past it
     const int32_t* table = nullptr;   // paged: the slot's block-table row; its page T / 16 is opened
     int64_t pool_pages = 0;
+    int32_t* host = nullptr;          // mapped host memory: the counter to host[1], then tag to host[0]
+    int32_t tag = 0;
+    int32_t* arrivals = nullptr;      // with host: the scan's blocks count in here (zero between calls)
 };
+
+// A word to mapped host memory, past the caches: complete at this wave's next vmcnt(0).
+__device__ inline void to_host(int32_t* p, int32_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // One block of 1,024 threads.
 template <int D>
@@ -616,6 +624,41 @@ __device__ inline void prefill_end(const EncArgs& a, const PrefillEnd& e) {
 template <int D>
 __global__ void __launch_bounds__(1024) prefill_end_kernel(EncArgs a, PrefillEnd e) {
     prefill_end<D>(a, e);
+    if (e.host == nullptr) return;                     // uniform
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        to_host(e.host + 1, *a.cnt);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        to_host(e.host, e.tag);
+    }
+}
+
+// Count this block in on *arrivals (zero between calls): true for the last of the grid's. Every
+// thread calls it; a wave's loads and stores are complete first (stores: it waits for them).
+__device__ inline bool last_block(int32_t* arrivals, bool stores) {
+    __shared__ int s_last;
+    if (stores) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int old = __hip_atomic_fetch_add(arrivals, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = old == (int)gridDim.x - 1;
+    }
+    __syncthreads();
+    return s_last != 0;
+}
+
+// The last block to arrive, after the block with the counter's value has stored it and every
+// block has read its rows, tells the host, which waits for that: a launch of its own for it took
+// 1 us more of a prefill at every size (one cache, with its counter's fill: 2,045 units 28.4 ->
+// 27.2 us, 8,190 35.7 -> 34.7, 32,760 in 257 blocks 63.2 -> 62.5).
+__device__ inline void tell_host(const PrefillEnd& e) {
+    if (e.host == nullptr) return;                     // uniform
+    if (last_block(e.arrivals, true) && threadIdx.x == 0) {
+        __hip_atomic_store(e.arrivals, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        to_host(e.host, e.tag);
+    }
 }
 
 // nscan blocks of ub units; END: one more, which does a prefill's end beside them.
@@ -623,6 +666,7 @@ template <bool PAGED, bool VEC16, bool END, int D>
 __global__ void __launch_bounds__(1024) scan_direct_kernel(EncArgs a, int nunits, int ub, int nscan, PrefillEnd e) {
     if (END && (int)blockIdx.x == nscan) {
         prefill_end<D>(a, e);
+        tell_host(e);
         return;
     }
     __shared__ int s_before[16], s_own[16];
@@ -654,9 +698,13 @@ __global__ void __launch_bounds__(1024) scan_direct_kernel(EncArgs a, int nunits
     if (mine) a.rowoff[page] = off;
     if (threadIdx.x == 0) {
         if (blockIdx.x == 0 && a.before != nullptr) *a.before = cnt0;
-        if ((int)blockIdx.x == nscan - 1) *a.cnt = cnt0 + total;
+        if ((int)blockIdx.x == nscan - 1) {
+            *a.cnt = cnt0 + total;
+            if (END && e.host != nullptr) to_host(e.host + 1, cnt0 + total);
+        }
     }
     if (a.cap > 0) copy_escaped_rows<VEC16, D>(a, m, off, a.src + bi * a.s_b + pg * a.s_pg + hk * a.s_h, lane);
+    if (END) tell_host(e);
 }
 
 template <int D, bool END>
@@ -916,20 +964,6 @@ __device__ inline void write_rows(const Units& units, int n, int tid, int nthrea
             if (i < total && tok[k] >= 0) st_words<E / 2>(units.tail(u) + tok[k] % kPage * D + i % CH * E, v[k]);
         }
     }
-}
-
-// Count this block in on *arrivals (zero between calls): true for the last of the grid's. Every
-// thread calls it; a wave's stores are complete first (stores: it waits for them).
-__device__ inline bool last_block(int32_t* arrivals, bool stores) {
-    __shared__ int s_last;
-    if (stores) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int old = __hip_atomic_fetch_add(arrivals, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = old == (int)gridDim.x - 1;
-    }
-    __syncthreads();
-    return s_last != 0;
 }
 
 // Units of a contiguous cache's append at token T (-1: a full cache): every page fills at once
@@ -1410,8 +1444,8 @@ extern "C" int exkv_encode_pages_paged(const void* src, int64_t s_b, int64_t s_p
 // exkv_encode_pages encodes them, its last rows into the slot's open page, page T / 16 of every
 // sequence opened (exkv_cache_open_page), state[0] = T.
 static int prefill_slot(const char* what, EncArgs& a, PrefillEnd& e, int64_t s_t, int64_t s_h, int32_t T, int64_t slot,
-                        int64_t slots, int64_t raw_rows, int32_t D, void* scan_ws, int64_t scan_ws_words,
-                        hipStream_t stream) {
+                        int64_t slots, int64_t raw_rows, int32_t D, void* scan_ws, int64_t scan_ws_words, int32_t* host,
+                        int32_t tag, int32_t* arrivals, hipStream_t stream) {
     const int64_t tail_end = a.cap + slots * a.H * kPage;
     EXKV_REQUIRE(a.cap >= 0 && tail_end <= raw_rows && tail_end <= INT32_MAX,
                  "%s: raw pool (%lld rows) smaller than cap + open-page rows", what, (long long)raw_rows);
@@ -1423,7 +1457,17 @@ static int prefill_slot(const char* what, EncArgs& a, PrefillEnd& e, int64_t s_t
                  "%s: source rows must start at even elements (4-byte aligned)", what);
     EXKV_REQUIRE(n <= INT32_MAX - 1024, "%s: %lld pages x heads in one call (limit 2^31 - 1025)", what, (long long)n);
     EXKV_REQUIRE(scan_ws == nullptr || (uintptr_t)scan_ws % 8 == 0, "%s: scan workspace must be 8-byte aligned", what);
+    if (host != nullptr) {
+        EXKV_REQUIRE(arrivals, "%s: null pointer", what);
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        const hipError_t st = hipStreamIsCapturing(stream, &capturing);
+        if (st != hipSuccess) return hip_status(st, what);
+        EXKV_REQUIRE(capturing == hipStreamCaptureStatusNone, "%s: the stream is being captured", what);
+    }
     a.D = D;
+    e.host = host;
+    e.tag = tag;
+    e.arrivals = arrivals;
     e.tail = a.src + (int64_t)a.npg * kPage * s_t;
     e.s_t = s_t;
     e.s_h = s_h;
@@ -1431,13 +1475,15 @@ static int prefill_slot(const char* what, EncArgs& a, PrefillEnd& e, int64_t s_t
     e.tail0 = a.cap + slot * a.H * kPage;
     e.T = T;
     launch_encode(a, n, (uint64_t*)scan_ws, scan_ws_words, &e, stream);
-    return launch_status(what);
+    const int rc = launch_status(what);
+    return rc != EXKV_OK || host == nullptr ? rc : wait_for_tag(what, host, tag, stream);
 }
 
 extern "C" int exkv_prefill_slot(const void* src, int64_t s_t, int64_t s_h, int32_t T, void* sm, void* code, void* base,
                                  int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before,
                                  int32_t* state, int64_t cap, int64_t raw_rows, int32_t B, int32_t b, int32_t H,
-                                 int32_t TS, int32_t D, void* scan_ws, int64_t scan_ws_words, hipStream_t stream) {
+                                 int32_t TS, int32_t D, void* scan_ws, int64_t scan_ws_words, int32_t* host,
+                                 int32_t tag, hipStream_t stream) {
     EXKV_REQUIRE(head_dim_ok(D), "prefill_slot: head dim must be 64, 128 or 256 (got %d)", D);
     EXKV_REQUIRE(TS > 0 && TS % kPage == 0 && B > 0 && H > 0, "prefill_slot: bad shape B=%d H=%d TS=%d", B, H, TS);
     EXKV_REQUIRE(b >= 0 && b < B && T >= 0 && T <= TS, "prefill_slot: %d tokens into slot %d outside the cache", T, b);
@@ -1448,16 +1494,18 @@ extern "C" int exkv_prefill_slot(const void* src, int64_t s_t, int64_t s_h, int3
     e.state = state;
     e.B = B;
     e.open_pages = TS / kPage;
-    return prefill_slot("prefill_slot", a, e, s_t, s_h, T, b, B, raw_rows, D, scan_ws, scan_ws_words, stream);
+    return prefill_slot("prefill_slot", a, e, s_t, s_h, T, b, B, raw_rows, D, scan_ws, scan_ws_words, host, tag, state + 1,
+                        stream);
 }
 
 // The same into slot `slot` of a paged cache: its page p is pool page table[p] (entries clamped
 // to the pool), and page T / 16 is opened where the table has it.
 extern "C" int exkv_prefill_slot_paged(const void* src, int64_t s_t, int64_t s_h, int32_t T, void* sm, void* code,
                                        void* base, int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt,
-                                       int32_t* before, int64_t cap, int64_t raw_rows, const int32_t* table,
-                                       int32_t slot, int32_t max_seqs, int32_t max_pages, int32_t pool_pages, int32_t H,
-                                       int32_t D, void* scan_ws, int64_t scan_ws_words, hipStream_t stream) {
+                                       int32_t* before, int32_t* arrivals, int64_t cap, int64_t raw_rows,
+                                       const int32_t* table, int32_t slot, int32_t max_seqs, int32_t max_pages,
+                                       int32_t pool_pages, int32_t H, int32_t D, void* scan_ws, int64_t scan_ws_words,
+                                       int32_t* host, int32_t tag, hipStream_t stream) {
     EXKV_REQUIRE(head_dim_ok(D), "prefill_slot_paged: head dim must be 64, 128 or 256 (got %d)", D);
     EXKV_REQUIRE(H > 0 && max_seqs > 0 && max_pages > 0 && pool_pages > 0, "prefill_slot_paged: bad shape");
     EXKV_REQUIRE(slot >= 0 && slot < max_seqs && T >= 0 && T <= (int64_t)max_pages * kPage,
@@ -1472,8 +1520,8 @@ extern "C" int exkv_prefill_slot_paged(const void* src, int64_t s_t, int64_t s_h
     e.open_pages = max_pages;
     e.table = table;
     e.pool_pages = pool_pages;
-    return prefill_slot("prefill_slot_paged", a, e, s_t, s_h, T, slot, max_seqs, raw_rows, D, scan_ws, scan_ws_words,
-                        stream);
+    return prefill_slot("prefill_slot_paged", a, e, s_t, s_h, T, slot, max_seqs, raw_rows, D, scan_ws, scan_ws_words, host,
+                        tag, arrivals, stream);
 }
 
 extern "C" int exkv_cache_append(const void* x, int64_t sx_b, int64_t sx_h, void* sm, void* code, void* base,

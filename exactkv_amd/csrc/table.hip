@@ -93,6 +93,10 @@ extern "C" int exkv_fetch_words(const int32_t* const* words, int32_t n, int32_t*
     } while (i0 < n);
     e = hipGetLastError();
     if (e != hipSuccess) return hip_status(e, "fetch_words");
+    return wait_for_tag("fetch_words", host, tag, stream);
+}
+
+int exkv::wait_for_tag(const char* what, const int32_t* host, int32_t tag, hipStream_t stream) {
     const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(kPollUs);
     do {
         for (int k = 0; k < 64; ++k) {
@@ -100,8 +104,8 @@ extern "C" int exkv_fetch_words(const int32_t* const* words, int32_t n, int32_t*
             __builtin_ia32_pause();
         }
     } while (std::chrono::steady_clock::now() < end);
-    e = hipStreamSynchronize(stream);
-    if (e != hipSuccess) return hip_status(e, "fetch_words");
-    EXKV_REQUIRE(__atomic_load_n(host, __ATOMIC_ACQUIRE) == tag, "fetch_words: no answer from the GPU");
+    const hipError_t e = hipStreamSynchronize(stream);
+    if (e != hipSuccess) return hip_status(e, what);
+    EXKV_REQUIRE(__atomic_load_n(host, __ATOMIC_ACQUIRE) == tag, "%s: no answer from the GPU", what);
     return EXKV_OK;
 }

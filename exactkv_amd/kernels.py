@@ -449,7 +449,7 @@ def prefill_pages(x, c, *, b=0, table=None):
     """Prompt x [1, T, H, D] (prefill_ready) into slot b of a cache, all of a prefill's device work in
     two launches: full pages encoded, the rest into the open-page rows, that page opened, the
     token count set. c: a CompressedKV, or a PagedCompressedKV with its PageTable. Waits for the
-    stream and returns the raw-row counter, which passes cap when the pool overflowed, as after
+    counter and returns it, which passes cap when the pool overflowed, as after
     encode_pages."""
     H, D, T = c.H, c.D, x.shape[1]
     s_t, s_h = x.stride(1), x.stride(2)
@@ -458,16 +458,16 @@ def prefill_pages(x, c, *, b=0, table=None):
     ptrs = c._ptrs()
     units = (T // P) * H
     ws = _scan_ws(c.raw.device, units) if units > DIRECT_UNITS else None
-    st = _lib.stream()
-    scan = (_lib.ptr(ws), ws.numel() if ws is not None else 0, st)
+    w = _lib.tagged_words(c.raw.device.index, 2)
+    scan = (_lib.ptr(ws), ws.numel() if ws is not None else 0, w.addr, w.tag, _lib.stream())
     if table is None:
         _lib.call("exkv_prefill_slot", _lib.ptr(x, 2, "x"), s_t, s_h, T, *ptrs, c.cap, c.raw.shape[0], c.B, b, H, c.TS, D,
                   *scan)
     else:
         row = table.block_table.data_ptr() + 4 * b * table.max_pages
-        _lib.call("exkv_prefill_slot_paged", _lib.ptr(x, 2, "x"), s_t, s_h, T, *ptrs[:8], c.cap, c.raw.shape[0], row, b,
+        _lib.call("exkv_prefill_slot_paged", _lib.ptr(x, 2, "x"), s_t, s_h, T, *ptrs, c.cap, c.raw.shape[0], row, b,
                   table.max_seqs, table.max_pages, table.num_pages, H, D, *scan)
-    return _lib.fetch(c.raw.device.index, array("Q", ptrs[6:7]), st)[0]
+    return w.view[1]
 
 
 def table_write(lens, block_table, lens_at, lens_val, table_at, table_val):

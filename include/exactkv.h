@@ -102,20 +102,24 @@ int exkv_store_raw_rows(const void* src, int64_t s_b, int64_t s_pg, int64_t s_p,
  * exkv_encode_pages; the other rows go to the slot's open-page rows, raw rows
  * cap + (b*H + h)*16 on; page T / 16 of every sequence is opened as by exkv_cache_open_page;
  * and state[0] = T. Two launches up to 65,536 pages x heads. Overflow shows in *cnt, as for
- * exkv_encode_pages.
+ * exkv_encode_pages. host (may be NULL): two words of mapped host memory; the call then waits,
+ * on a stream that is not being captured, until *cnt is in host[1] and `tag`, which host[0] must not
+ * hold before, in host[0], by when src's full pages have been read. state[1] is zero between
+ * calls.
  * Replaces: cache.py:87-98 (encode, open-page copy). */
 int exkv_prefill_slot(const void* src, int64_t s_t, int64_t s_h, int32_t T, void* sm, void* code, void* base,
                       int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before, int32_t* state,
                       int64_t cap, int64_t raw_rows, int32_t B, int32_t b, int32_t H, int32_t TS, int32_t D,
-                      void* scan_ws, int64_t scan_ws_words, hipStream_t stream);
+                      void* scan_ws, int64_t scan_ws_words, int32_t* host, int32_t tag, hipStream_t stream);
 
 /* The same into slot `slot` of a paged cache whose page p is pool page table[p] (max_pages
- * entries, clamped to the pool); page T / 16 of the slot is opened where the table has it. */
+ * entries, clamped to the pool); page T / 16 of the slot is opened where the table has it.
+ * arrivals: a word that is zero between calls (with host). */
 int exkv_prefill_slot_paged(const void* src, int64_t s_t, int64_t s_h, int32_t T, void* sm, void* code, void* base,
-                            int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before, int64_t cap,
-                            int64_t raw_rows, const int32_t* table, int32_t slot, int32_t max_seqs,
-                            int32_t max_pages, int32_t pool_pages, int32_t H, int32_t D, void* scan_ws,
-                            int64_t scan_ws_words, hipStream_t stream);
+                            int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before,
+                            int32_t* arrivals, int64_t cap, int64_t raw_rows, const int32_t* table, int32_t slot,
+                            int32_t max_seqs, int32_t max_pages, int32_t pool_pages, int32_t H, int32_t D,
+                            void* scan_ws, int64_t scan_ws_words, int32_t* host, int32_t tag, hipStream_t stream);
 
 /* The page encoder into a paged cache: page pg of source sequence bi goes to page
  * dst_pages[bi*dst_stride + pg] of the B x TS arrays read as a list of B*TS/16 pages (entries

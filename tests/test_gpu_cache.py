@@ -214,3 +214,28 @@ def test_misaligned_cache_arrays_are_refused():
     for arrays, words in (((buf[8:],), (word,)), ((buf,), (buf[2:],)), ((buf.cpu(),), (word,))):
         with pytest.raises(ValueError):
             kernels.array_ptrs(arrays, words)
+
+
+@pytest.mark.parametrize("T,H", [(1, 8), (15, 2), (16, 1), (1040, 1), (1040, 8), (65536, 16), (32769, 33)])
+@pytest.mark.parametrize("paged", [False, True])
+def test_prefill_returns_the_counter(T, H, paged):
+    """The counter that a prefill's last block (without full pages, or above 65,536 units, its last
+    launch) gives the host, call after call: one block, several, 257 and a launch of its own."""
+    from exactkv_amd import kernels as k
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x = (1 + torch.rand(1, T, H, 64, generator=g, device=DEV)).bfloat16()        # no raw rows by chance
+    raw = torch.rand(T, H, generator=g, device=DEV) < 0.02
+    x[0, raw, 9] = 1e-30
+    full = T - T % 16
+    n = int(raw[:full].sum())
+    pages = -(-(T + 1) // 16)
+    if paged:
+        table = exactkv.PageTable(pages, 1, pages)
+        table.add(T)
+        c = exactkv.PagedCompressedKV(table, H, D=64, reserve=0.2)
+    else:
+        table, c = None, exactkv.CompressedKV(1, 16 * pages, H, 64, reserve=0.2)
+    word = c._arrivals[0] if paged else c.state[1]
+    for i in range(1, 4):
+        assert k.prefill_pages(x, c, table=table) == i * n == int(c.cnt.item())
+        assert int(word.item()) == 0
