@@ -162,6 +162,9 @@ def pack_many(cache, seqs):
     if not seqs:
         return []
     H, dev = cache.H, cache.sm.device
+    if dev.index != torch.cuda.current_device():       # uploads and launches on one stream, the cache's GPU's
+        with torch.cuda.device(dev):
+            return pack_many(cache, seqs)
     infos = [_sequence(cache, s) for s in seqs]
     host, n = _host_pages(cache, infos), len(seqs)
     d, width = _upload(host, dev), host["pages"].shape[1]
@@ -217,11 +220,14 @@ def unpack_many(blobs, cache, seqs):
         raise ValueError("one distinct sequence per blob")
     if not seqs:
         return
+    dev, n = cache.sm.device, len(seqs)
+    if dev.index != torch.cuda.current_device():       # uploads and launches on one stream, the cache's GPU's
+        with torch.cuda.device(dev):
+            return unpack_many(blobs, cache, seqs)
     for b in blobs:
         _blob_shape(b)
         if b.stride(0) != 1:                           # the GPU reads it through its address
             raise ValueError("a wire blob must be contiguous")
-    dev, n = cache.sm.device, len(seqs)
     blobs = [b if b.device == dev else b.to(dev) for b in blobs]
     up = _upload(_host_blobs(blobs), dev)
     st = _lib.stream()
