@@ -226,7 +226,9 @@ def unpack_many(blobs, cache, seqs):
             return unpack_many(blobs, cache, seqs)
     for b in blobs:
         _blob_shape(b)
-        if b.stride(0) != 1:                           # the GPU reads it through its address
+        # the GPU reads a blob through its address; one that is copied there first comes out dense, and
+        # has been taken strided where it holds no whole page, whose masks need dense words
+        if b.stride(0) != 1 and (b.device == dev or header(b)["full_pages"]):
             raise ValueError("a wire blob must be contiguous")
     blobs = [b if b.device == dev else b.to(dev) for b in blobs]
     up = _upload(_host_blobs(blobs), dev)

@@ -145,6 +145,21 @@ def test_strided_blobs_are_refused():
         wire.unpack(torch.stack([blob, blob], 1)[:, 0], c, 0)
 
 
+@pytest.mark.parametrize("T", [11, 40])
+def test_strided_blobs_in_host_memory(T):
+    """Taken where they hold no whole page, refused where they do."""
+    x = synthetic.make_kv(1, T, 2, kind="k", seed=1)
+    host = wire.pack(_cache(x), 0).cpu()
+    blob = torch.stack([host, torch.zeros_like(host)], 1)[:, 0]
+    dst = exactkv.CompressedKV(1, 64, 2, 128)
+    if T >= P:
+        with pytest.raises(ValueError, match="contiguous"):
+            wire.unpack(blob, dst, 0)
+        return
+    wire.unpack(blob, dst, 0)
+    assert dst.T == T and same_bits(kernels.decode_to_bf16(dst.buffers(), T), x.to(DEV))
+
+
 def test_unpack_skips_a_blob_whose_rowmask_disagrees_with_its_header(monkeypatch):
     """The kernel's own check (behind the host's): a blob whose rowmask marks more raw rows
     than its header declares is skipped on the device -- its sequence is not written and
