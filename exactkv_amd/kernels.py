@@ -16,6 +16,7 @@ split plan), out (output tensor).
 import ctypes
 import functools
 import math
+import operator
 from array import array
 
 import torch
@@ -198,7 +199,7 @@ def _plan(B, Hkv, Hq, T, TS, lens, nsplit, split_len, window=0, D=128):
     reach = TS if lens is not None else T
     if window:                                 # the splits start at the window's first page
         reach = min(reach, window + P - 1)
-    return _default_plan(B, Hkv, Hq, reach, D)
+    return _default_plan(B, Hkv, Hq, operator.index(reach), D)   # T may be a tensor: its value, not the object
 
 
 def _window_arg(window):

@@ -141,6 +141,18 @@ def test_plan_rounds(B, Hkv, Hq, T, D, slots, expect):
     assert B * Hq * ns * (D + 2) * 4 <= _lib.load().exkv_noalloc_scratch_bytes()
 
 
+def test_default_plans_follow_the_value_of_a_tensor():
+    """A token count in a tensor that a program advances in place: each call plans for its value."""
+    import torch
+    from exactkv_amd.kernels import _plan, plan_splits
+    T = torch.tensor(100)
+    for n in (100, 1000, 4000):
+        T.fill_(n)
+        assert _plan(1, 8, 32, T, 4096, None, None, None) == plan_splits(1, 8, 32, n)
+    with pytest.raises(TypeError):
+        _plan(1, 8, 32, 4000.0, 4096, None, None, None)
+
+
 def test_rebuild_bitmath_exhaustive(tmp_path):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
