@@ -440,10 +440,11 @@ def encode_pages_paged(src, strides, buf, dst_pages, nb, npg, *, chained=True):
 
 def prefill_ready(x, dev, H, D):
     """Whether prompt x [1, T, H, D] can go through prefill_pages as it stands: bf16 rows on the
-    cache's GPU, T > 0, and of the cache's shape where a part of a page is left over."""
+    cache's GPU, T > 0, and of the cache's shape where a part of a page is left over, whose rows
+    nothing else checks."""
     T = x.shape[1] if x.dim() == 4 else 0
     return (T > 0 and x.dtype == torch.bfloat16 and x.device == dev and x.stride(3) == 1
-            and (T % P == 0 or (x.shape[2] == H and x.shape[3] == D)))
+            and (T % P == 0 or (x.shape[0] > 0 and x.shape[2] == H and x.shape[3] == D)))
 
 
 def prefill_pages(x, c, *, b=0, table=None):

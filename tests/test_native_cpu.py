@@ -153,6 +153,20 @@ def test_default_plans_follow_the_value_of_a_tensor():
         _plan(1, 8, 32, 4000.0, 4096, None, None, None)
 
 
+@pytest.mark.parametrize("shape,ready", [
+    ((1, 5, 2, 128), True), ((1, 37, 2, 128), True), ((2, 37, 2, 128), True), ((1, 32, 2, 128), True),
+    ((0, 5, 2, 128), False), ((0, 37, 2, 128), False),     # no prompt: its rows lie outside the tensor
+    ((1, 37, 1, 128), False), ((1, 37, 2, 64), False), ((1, 0, 2, 128), False), ((5, 2, 128), False),
+])
+def test_prompts_that_a_prefill_reads_by_address(shape, ready):
+    import torch
+    from exactkv_amd.kernels import prefill_ready
+    x = torch.zeros(3, 40, 2, 128, dtype=torch.bfloat16)
+    x = x[:shape[0], :shape[1], :shape[2], :shape[3]] if len(shape) == 4 else x[0]
+    assert prefill_ready(x, x.device, 2, 128) == ready
+    assert not prefill_ready(x.float(), x.device, 2, 128)
+
+
 def test_rebuild_bitmath_exhaustive(tmp_path):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
