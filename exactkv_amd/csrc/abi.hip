@@ -99,6 +99,13 @@ static void plan_core(int64_t units, int32_t T, int64_t slots, int32_t min_split
     const int64_t pages = ((int64_t)T + exkv::kPage - 1) / exkv::kPage;
     const int64_t cap = std::max<int64_t>(1, ((int64_t)T + min_split - 1) / min_split);
     const int64_t first = (units + slots - 1) / slots;
+    // no split is shorter than min_split (or all of T): ceil(T / cap) may be
+    const int64_t least = std::min(pages, ((int64_t)min_split + exkv::kPage - 1) / exkv::kPage) * exkv::kPage;
+    const auto plan = [&](int64_t sl) {
+        sl = std::max(sl, least);
+        *split_len = (int32_t)sl;
+        *nsplit = (int32_t)(((int64_t)T + sl - 1) / sl);
+    };
     int64_t ns = 1;
     double cost = 0.0;
     for (int64_t r = first; r < first + 8; ++r) {
@@ -114,13 +121,11 @@ static void plan_core(int64_t units, int32_t T, int64_t slots, int32_t min_split
         const int64_t n = std::min(full_rounds(units, slots), cap);
         if (plan_cost(units, n, pages, slots, nph, ramp) <= cost * 17.0 / 16.0) {
             const int64_t sl = ((int64_t)T + n - 1) / n;
-            *split_len = (int32_t)(sl <= exkv::kPage ? exkv::kPage : (sl + 31) / 32 * 32);
-            *nsplit = (int32_t)(((int64_t)T + *split_len - 1) / *split_len);
+            plan(sl <= exkv::kPage ? exkv::kPage : (sl + 31) / 32 * 32);
             return;
         }
     }
-    *split_len = (int32_t)((pages + ns - 1) / ns * exkv::kPage);
-    *nsplit = (int32_t)(((int64_t)T + *split_len - 1) / *split_len);
+    plan((pages + ns - 1) / ns * exkv::kPage);
 }
 
 // KV heads (or pairs of them) per workgroup: min(gcd(n, 8), 4)

@@ -167,6 +167,15 @@ def test_prompts_that_a_prefill_reads_by_address(shape, ready):
     assert not prefill_ready(x.float(), x.device, 2, 128)
 
 
+@pytest.mark.parametrize("min_split", [1, 16, 48, 64, 100, 250])
+@pytest.mark.parametrize("B,Hkv,Hq", [(1, 8, 32), (7, 4, 28), (300, 8, 32)])
+def test_no_split_is_shorter_than_the_least(B, Hkv, Hq, min_split):
+    from exactkv_amd.kernels import plan_splits
+    for T in (1, 15, 16, 65, 130, 250, 997, 1000, 4093):
+        ns, sl = plan_splits(B, Hkv, Hq, T, 256, min_split)
+        assert sl >= min(min_split, T) and sl % 16 == 0 and ns * sl >= T and (ns - 1) * sl < T, (T, ns, sl)
+
+
 def test_rebuild_bitmath_exhaustive(tmp_path):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
