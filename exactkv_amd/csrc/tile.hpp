@@ -109,10 +109,13 @@ struct Run {
     static constexpr int V = D / 8;        // dwords of values per lane (two runs)
 };
 
-// n dwords from p (8- or 16-byte aligned for n = 2, n >= 4)
+// n dwords from p (4-, 8- or 16-byte aligned for n = 1, 2, n >= 4)
 template <int N>
 __device__ inline void ld_words(const void* p, uint32_t* out) {
-    if constexpr (N == 2) {
+    static_assert(N == 1 || N == 2 || (N > 0 && N % 4 == 0), "one, two or whole fours of dwords");
+    if constexpr (N == 1) {
+        out[0] = *reinterpret_cast<const uint32_t*>(p);
+    } else if constexpr (N == 2) {
         const uint2 v = *reinterpret_cast<const uint2*>(p);
         out[0] = v.x; out[1] = v.y;
     } else {
@@ -125,7 +128,10 @@ __device__ inline void ld_words(const void* p, uint32_t* out) {
 }
 template <int N>
 __device__ inline void st_words(void* p, const uint32_t* in) {
-    if constexpr (N == 2) {
+    static_assert(N == 1 || N == 2 || (N > 0 && N % 4 == 0), "one, two or whole fours of dwords");
+    if constexpr (N == 1) {
+        *reinterpret_cast<uint32_t*>(p) = in[0];
+    } else if constexpr (N == 2) {
         *reinterpret_cast<uint2*>(p) = make_uint2(in[0], in[1]);
     } else {
 #pragma unroll

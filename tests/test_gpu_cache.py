@@ -206,6 +206,35 @@ def test_prefill_takes_any_index_type(T):
         assert torch.equal(getattr(a, n), getattr(c, n)), n
 
 
+@pytest.mark.parametrize("B,H,D", [(1, 1, 64), (2, 8, 128), (9, 8, 128), (3, 5, 256), (300, 4, 64)])
+@pytest.mark.parametrize("offset,pitch", [(0, 0), (2, 0), (0, 2), (4, 4), (0, 6)])
+@pytest.mark.parametrize("paged", [False, True])
+def test_append_row_alignment(B, H, D, offset, pitch, paged):
+    """Token rows inside wider ones, 16-, 8- and 4-byte aligned, one block of units and more: after
+    every append the cache decodes to the tokens given so far."""
+    g = torch.Generator(device=DEV).manual_seed(B + D + offset)
+    T0, N = 10, 9                                          # appends before, at and after a page end
+    x = torch.randn(B, T0 + N, H, D, generator=g, device=DEV).bfloat16()
+    x[torch.rand(B, T0 + N, H, generator=g, device=DEV) < 0.1, 5] *= 2.0 ** -30
+    if paged:
+        table = exactkv.PageTable(2 * B, B, 2)
+        c = exactkv.PagedCompressedKV(table, H, D=D, reserve=1.0)
+    else:
+        table, c = None, exactkv.CompressedKV(B, 32, H, D, reserve=1.0)
+    for b in range(B):
+        c.prefill_slot(b if table is None else table.add(T0), x[b:b + 1, :T0].contiguous())
+    for t in range(T0, T0 + N):
+        flat = torch.full((B * H * (D + pitch) + offset,), 3.0, dtype=torch.bfloat16, device=DEV)
+        row = flat[offset:].view(B, H, D + pitch)[..., :D]
+        row.copy_(x[:, t])
+        if paged:
+            table.begin_step()
+        c.append(row)
+        exactkv.check_overflow([c])
+        got = kernels.decode_to_bf16(c.buffers(), t + 1, block_table=table.block_table if paged else None)
+        assert same_bits(got, x[:, :t + 1]), t
+
+
 def test_misaligned_cache_arrays_are_refused():
     """array_ptrs names what is at fault: an array off 16 bytes, a word off 4, a tensor not on the GPU."""
     buf = torch.zeros(64, dtype=torch.uint8, device=DEV)
