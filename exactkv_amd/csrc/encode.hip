@@ -2,8 +2,9 @@
 // compressed -> bf16 decoder, for gfx950.
 //
 // Encoding one call's pages takes two launches on the caller's stream up to 65,536 units (the
-// page kernel, then scan_direct_kernel for 2-4 below); above, four, or two when the caller
-// gives a scan workspace (2-4 then run as one chained scan kernel, scan_chain_kernel):
+// page kernel, then scan_direct_kernel for 2-4 below; fewer where the rowmasks lie scattered or
+// unaligned, direct_units()); above, four, or two when the caller gives a scan workspace (2-4 then
+// run as one chained scan kernel, scan_chain_kernel):
 //   1. enc_pages_kernel    one wavefront per (sequence, page, head): exponent window,
 //                          zero flag, codes, sign|mantissa bytes, base bytes, rowmask
 //                          (reference kernels.py:216-264, codec.py:31-49);
@@ -511,8 +512,28 @@ __global__ void __launch_bounds__(1024) scan_chain_kernel(EncArgs a, int nunits,
 // heads runs 32 of them instead of the chain's 2 of 1,024) and their 16 wavefronts take 4 to
 // 16 units each, which is what the raw-row copies need: their loads are a dependent round
 // trip after the masks. The masks read grow with the square of the units (33 MB at 65,536, in
-// 256 blocks), hence the limit.
-constexpr int kDirectUnits = 65536;
+// 256 blocks), hence the limit; where they can't be read four at a time (a block table, or
+// masks that are not 16-byte aligned) a mask costs two divisions, and with a table a load before
+// its own, so the line lies where the chain gets ahead: encodes direct / chained at head dim 128
+// through a table, 8,192 units 20.0 / 21.2 us, 10,240 23.0 / 23.4, 16,384 32.8 / 30.6, 65,536
+// 132.4 / 102.7; unaligned, 10,240 21.5 / 22.8, 12,288 24.5 / 24.9, 16,384 30.0 / 29.3, 65,536
+// 118.0 / 98.0 (head dim 64 crosses at 8,192 and 12,288). A prefill's end rides in the direct
+// scan's launch and needs one of its own beside the chain: a paged slot of 10,000 units 43.0 /
+// 46.2, 16,376 53.7 / 53.9, 30,000 75.2 / 64.7.
+constexpr int kDirectUnits = 65536, kDirectUnitsUnaligned = 12288, kDirectUnitsPaged = 8192;
+constexpr int kDirectUnitsPrefill = 16384;             // with a prefill's end, of masks read one by one
+
+// Whether the masks of the call's units lie in rows whose parts of four words are 16-byte aligned.
+__host__ __device__ inline bool masks_by_four(const EncArgs& a) {
+    if (a.dst_pages != nullptr) return false;
+    const int64_t L = (int64_t)a.npg * a.H, S = (int64_t)(a.TS / kPage) * a.H;   // words a sequence, and to the next
+    return (uintptr_t)(a.rowmask + a.b0 * S + (int64_t)a.pg0 * a.H) % 16 == 0 && (a.nb == 1 || (L % 4 == 0 && S % 4 == 0));
+}
+
+static int direct_units(const EncArgs& a, bool prefill) {
+    if (masks_by_four(a)) return kDirectUnits;
+    return prefill ? kDirectUnitsPrefill : a.dst_pages != nullptr ? kDirectUnitsPaged : kDirectUnitsUnaligned;
+}
 
 static int direct_block_units(int64_t n) { return n <= 16384 ? 64 : n <= 32768 ? 128 : 256; }
 
@@ -526,7 +547,7 @@ __device__ inline int raw_rows_before(const EncArgs& a, int u0) {
         const int64_t S = (int64_t)(a.TS / kPage) * a.H;
         const int32_t* p0 = a.rowmask + (int64_t)a.b0 * S + (int64_t)a.pg0 * a.H;
         const bool one = a.nb == 1;
-        if ((uintptr_t)p0 % 16 == 0 && (one || (L % 4 == 0 && S % 4 == 0))) {   // uniform
+        if (masks_by_four(a)) {                        // uniform
             for (int v0 = 4 * (int)threadIdx.x; v0 < u0; v0 += 4 * 4096) {
                 uint4 m[4];
 #pragma unroll
@@ -715,7 +736,7 @@ static void launch_direct(const EncArgs& a, int64_t n, bool paged, bool vec16, c
     hipLaunchKernelGGL(k, dim3((unsigned)(nscan + END)), dim3(1024), 0, stream, a, (int)n, ub, nscan, e);
 }
 
-// Encode n units: the page kernel, then the direct scan up to kDirectUnits units; above, the
+// Encode n units: the page kernel, then the direct scan up to direct_units() units; above, the
 // chained scan when the workspace has at least 2 + ceil(n / kScanUnits) words, else the
 // three-launch scan. end: a prefill's end too, in the direct scan's launch or in one of its own.
 template <int D>
@@ -727,7 +748,7 @@ static void launch_encode_d(const EncArgs& a, int64_t n, uint64_t* ws, int64_t w
     }
     hipLaunchKernelGGL(enc_pages_kernel<D>, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream, a, (int)n);
     const bool paged = a.dst_pages != nullptr, vec16 = rows_of_16_bytes(a);
-    if (n <= kDirectUnits) {
+    if (n <= direct_units(a, end != nullptr)) {
         if (end)
             launch_direct<D, true>(a, n, paged, vec16, *end, stream);
         else

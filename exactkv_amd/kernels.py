@@ -366,7 +366,9 @@ def _check_source(src, strides, nb, npg, H, D):
         raise ValueError(f"encode source too small: needs element {last}, has {avail}")
 
 
-DIRECT_UNITS = 65536   # pages x heads of one encode up to which its slot scan needs no workspace
+# pages x heads of one encode up to which its slot scan needs no workspace: where it reads the
+# rowmasks four at a time, and the least limit where it can't (a block table, unaligned masks)
+DIRECT_UNITS, DIRECT_UNITS_ONE_BY_ONE = 65536, 8192
 _SCAN = {}  # page-encoder scan workspaces per (device, stream)
 
 
@@ -382,6 +384,11 @@ def _scan_ws(dev, units):
     return ws
 
 
+def _scan_ws_for(dev, units, H, paged):
+    """The scan workspace that an encode of `units` pages x heads may use, or None."""
+    return None if units <= (DIRECT_UNITS_ONE_BY_ONE if paged or H % 4 else DIRECT_UNITS) else _scan_ws(dev, units)
+
+
 def encode_pages(src, strides, buf, b0, pg0, nb, npg, *, chained=True):
     """Page encoder (reference kernels.py:216-268, same arguments). Source page pg0 + p of
     sequence b0 + i sits at src + i*s_b + p*s_pg, its token rows s_p apart and heads s_h
@@ -390,14 +397,15 @@ def encode_pages(src, strides, buf, b0, pg0, nb, npg, *, chained=True):
     arrays, the raw-row counter cnt, cap, TS, H, D and optionally 'before', which receives
     the counter's value before the call. Escaped rows take pool slots from the counter on,
     in (sequence, page, head, token) order. Two launches: the page kernel, then the slot scan
-    (above 65,536 pages x heads a chained one, in a per-stream workspace; there
-    chained=False makes it three launches: same bytes)."""
+    (above 65,536 pages x heads, or 12,288 where H is no multiple of 4 and the masks lie
+    unaligned, a chained one, in a per-stream workspace; there chained=False makes it three
+    launches: same bytes)."""
     H, TS, D = buf["H"], buf["TS"], buf["D"]
     _check_source(src, strides, nb, npg, H, D)
     raw = buf["raw"]
     before = buf.get("before")
     units = int(nb) * int(npg) * H
-    ws = _scan_ws(raw.device, units) if chained and units > DIRECT_UNITS else None
+    ws = _scan_ws_for(raw.device, units, H, False) if chained else None
     _lib.call("exkv_encode_pages", _lib.ptr(src, align=2, what="src"), *[int(s) for s in strides],
               _lib.ptr(buf["sm"]), _lib.ptr(buf["code"]), _lib.ptr(buf["base"]), _lib.ptr(buf["rowmask"]),
               _lib.ptr(buf["rowoff"]), _lib.ptr(raw), _lib.ptr(buf["cnt"], align=4),
@@ -420,7 +428,8 @@ def store_raw_rows(src, strides, buf, b0, pg0, nb, npg):
 def encode_pages_paged(src, strides, buf, dst_pages, nb, npg, *, chained=True):
     """encode_pages into a paged cache: page pg of source sequence bi (strides as in
     encode_pages) goes to page dst_pages[bi, pg] of the cache's arrays read as a list of
-    B * TS / 16 pages. dst_pages: int32 [>= nb, >= npg] on the GPU."""
+    B * TS / 16 pages. dst_pages: int32 [>= nb, >= npg] on the GPU. The scan is the chained one
+    above 8,192 pages x heads."""
     H, TS, D = buf["H"], buf["TS"], buf["D"]
     _check_source(src, strides, nb, npg, H, D)
     if (dst_pages.dtype != torch.int32 or dst_pages.dim() != 2 or dst_pages.stride(1) != 1 or dst_pages.shape[0] < nb
@@ -429,7 +438,7 @@ def encode_pages_paged(src, strides, buf, dst_pages, nb, npg, *, chained=True):
     raw = buf["raw"]
     before = buf.get("before")
     units = int(nb) * int(npg) * H
-    ws = _scan_ws(raw.device, units) if chained and units > DIRECT_UNITS else None
+    ws = _scan_ws_for(raw.device, units, H, True) if chained else None
     _lib.call("exkv_encode_pages_paged", _lib.ptr(src, align=2, what="src"), *[int(s) for s in strides],
               _lib.ptr(buf["sm"]), _lib.ptr(buf["code"]), _lib.ptr(buf["base"]), _lib.ptr(buf["rowmask"]),
               _lib.ptr(buf["rowoff"]), _lib.ptr(raw), _lib.ptr(buf["cnt"], align=4),
@@ -459,7 +468,7 @@ def prefill_pages(x, c, *, b=0, table=None):
         _check_source(x, (x.stride(0), P * s_t, s_t, s_h), 1, T // P, H, D)
     ptrs = c._ptrs()
     units = (T // P) * H
-    ws = _scan_ws(c.raw.device, units) if units > DIRECT_UNITS else None
+    ws = _scan_ws_for(c.raw.device, units, H, table is not None)
     w = _lib.tagged_words(c.raw.device.index, 2)
     scan = (_lib.ptr(ws), ws.numel() if ws is not None else 0, w.addr, w.tag, _lib.stream())
     if table is None:

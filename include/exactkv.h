@@ -77,9 +77,10 @@ const char* exkv_last_error(void);
  * *before (may be NULL) receives the counter's value before the call.
  * scan_ws (8-byte aligned, may be NULL): a workspace of scan_ws_words 64-bit words, all zero
  * when first used and reserved for this library's encodes on one stream. Up to 65,536 pages x
- * heads the encode is two launches and does not use it; above, with at least
- * 2 + ceil(nb*npg*H / 1024) words it is two launches (the page kernel, then one chained slot
- * scan), else four (the page kernel, then a three-launch scan). Same bytes either way.
+ * heads (12,288 where H is no multiple of 4 and the call's rowmasks are not 16-byte aligned) the
+ * encode is two launches and does not use it; above, with at least 2 + ceil(nb*npg*H / 1024)
+ * words it is two launches (the page kernel, then one chained slot scan), else four (the page
+ * kernel, then a three-launch scan). Same bytes either way.
  * Replaces: kernels.py:340-346 encode_pages (launch of _encode_pages_kernel :233-268),
  * byte-identical to codec.py:31-55 encode_reference. */
 int exkv_encode_pages(const void* src, int64_t s_b, int64_t s_pg, int64_t s_p, int64_t s_h,
@@ -101,7 +102,8 @@ int exkv_store_raw_rows(const void* src, int64_t s_b, int64_t s_pg, int64_t s_p,
  * s_t, s_h for token and head; channels contiguous). Its T / 16 full pages are encoded as by
  * exkv_encode_pages; the other rows go to the slot's open-page rows, raw rows
  * cap + (b*H + h)*16 on; page T / 16 of every sequence is opened as by exkv_cache_open_page;
- * and state[0] = T. Two launches up to 65,536 pages x heads. Overflow shows in *cnt, as for
+ * and state[0] = T. Two launches up to 65,536 pages x heads (16,384 where H is no multiple of 4
+ * and the slot's rowmasks are not 16-byte aligned). Overflow shows in *cnt, as for
  * exkv_encode_pages. host (may be NULL): two words of mapped host memory; the call then waits,
  * on a stream that is not being captured, until *cnt is in host[1] and `tag`, which host[0] must not
  * hold before, in host[0], by when src's full pages have been read. state[1] is zero between
@@ -113,7 +115,8 @@ int exkv_prefill_slot(const void* src, int64_t s_t, int64_t s_h, int32_t T, void
                       void* scan_ws, int64_t scan_ws_words, int32_t* host, int32_t tag, hipStream_t stream);
 
 /* The same into slot `slot` of a paged cache whose page p is pool page table[p] (max_pages
- * entries, clamped to the pool); page T / 16 of the slot is opened where the table has it.
+ * entries, clamped to the pool; two launches up to 16,384 pages x heads); page T / 16 of the slot
+ * is opened where the table has it.
  * arrivals: a word that is zero between calls (with host). */
 int exkv_prefill_slot_paged(const void* src, int64_t s_t, int64_t s_h, int32_t T, void* sm, void* code, void* base,
                             int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before,
@@ -124,7 +127,7 @@ int exkv_prefill_slot_paged(const void* src, int64_t s_t, int64_t s_h, int32_t T
 /* The page encoder into a paged cache: page pg of source sequence bi goes to page
  * dst_pages[bi*dst_stride + pg] of the B x TS arrays read as a list of B*TS/16 pages (entries
  * clamped to it). Same bytes and raw-slot order as exkv_encode_pages, and the same scan
- * workspace.
+ * workspace, which it uses above 8,192 pages x heads.
  * No counterpart in the reference (contiguous caches only); paged KV is in its future
  * work (README.md:121-123). */
 int exkv_encode_pages_paged(const void* src, int64_t s_b, int64_t s_pg, int64_t s_p, int64_t s_h,

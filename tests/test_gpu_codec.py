@@ -254,6 +254,67 @@ def test_encoder_slot_scan_block_edges(B, npg, H, b0, pg0, D, paged):
     assert not bool(c.raw[:5].view(torch.int16).any()) and not bool(c.raw[5 + n:c.cap].view(torch.int16).any())
 
 
+def _source(B, T, H, D, rate, g, shift=0):
+    """bf16 [B, T, H, D], a share of rows raw, its memory `shift` elements off an allocation's start."""
+    x = torch.empty(B * T * H * D + shift, dtype=torch.bfloat16, device=DEV)[shift:].view(B, T, H, D)
+    for b in range(B):
+        x[b] = torch.randn(T, H, D, generator=g, device=DEV)
+    x[torch.rand(B, T, H, generator=g, device=DEV) < rate, 3] *= 2.0 ** -30
+    return x
+
+
+def _check_slots(x, rm, off, raw, cap, cnt0, cnt):
+    """Raw-row slots of pages encoded from x [B, T, H, D], masks and offsets [B, T / 16, H]: each unit's
+    offset is cnt0 plus the raw rows of the units before it, those below cap are in their slots, the
+    counter is past all of them."""
+    B, T, H, D = x.shape
+    bits = ((rm[..., None] >> torch.arange(16, device=DEV)) & 1).bool()          # [B, pages, H, 16]
+    per = bits.sum(-1).reshape(-1)
+    assert torch.equal(off.reshape(-1).long(), torch.cumsum(per, 0) - per + cnt0)
+    n = int(per.sum())
+    assert cnt == cnt0 + n
+    want = x.view(B, T // 16, 16, H, D).permute(0, 1, 3, 2, 4)[bits]             # (sequence, page, head, token) order
+    m = min(cap - cnt0, n)
+    assert torch.equal(raw[cnt0:cnt0 + m].view(torch.int16), want[:m].view(torch.int16))
+    return n
+
+
+@pytest.mark.parametrize("npg,H,pg0,paged,prefill,direct", [
+    (8192, 8, 0, False, False, True), (8193, 8, 0, False, False, False),      # 65,536 units of masks read by fours
+    (4096, 3, 1, False, False, True), (4097, 3, 1, False, False, False),      # 12,288 and 12,291 of masks off 16 bytes
+    (21845, 3, 0, False, False, True),                                        # as many heads, aligned
+    (1024, 8, 0, True, False, True), (1025, 8, 0, True, False, False),        # 8,192 through a table
+    (2048, 8, 0, True, True, True), (2049, 8, 0, True, True, False),          # 16,384, the scan with a prefill's end
+])
+def test_slot_scan_by_mask_layout(npg, H, pg0, paged, prefill, direct):
+    """Which slot scan an encode takes, seen by whether the chained one's workspace was used, and its
+    slots, on both sides of each limit."""
+    g = torch.Generator(device=DEV).manual_seed(npg + H)
+    x = _source(1, npg * 16, H, 64, 0.02, g)
+    _say("slot scan by layout", npg, H, pg0, paged, prefill)
+    kernels.release_workspaces()
+    if paged:
+        table = exactkv.PageTable(npg + 1, 1, npg + 1)
+        table._free = torch.randperm(npg + 1, generator=torch.Generator().manual_seed(1)).tolist()
+        table.add(npg * 16)
+        c = exactkv.PagedCompressedKV(table, H, D=64, reserve=0.2)
+        pages = torch.tensor(table.pages(0)[:npg], device=DEV)
+    else:
+        c = exactkv.CompressedKV(1, (pg0 + npg) * 16, H, 64, reserve=0.2)
+        pages = torch.arange(pg0, pg0 + npg, device=DEV)
+    c.cnt.fill_(5)
+    if prefill:
+        assert kernels.prefill_pages(x, c, table=table) == int(c.cnt.item())
+    elif paged:
+        c._encode_pages(x, (x.stride(0), 16 * x.stride(1), x.stride(1), x.stride(2)), table.block_table, npg)
+    else:
+        kernels.encode_pages(x, (x.stride(0), 16 * x.stride(1), x.stride(1), x.stride(2)), c._buf(), 0, pg0, 1, npg)
+    assert any(bool(ws.any()) for ws in kernels._SCAN.values()) != direct
+    rm, off = (t.view(-1, H)[pages].view(1, npg, H) for t in (c.rowmask, c.rowoff))
+    assert int(c._before.item()) == 5
+    assert _check_slots(x, rm, off, c.raw, c.cap, 5, int(c.cnt.item())) > 0.01 * npg * 16 * H
+
+
 @pytest.mark.parametrize("B,T,H,D,rate", [(1, 16, 1, 64, 1.0), (2, 160, 3, 128, 0.2), (3, 1040, 5, 256, 0.02),
                                           (1, 4096, 8, 128, 1.0), (4, 2048, 8, 64, 0.0)])
 @pytest.mark.parametrize("shift", [0, 2])
