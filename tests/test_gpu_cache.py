@@ -206,6 +206,36 @@ def test_prefill_takes_any_index_type(T):
         assert torch.equal(getattr(a, n), getattr(c, n)), n
 
 
+@pytest.mark.parametrize("T,H,D", [(1, 1, 64), (15, 128, 256), (31, 128, 256), (31, 33, 128), (20, 64, 128), (31, 70, 64)])
+@pytest.mark.parametrize("kind", ["plain", "heads", "pairs", "odd"])
+@pytest.mark.parametrize("paged", [False, True])
+def test_prefill_open_rows(T, H, D, kind, paged):
+    """A prompt's last rows in the open page, in 16-, 4- and 2-byte pieces, a few and more than the
+    block has in flight at once."""
+    if kind == "odd" and T >= 16:
+        pytest.skip("full pages need 4-byte aligned rows")
+    g = torch.Generator(device=DEV).manual_seed(T + H)
+    x = torch.randn(1, T, H, D, generator=g, device=DEV).bfloat16()
+    if paged:
+        table = exactkv.PageTable(8, 2, 3)
+        c = exactkv.PagedCompressedKV(table, H, D=D, reserve=3.0)
+        c.prefill(table.add(17), torch.ones(1, 17, H, D, dtype=torch.bfloat16, device=DEV))
+        slot = table.add(T)
+        first = c.cap + slot * H * 16
+    else:
+        slot, c = 1, exactkv.CompressedKV(2, 48, H, D, reserve=3.0)
+        first = c.cap + H * 16
+    before = c.raw.clone()
+    (c.prefill if paged else c.prefill_slot)(slot, _layout(x, kind))
+    assert c.grows == 0
+    got = kernels.decode_to_bf16(c.buffers(), T, block_table=table.block_table if paged else None)
+    assert same_bits(got[slot], x[0])
+    rows = c.raw[first:first + H * 16].view(H, 16, D)
+    assert same_bits(rows[:, :T % 16], x[0, T - T % 16:].transpose(0, 1))
+    rows[:, :T % 16] = before[first:first + H * 16].view(H, 16, D)[:, :T % 16]
+    assert same_bits(c.raw[c.cap:], before[c.cap:])        # no other row
+
+
 @pytest.mark.parametrize("B,H,D", [(1, 1, 64), (2, 8, 128), (9, 8, 128), (3, 5, 256), (300, 4, 64)])
 @pytest.mark.parametrize("offset,pitch", [(0, 0), (2, 0), (0, 2), (4, 4), (0, 6)])
 @pytest.mark.parametrize("paged", [False, True])
