@@ -148,10 +148,10 @@ def _popc16(t):
 
 
 @pytest.mark.parametrize("chained", [True, False])
-@pytest.mark.parametrize("B,T,H", [(8, 8192, 16), (5, 8192, 32)])
+@pytest.mark.parametrize("B,T,H", [(8, 8208, 16), (5, 8192, 32)])
 def test_encoder_slot_scan_full_size(B, T, H, chained):
-    """65,536 and 81,920 units, 5% outlier rows, counter starting at 7, through the
-    chained scan (look-back over 64 and 80 blocks) and the three-launch scan:
+    """65,664 and 81,920 units, 5% outlier rows, counter starting at 7, through the
+    chained scan (look-back over 65 and 80 blocks) and the three-launch scan:
     every rowoff is 7 + the raw rows of the units before it in (sequence, page, head)
     order, the counter ends at 7 + all of them, and decoding gives back every bit."""
     x = synthetic.make_kv(B, T, H, kind="k", seed=31, raw_row_rate=0.05, device=DEV)
@@ -175,10 +175,12 @@ def test_encoder_chained_equals_multi_launch():
     the three-launch scan on the same input and counter, including a raw pool too small for
     every raw row (slots past cap skipped, counter past cap), head dims 64 and 256, a unit
     with every row raw, and source rows 4-byte but not 16-byte aligned (the raw-row copy's
-    word path)."""
-    cases = [(2, 64, 8, 0.05, 0.5, 128), (4, 4096, 8, 0.02, 0.5, 128), (1, 32, 2, 0.3, 0.5, 128),
-             (3, 1024, 16, 0.05, 0.002, 128), (2, 512, 8, 0.05, 0.5, 128), (4, 2048, 8, 0.05, 0.5, 64),
-             (2, 1024, 4, 0.05, 0.5, 256), (64, 512, 8, 0.01, 0.5, 128)]
+    word path). All but the last have masks that are not read by fours, so that 12,289 units
+    are enough for these scans."""
+    cases = [(3, 16 * 1367, 3, 0.05, 0.5, 128), (2, 16 * 2051, 5, 0.02, 0.5, 128), (3, 16 * 1389, 3, 0.3, 0.5, 128),
+             (5, 16 * 839, 3, 0.05, 0.002, 128), (3, 16 * 1367, 3, 0.05, 0.5, 128), (7, 16 * 1795, 1, 0.05, 0.5, 64),
+             (2, 16 * 2051, 3, 0.05, 0.5, 256), (8, 8208, 16, 0.01, 0.5, 64)]
+    kernels.release_workspaces()
     for i, (B, T, H, rate, reserve, D) in enumerate(cases):
         x = synthetic.make_kv(B, T, H, D=D, kind="k", seed=40 + i, raw_row_rate=rate, device=DEV)
         if i == 2:
@@ -194,6 +196,8 @@ def test_encoder_chained_equals_multi_launch():
             c.cnt.fill_(3)
             kernels.encode_pages(x, st, c._buf(), 0, 0, B, T // 16, chained=chained)
             out.append(c)
+        ws, = kernels._SCAN.values()
+        assert ws[:2].tolist() == [0, i + 1]               # no ticket out, a generation for each chained call
         a, b = out
         _say("chained vs three-launch scan", B, T, H, D, "counter", int(a.cnt.item()), "cap", a.cap)
         for f in ("sm", "code", "base", "rowmask", "rowoff", "cnt", "_before"):
@@ -313,6 +317,43 @@ def test_slot_scan_by_mask_layout(npg, H, pg0, paged, prefill, direct):
     rm, off = (t.view(-1, H)[pages].view(1, npg, H) for t in (c.rowmask, c.rowoff))
     assert int(c._before.item()) == 5
     assert _check_slots(x, rm, off, c.raw, c.cap, 5, int(c.cnt.item())) > 0.01 * npg * 16 * H
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("shift", [0, 2])
+@pytest.mark.parametrize("reserve", [0.3, 0.01])
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("chained", [True, False])
+def test_chained_and_three_launch_scans(D, shift, reserve, paged, chained):
+    """The scans above the direct one's limits, contiguous and through a block table, with rows 16- and
+    4-byte aligned and a pool with and without room: masks as the direct scan's encode of the same
+    pages, slots, raw rows and counter; nothing behind cap."""
+    B, npg, H = (2, 1367, 3) if paged else (3, 1367, 3)        # 8,202 and 12,303 units
+    g = torch.Generator(device=DEV).manual_seed(D + shift)
+    x = _source(B, npg * 16, H, D, 0.05, g, shift)
+    st = (x.stride(0), 16 * x.stride(1), x.stride(1), x.stride(2))
+    _say("scans above the limits", D, shift, reserve, paged, chained)
+    kernels.release_workspaces()
+    c = exactkv.CompressedKV(B, (npg + 1) * 16, H, D, reserve=reserve)
+    c.cnt.fill_(5)
+    c.raw.fill_(7.0)
+    old = c.raw.clone()
+    if paged:
+        order = torch.randperm(B * (npg + 1), generator=g, device=DEV)[:B * npg].view(B, npg)
+        kernels.encode_pages_paged(x, st, c._buf(), order.to(torch.int32), B, npg, chained=chained)
+        rm, off = (t.view(-1, H)[order] for t in (c.rowmask, c.rowoff))
+    else:
+        kernels.encode_pages(x, st, c._buf(), 0, 1, B, npg, chained=chained)
+        rm, off = (t[:, 1:] for t in (c.rowmask, c.rowoff))
+    assert len(kernels._SCAN) == chained
+    one = exactkv.CompressedKV(1, npg * 16, H, D, reserve=0.3)     # a sequence alone: 4,101 units
+    for b in range(B):
+        kernels.encode_pages(x[b:b + 1], st, one._buf(), 0, 0, 1, npg)
+        assert torch.equal(one.rowmask[0], rm[b])
+    n = _check_slots(x, rm, off, c.raw, c.cap, 5, int(c.cnt.item()))
+    assert int(c._before.item()) == 5 and (5 + n > c.cap) == (reserve < 0.1)
+    end = min(5 + n, c.cap)
+    assert same_bits(c.raw[:5], old[:5]) and same_bits(c.raw[end:], old[end:])
 
 
 @pytest.mark.parametrize("B,T,H,D,rate", [(1, 16, 1, 64, 1.0), (2, 160, 3, 128, 0.2), (3, 1040, 5, 256, 0.02),

@@ -131,11 +131,11 @@ def test_paged_bad_arguments_raise():
 @pytest.mark.parametrize("chained", [True, False])
 def test_paged_encoder_bytes_match_contiguous(chained):
     """encode_pages_paged writes, at each mapped pool page, the bytes encode_pages writes
-    at the contiguous page (same raw-slot order, so rowoff and raw agree too); through the
-    chained scan and through the three-launch scan."""
-    B, TS, H = 3, 512, 8
+    at the contiguous page (same raw-slot order, so rowoff and raw agree too); 8,256 units,
+    through the chained scan and through the three-launch scan, against the direct scan."""
+    B, TS, H = 3, 5504, 8
     npg = TS // P
-    x = synthetic.make_kv(B, TS, H, kind="k", seed=71, raw_row_rate=0.02).to(DEV)
+    x = synthetic.make_kv(B, TS, H, kind="k", seed=71, raw_row_rate=0.02, device=DEV)
     pool_pages = B * npg + 9
     table = torch.randperm(pool_pages, generator=torch.Generator().manual_seed(8))[:B * npg].view(B, npg)
     c = _encode(x)

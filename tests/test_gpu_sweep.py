@@ -404,10 +404,11 @@ def test_encoder_sweep(c):
     """encode_pages (reference kernels.py:216-268, 340-346) of pages [pg0, pg0 + npg) of
     sequences [b0, b0 + nb) from token-major, head-major and every-other-head strided
     sources, the counter starting at 0 or not, a pool large enough or not (rows past cap are
-    dropped while the counter advances), chained or three-launch slot scan, head dims 64 /
-    128 / 256, pages of NaN and inf: every written byte equals the oracle's encode of the same
-    pages (rowoff shifted by the counter's start), nothing outside the pages is written, and
-    the counter and 'before' are the oracle's."""
+    dropped while the counter advances), with and without a scan workspace on offer (sizes of
+    the direct slot scan, which uses none), head dims 64 / 128 / 256, pages of NaN and inf:
+    every written byte equals the oracle's encode of the same pages (rowoff shifted by the
+    counter's start), nothing outside the pages is written, and the counter and 'before' are
+    the oracle's."""
     from oracle import codec as ocodec
     print("[case]", c, flush=True)
     D, H, nb, npg, b0, pg0 = c["D"], c["H"], c["nb"], c["npg"], c["b0"], c["pg0"]
