@@ -367,7 +367,7 @@ def main():
     if a.profile:
         a.copies = 1
     if a.gpus != 1:
-        print(f"bench.py measures one GPU; --gpus {a.gpus} is not supported in this build "
+        print(f"bench.py measures one GPU; --gpus {a.gpus} is not supported "
               "(the decode path shards by KV head or sequence with no exchange)", file=sys.stderr)
         sys.exit(2)
 

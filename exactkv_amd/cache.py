@@ -6,8 +6,8 @@ How CompressedKV is organised here:
 
 * Six device arrays per cache in the codec's layout (sm, code, base, rowmask, rowoff, raw)
   plus int32 words on the device: the raw-row counter `cnt`, its value before the latest
-  page encode, and `state[0]`, the number of tokens held (`state[1]` is the append
-  kernel's arrival counter, zero between calls).
+  page encode, and `state[0]`, the number of tokens held (`state[1]` counts
+  the workgroups of appends and prefills in, zero between calls).
 * The raw array is two regions. Rows [0, cap) take escaped rows in the codec's order
   (sequence, page, head, token), which keeps every byte equal to codec.encode's. Behind
   them each (sequence, head) owns 16 rows holding its open page -- the newest, partly

@@ -51,14 +51,15 @@ extern "C" const char* exkv_last_error(void) { return exkv::g_err; }
 // `ramp` more (a workgroup's first page's latency and its epilogue, 6 us), and the last
 // workgroups end spread over a sixteenth of their own time:
 //   cost = R ramp + j (R - 1 + max(last round's share, 0.85)) + (ramp + j) / 16.
-// It fits the sweep behind it (B 1 to 220, 2 to 440 units, T 1000 to 16000) within 5%:
-// 24 x 4093 at 32q/8kv, 5 splits x 832 (240 workgroups) 57.0 us, 6 x 704 (288: two rounds, the
-// second nearly empty) 86.9, 10 x 416 63.2. For each R the best plan is the most splits that
-// fit R rounds, so eight of them are compared, and of equal ones the first (fewer rounds,
-// more splits) is taken. Rounding the split count up instead of down, as before, cost 1.3 to
-// 1.65 times the time wherever the unit count does not divide 256 (same calls, split count
-// up / down: 3 x 4093 24.0 / 17.0 us, 6 x 8192 53.8 / 33.0, 12 x 4093 51.4 / 33.3, 40 x 2048
-// 73.1 / 49.4; head dim 64 24 x 4093 57.0 / 38.8; head dim 256 9 x 4093 88.8 / 56.2).
+// Over a sweep of 43 shapes (B 1 to 220, 1 to 440 units, T 512 to 32763; profiles/plan_sweep.md) it
+// is 0.91 to 1.13 of the time of the plans it chooses from 30 us on, and the plan is within 2% of
+// the best one timed but for one shape (10%): 24 x 4093 at 32q/8kv, 5 splits x 832 (240
+// workgroups) 56.5 us, 6 x 704 (288: two rounds, the second nearly empty) 82.8, 10 x 416 59.7. For
+// each R the best plan is the most splits that fit R rounds, so eight of them are compared, and of
+// equal ones the first (fewer rounds, more splits) is taken. Rounding the split count up instead of
+// down costs 1.3 to 1.6 times the time wherever the unit count does not divide 256 (same calls,
+// split count up / down: 3 x 4093 21.2 / 15.6 us, 6 x 8192 50.6 / 31.8, 12 x 4093 45.5 / 31.6,
+// 40 x 2048 64.1 / 46.7; head dim 64 24 x 4093 50.1 / 35.3; head dim 256 9 x 4093 80.7 / 52.7).
 // Short splits cost little: a wavefront's pages follow one another at about one memory round
 // trip each, so few units are served best by many splits, down to min_split tokens (16 by
 // default, one page; measured with one round, 64- / 32- / 16-token splits: a 1024-token window
@@ -74,8 +75,8 @@ static double plan_cost(int64_t units, int64_t ns, int64_t pages, int64_t slots,
 // fullest: the plan of grids larger than the GPU (the second round's workgroups start as the
 // first ones end, which staggers the tail; measured at B256 x 4352, 1/2/4/8 splits:
 // 610/601/614/636 us; B620: 2 splits 1454 us, 4 splits 1490 us), unless plan_cost finds one
-// more than a sixteenth (its error) cheaper, as it does for short contexts (B220 x 1000:
-// 4 x 256 152.7 us, 1 x 1008 125.2).
+// more than a sixteenth (about its error) cheaper, as it does for short contexts (B220 x 1000:
+// 4 x 256 150.3 us, 1 x 1008 122.0).
 static int64_t full_rounds(int64_t units, int64_t slots) {
     int64_t ns = 1;
     double best = -1.0;
@@ -93,7 +94,10 @@ static int64_t full_rounds(int64_t units, int64_t slots) {
 }
 
 // The plan, for workgroups of nph page phases; `most`: the splits whose partials fit the
-// no-alloc entry point's scratch, so that it takes every plan.
+// no-alloc entry point's scratch, which bounds what the cost model is asked. The plans of
+// full_rounds, and of head dim 64 with odd KV heads, are not bounded by it: for many long sequences
+// that entry point needs its caller's own, smaller plan (129 x 8192 at 32q/8kv: 16 splits, of
+// which 15 fit).
 static void plan_core(int64_t units, int32_t T, int64_t slots, int32_t min_split, int nph, double ramp, int64_t most,
                       int32_t* nsplit, int32_t* split_len) {
     const int64_t pages = ((int64_t)T + exkv::kPage - 1) / exkv::kPage;

@@ -179,7 +179,7 @@ class PagedCompressedKV:
         self.rowoff = torch.zeros(1, NPg, H, dtype=torch.int32, device=dev)
         self.cnt = torch.zeros(1, dtype=torch.int32, device=dev)
         self._before = torch.zeros(1, dtype=torch.int32, device=dev)
-        self._arrivals = torch.zeros(1, dtype=torch.int32, device=dev)   # the append kernel's, zero between calls
+        self._arrivals = torch.zeros(1, dtype=torch.int32, device=dev)   # of appends and prefills, zero between calls
         self._step_room = table.max_seqs * H * P                  # rows one step can add at most
         self.cap = max(64, int(self.TS * H * reserve), self._step_room)
         self.raw = torch.zeros(self.cap + self._step_room, D, dtype=torch.bfloat16, device=dev)

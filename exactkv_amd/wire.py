@@ -3,7 +3,7 @@
 unpack it into a contiguous or paged cache, on the GPU.
 
 No counterpart in the reference: its caches hand out their six tensors (buffers(),
-cache.py:121-123); a byte form of them is this build's own. The blob keeps the
+cache.py:121-123); a byte form of them is this package's own. The blob keeps the
 reference format's fields (codec.py:1-25) for one sequence, about 200 bytes per
 (token, head) against 256 for bf16. Layout (little-endian, sections at multiples of
 256 bytes, gaps zero):

@@ -5,9 +5,14 @@
  * it stands in for is given above each declaration.
  *
  * Conventions
- *   - All pointers are device pointers (HIP), except the outputs of the split planners.
- *   - Work is enqueued on `stream` only; nothing synchronizes, nothing allocates, so
- *     calls can be captured in a HIP graph. The library's one piece of device state is
+ *   - All pointers are device pointers (HIP), except the outputs of the split planners, the
+ *     arrays that exkv_table_write and exkv_fetch_words read (host memory), and what is
+ *     named host_... or `host`: host memory that the GPU can write (pinned and mapped).
+ *   - Work is enqueued on `stream` only; nothing allocates, and nothing synchronizes but
+ *     exkv_fetch_words and, given `host`, the exkv_prefill_slot calls, which wait for the
+ *     stream's work up to their own. Calls can be captured in a HIP graph, except those that wait and
+ *     exkv_table_write (a replay would write its values again), which refuse a capturing
+ *     stream. The library's device state is the sticky error words and
  *     exkv_attn_compressed_noalloc's fixed scratch array on each GPU it runs on.
  *   - bf16 tensors are passed as raw 16-bit patterns. Tensors are row-major with the
  *     shapes given; "elements" strides count bf16 elements.
@@ -186,8 +191,8 @@ int exkv_cache_append_paged(const void* x, int64_t sx_b, int64_t sx_h, void* sm,
                             hipStream_t stream);
 
 /* The same with an int32 word *arrivals of the caller's, zero when first used and reserved for
- * this cache's appends on one stream: one launch at every size (without it more than 128
- * sequences x heads take two). */
+ * this cache's appends and prefills on one stream: one launch at every size (without it more
+ * than 64 sequences x heads take two). */
 int exkv_cache_append_paged_counted(const void* x, int64_t sx_b, int64_t sx_h, void* sm, void* code, void* base,
                                     int32_t* rowmask, int32_t* rowoff, void* raw, int32_t* cnt, int32_t* before,
                                     int32_t* arrivals, int64_t cap, int64_t raw_rows, const int32_t* slots,

@@ -1,7 +1,7 @@
 """CPU model of the CompressedKV bookkeeping protocol (test infrastructure only).
 
 Restates reference exactkv/cache.py:17-158 with the two deliberate differences of
-this build, so that the GPU cache's buffers can be compared byte for byte:
+this package, so that the GPU cache's buffers can be compared byte for byte:
 
   * raw-row slots are assigned deterministically: within one encode call, pages are
     visited in (sequence, page, head) order and rows in token order, starting at the

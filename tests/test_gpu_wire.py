@@ -1,7 +1,7 @@
 """Wire form on the GPU: pack / unpack of one sequence's compressed cache.
 
 No counterpart in the reference (a byte form of buffers(), cache.py:121-123, is this
-build's own). Gates:
+package's own). Gates:
   * the GPU blob equals the oracle's blob byte for byte (oracle/wire.py);
   * unpacking into another cache, contiguous or paged, gives the same decoded values and
     bit-identical attention, and decoding can go on from there;

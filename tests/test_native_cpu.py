@@ -137,7 +137,7 @@ def test_plan_rounds(B, Hkv, Hq, T, D, slots, expect):
     ns, sl = plan_splits_hd(B, Hkv, Hq, T, D)
     assert (ns, sl) == expect
     assert sl % 16 == 0 and ns * sl >= T and (ns - 1) * sl < T
-    # every plan's partials fit the no-alloc entry point's scratch
+    # these plans' partials fit the no-alloc entry point's scratch
     assert B * Hq * ns * (D + 2) * 4 <= _lib.load().exkv_noalloc_scratch_bytes()
 
 

@@ -2,7 +2,7 @@
 oracle's layout, and malformed headers are rejected before anything is launched.
 
 No counterpart in the reference (a byte form of buffers(), cache.py:121-123, is this
-build's own)."""
+package's own)."""
 import ctypes
 from types import SimpleNamespace
 

@@ -1,7 +1,7 @@
 """CPU checks that pin the wire-form oracle (oracle/wire.py) and the library's layout.
 
 No counterpart in the reference (a byte form of buffers(), cache.py:121-123, is this
-build's own); the fields inside are the reference format's (codec.py:1-25)."""
+package's own); the fields inside are the reference format's (codec.py:1-25)."""
 import numpy as np
 import pytest
 
