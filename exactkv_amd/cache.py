@@ -137,7 +137,7 @@ class CompressedKV:
             raise AssertionError(f"{T} prompt tokens do not fit a cache of {self.TS}")
         full = T - T % P
         self.T = T
-        if isinstance(b, int) and 0 <= b < self.B and prefill_ready(x, self.sm.device, self.H, self.D):
+        if type(b) is int and 0 <= b < self.B and prefill_ready(x, self.sm.device, self.H, self.D):
             used = prefill_pages(x, self, b=b)
             if full and used > self.cap:
                 strides = (x.stride(0), P * x.stride(1), x.stride(1), x.stride(2))

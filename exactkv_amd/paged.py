@@ -253,7 +253,7 @@ class PagedCompressedKV:
         Tf = T // P * P
         t = self.table
         dst = t.block_table[slot: slot + 1]
-        if (isinstance(slot, int) and 0 <= slot < t.max_seqs and prefill_ready(x, self.sm.device, self.H, self.D)
+        if (type(slot) is int and 0 <= slot < t.max_seqs and prefill_ready(x, self.sm.device, self.H, self.D)
                 and t.block_table.stride(0) == t.max_pages):
             n = prefill_pages(x, self, b=slot, table=t)
             if Tf and n > self.cap:

@@ -206,6 +206,13 @@ def test_prefill_takes_any_index_type(T):
         assert torch.equal(getattr(a, n), getattr(c, n)), n
 
 
+@pytest.mark.parametrize("T", [7, 40])
+def test_prefill_refuses_a_truth_value_as_slot(T):
+    c = exactkv.CompressedKV(3, 64, 2, 128, reserve=0.6)
+    with pytest.raises(RuntimeError):
+        c.prefill_slot(True, torch.ones(1, T, 2, 128, dtype=torch.bfloat16, device=DEV))
+
+
 @pytest.mark.parametrize("T,H,D,kind", [
     (T, H, D, kind) for T, H, D in ((1, 1, 64), (15, 128, 256), (31, 128, 256), (31, 33, 128), (20, 64, 128), (31, 70, 64))
     for kind in ("plain", "heads", "pairs", "odd") if kind != "odd" or T < 16])    # full pages need 4-byte aligned rows
